@@ -281,7 +281,11 @@ int alloc_rdf_scratch(fa_batch* b)
 {
     fa::device_free(b->rs.nclus);
     fa::device_free(b->rs.table);
-    b->rs = fa::BatchRdfScratch{};
+    fa::BatchRdfScratch fresh{};
+    fresh.est_lo = b->rs.est_lo; // the range belongs to the plan, not to the buffers
+    fresh.est_hi = b->rs.est_hi;
+    fresh.est_slack = b->rs.est_slack;
+    b->rs = fresh;
     uint64_t const rows = b->gr.total_rows;
     uint64_t const maxc = uint64_t(b->total) / 8 + rows + 1;
     uint32_t* u = nullptr;
@@ -359,7 +363,7 @@ int enqueue_rdf(fa_batch* b)
         return rc;
     b->rs.scan_tmp = b->d_scan;
     b->rs.scan_bytes = b->scan_bytes;
-    return fa::batch_rdf(b->gr, b->rdf_R, b->plan.rdf_r_max, b->plan.rdf_bins, b->rs, b->d_rdf);
+    return fa::batch_rdf(b->gr, b->d_tile_frame, b->ntiles, b->rdf_R, b->plan.rdf_r_max, b->plan.rdf_bins, b->rs, b->d_rdf);
 }
 
 int enqueue_ql(fa_batch* b)
@@ -628,7 +632,7 @@ int fa_batch_create(uint32_t n_frames, const fa_box* boxes, const uint64_t* poin
     {
         if (int rc = fa::device_alloc((void**) &b->d_T, sizeof(float) * fa::rdf_table_floats(plan->rdf_bins)))
             return fail_out(rc);
-        if (int rc = fa::thresholds_for(plan->rdf_bins, plan->rdf_r_max, b->d_T))
+        if (int rc = fa::thresholds_for(plan->rdf_bins, plan->rdf_r_max, b->d_T, b->rs))
             return fail_out(rc);
         if (int rc = fa::device_alloc((void**) &b->d_rdf,
                                       sizeof(uint32_t) * std::max<uint64_t>(uint64_t(n_frames) * plan->rdf_bins, 1)))

@@ -761,11 +761,15 @@ struct BatchRdfScratch
     void* scan_tmp;
     size_t scan_bytes;
     uint64_t max_clusters;
+    // r_sq range of the estimate kernel (est_hi = 0: the exact one), set by thresholds_for
+    float est_lo = 0.0f, est_hi = 0.0f, est_slack = 0.0f;
 };
-int batch_rdf(const BatchGrid& G, int R, float r_max, uint32_t bins, const BatchRdfScratch& S, uint32_t* d_counts);
+int batch_rdf(const BatchGrid& G, const uint32_t* d_tile_frame, uint32_t ntiles, int R, float r_max, uint32_t bins,
+              const BatchRdfScratch& S, uint32_t* d_counts);
 // The bins + 1 r_sq thresholds of RegularAxis(bins, 0, r_max) binning of
-// sqrt(r_sq), computed on the host and copied (synchronously) to d_T.
-int thresholds_for(uint32_t bins, float r_max, float* d_T);
+// sqrt(r_sq), computed on the host and copied (synchronously) to d_T; sets the
+// estimate range of S.
+int thresholds_for(uint32_t bins, float r_max, float* d_T, BatchRdfScratch& S);
 // Floats of the bin table thresholds_for writes (thresholds + lookup table).
 size_t rdf_table_floats(uint32_t bins);
 int batch_steinhardt(const BatchGrid& G, const uint32_t* d_tile_frame, uint32_t ntiles, const float* d_pts,

@@ -14,8 +14,12 @@
 // own expression.  A kernel estimates the bin with the hardware square root and
 // corrects it against T, giving exactly the reference's bin.
 //
-// Self RDF (query points == points, AABB formula, all points inside the box):
-// a cluster-pair kernel over cells at least r_max/2 wide; each wave takes a
+// RDF over AABB queries (up to kEstMaxBins bins over the query's own range): the
+// pair kernel of rows_est below, over row clusters, on estimates of r_sq that
+// fall back to the reference's arithmetic near a bin's threshold.
+//
+// Self RDF with more bins or a narrower query (query points == points, AABB
+// formula, all points inside the box): a cluster-pair kernel over cells at least r_max/2 wide; each wave takes a
 // cluster of up to 8 cell-ordered points and its 64 lanes test 8 x 8 pairs per
 // step against 8-point chunks of the 5x5x5 stencil cells.  For two cells related
 // without a periodic shift the AABB formula gives bitwise-equal r_sq for (i,j)
@@ -99,9 +103,67 @@ uint32_t lut_cell(float x, float inv_delta)
     return q >= float(kLut) ? kLut : uint32_t(q);
 }
 
-__host__ __device__ constexpr uint32_t table_floats(uint32_t nbins)
+__host__ __device__ constexpr uint32_t exact_table_floats(uint32_t nbins)
 {
     return nbins + 3 + uint32_t((kLut * sizeof(uint16_t) + sizeof(float) - 1) / sizeof(float));
+}
+
+// Estimate table (up to kEstMaxBins bins), behind the exact one.  The pair
+// kernels bin an estimate x' of r_sq whose distance from the reference's r_sq
+// is at most a bound eps that the kernel knows, and fall back to the
+// reference's own arithmetic where that leaves the bin open.  Cell c covers
+// the x' that round to c in units of 1 / inv (inv = (kEstCells - 2) / T[nbins]).
+// Histogram words: 0 below T[0], 1 + bin, nbins + 1 at or above T[nbins].  A
+// cell's entry (t, a) says: the word is a / 4 - 1 for x' <= t - eps and a / 4
+// for x' >= t + eps; in between, and in cells with t = NaN (more than one
+// threshold), it is open.  A cell is widened by a quarter of its width on each
+// side before its thresholds are counted, so eps may be up to kEstEps cells.
+constexpr uint32_t kEstCells = 2048;
+constexpr uint32_t kEstMaxBins = 512;
+constexpr float kEstEps = 0.24f;
+__host__ __device__ constexpr uint32_t est_table_start(uint32_t nbins)
+{
+    return (exact_table_floats(nbins) + 3u) & ~3u; // 16-byte aligned
+}
+__host__ __device__ constexpr uint32_t table_floats(uint32_t nbins)
+{
+    // inv, x_open, 2 pad, then kEstCells entries of two words
+    return nbins <= kEstMaxBins ? est_table_start(nbins) + 4u + 2u * kEstCells : exact_table_floats(nbins);
+}
+
+void build_est_table(float* tab, uint32_t nbins)
+{
+    const float* T = tab;
+    float* const est = tab + est_table_start(nbins);
+    float const tn = T[nbins];
+    est[0] = est[1] = est[2] = est[3] = 0.0f;
+    if (!(tn > 0.0f) || !std::isfinite(tn))
+        return; // inv = 0: the estimate kernels are not used
+    float const inv = float(double(kEstCells - 2) / double(tn));
+    if (!(inv > 0.0f) || !std::isfinite(inv))
+        return;
+    est[0] = inv;
+    for (uint32_t c = 0; c < kEstCells; ++c) // the last cell is set below
+    {
+        double const a = (double(c) - 0.7501) / double(inv), b = (double(c) + 0.7501) / double(inv);
+        const float* const first = std::lower_bound(T, T + nbins + 1, a, [](float t, double x) { return double(t) < x; });
+        const float* const last = std::upper_bound(T, T + nbins + 1, b, [](double x, float t) { return x < double(t); });
+        uint32_t const below = uint32_t(first - T); // thresholds under the cell = word of its smallest x'
+        size_t const inside = size_t(last - first);
+        float t = std::numeric_limits<float>::infinity();
+        uint32_t word = below + 1; // the word is word - 1 for every x' < infinity
+        if (inside == 1)
+            t = *first;
+        else if (inside > 1)
+            t = std::numeric_limits<float>::quiet_NaN();
+        if (inside > 1 && c + 1 < kEstCells)
+            est[1] = float(b); // x_open: the far end of the last such cell
+        if (c + 1 == kEstCells)
+            t = std::numeric_limits<float>::quiet_NaN();
+        uint32_t const addr = 4u * word;
+        std::memcpy(&est[4 + 2 * c], &t, sizeof(float));
+        std::memcpy(&est[4 + 2 * c + 1], &addr, sizeof(float));
+    }
 }
 
 std::vector<float> build_table(uint32_t nbins, float vmin, float vmax)
@@ -112,6 +174,8 @@ std::vector<float> build_table(uint32_t nbins, float vmin, float vmax)
     float* T = tab.data();
     for (uint32_t k = 0; k <= nbins; ++k)
         T[k] = first_rsq_with_bin_at_least(int(k), vmin, vmax, inv_width, nbins);
+    if (nbins <= kEstMaxBins)
+        build_est_table(T, nbins);
     float const tn = T[nbins];
     float inv_delta = 0.0f;
     if (tn > 0.0f && std::isfinite(tn))
@@ -177,6 +241,8 @@ struct Thresholds
     size_t cap = 0;
     uint32_t nbins = 0;
     float vmin = 0, vmax = 0;
+    float first = 0, last = 0; // T[0], T[nbins]
+    bool est = false;          // an estimate table follows
 };
 Thresholds g_thr;
 
@@ -200,6 +266,9 @@ int thresholds(uint32_t nbins, float vmin, float vmax, float** d_out)
     g_thr.nbins = nbins;
     g_thr.vmin = vmin;
     g_thr.vmax = vmax;
+    g_thr.first = tab[0];
+    g_thr.last = tab[nbins];
+    g_thr.est = nbins <= kEstMaxBins && tab[est_table_start(nbins)] > 0.0f;
     *d_out = g_thr.dev;
     return FA_OK;
 }
@@ -766,6 +835,498 @@ __device__ inline void rows_body(const DevBox& b, const DevGrid& g, uint32_t row
     }
 }
 
+// ------------------------------------------------------------------ row clusters, estimated r_sq
+// What bounds the pair kernel is VALU issue: the reference's r_sq (none of its
+// products and sums fused) and its exact bin cost about 20 instructions per
+// candidate pair, of which only a third lies in range.  Almost no pair needs
+// them: an estimate x' of r_sq from fused products is a few ulps off, far less
+// than the width of a bin in r_sq.  A pair whose x' lies at least eps from the
+// threshold of its table cell has the reference's bin whichever way either is
+// rounded; the others are evaluated and binned as the reference does it.  The
+// counts are the reference's bit for bit.  1,048,576 lattice points, r_max = 5,
+// 200 bins: 0.755 -> 0.652 ms (the exact kernel below); 17.7 M points in 256
+// frames: 23.4 -> 20.8 ms for the whole batch.  What is left is VALU issue (55 %
+// of the cycles) and the waits at each cluster's start.
+//
+// eps: unshifted pairs take the reference's own differences, and x' and its
+// r_sq are each within 3 x 2^-24 of their exact sum of squares (7 x 2^-24
+// covers both).  Across the box edge the reference rounds q + image, the
+// estimate p - image, both at the scale of the box: with |p|, |q| <= D the
+// vectors differ by less than 2^-24 (2 D + 2 r_max), which moves r_sq by up to
+// twice that times r_max (8 x 2^-24 r_max (D + r_max) covers it).
+struct EstBins
+{
+    uint32_t cells;    // LDS address of the cell table - (bits of 2^23) * 8
+    uint32_t hist;     // LDS address of the histogram's word 0
+    uint32_t wave_off; // WAVE_HIST: offset of the wave's histogram from `hist`
+    float inv, x_open;
+    const float* T; // exact thresholds (device memory)
+    uint32_t nbins;
+    float vmin, inv_width;
+    float lo, hi; // pairs counted: lo <= r_sq < hi
+    float slack;  // how far lo and hi lie inside the table's range
+};
+
+template<bool WAVE_HIST> __device__ __forceinline__ void est_atomic(const EstBins& B, uint32_t a, uint32_t w)
+{
+    __atomic_fetch_add((lds_u32*) (uintptr_t) (WAVE_HIST ? a + B.wave_off : a), w, __ATOMIC_RELAXED);
+}
+
+// the table cell of an estimate of at most kEstCells - 1 cells
+__device__ __forceinline__ uint64_t est_cell(const EstBins& B, float x)
+{
+    uint32_t const y = __float_as_uint(__builtin_fmaf(x, B.inv, 8388608.0f));
+    typedef __attribute__((address_space(3))) const uint64_t lds_cu64;
+    return *(lds_cu64*) (uintptr_t) ((y << 3) + B.cells);
+}
+
+// the histogram word (LDS address) on the side of the cell's threshold that d
+// (estimate minus threshold) lies on
+__device__ __forceinline__ uint32_t est_word(uint64_t cell, float d)
+{
+    int below = __float_as_int(d) >> 31; // -1 under the threshold, 0 from it on
+    asm("" : "+v"(below));               // keeps the shift and the sum one instruction
+    return (uint32_t(below) << 2) + uint32_t(cell >> 32);
+}
+
+// one r_sq as the reference computes it: the threshold's side is exact
+template<bool WAVE_HIST> __device__ __forceinline__ void est_exact(const EstBins& B, float x, uint32_t w)
+{
+    if (x >= B.lo && x < B.hi)
+    {
+        uint64_t const cell = est_cell(B, x);
+        float const t = __uint_as_float(uint32_t(cell));
+        uint32_t a = est_word(cell, x - t);
+        if (t != t) // several thresholds in the cell
+            a = B.hist + 4u * (1u + bin_in_range(x, B.T, B.nbins, B.vmin, B.inv_width));
+        est_atomic<WAVE_HIST>(B, a, w);
+    }
+}
+
+// One wave's share of a cluster (cells cx_lo .. cx_hi of row (cy0, cz0), na
+// points from A0 on) of the query points qpos against the points `g` (two
+// grids of one shape): the stencil rows with index s mod `split` (split waves
+// share a cluster where clusters are few).
+//
+// HALF (the query points are the points): every unordered pair once.
+// Unshifted pairs are counted from the point earlier in cell order, pairs
+// across the box edge from the side whose image code is above 13, with weight
+// 2: for the latter the reference's two r_sq differ in rounding only, so an
+// estimate eps away from a threshold bins both, and an open one evaluates the
+// two directions.  !HALF: every (query, point, image) once, weight 1.
+//
+// Lane t resolves stencil row r0 + t into pieces that share an image each (the
+// cstart reads of all rows are in flight together).  The pieces of one kind are
+// concatenated in row order and taken 64 candidates at a time, one per lane,
+// against the cluster's query points in scalar registers, four table look-ups
+// in flight at once.
+//
+// pa: query point lane / 8 (of A0 + min(lane / 8, na - 1)).  prefetch() is called
+// once the first rows are resolved, ahead of the pair work, to load what the
+// next cluster starts from.
+template<int R, bool IS2D, bool HALF, bool WAVE_HIST, class Prefetch>
+__device__ inline void rows_est(const DevBox& b, const DevGrid& g, float4 pa, int cy0, int cz0, uint32_t A0,
+                                uint32_t na, int cx_lo, int cx_hi, int RX, uint32_t s, uint32_t split, const EstBins& B,
+                                Prefetch&& prefetch)
+{
+    constexpr int kRowsY = 2 * R + 1;
+    constexpr int Rz = IS2D ? 0 : R;
+    constexpr int nrows = kRowsY * (2 * Rz + 1);
+    constexpr uint32_t W = HALF ? 2u : 1u;
+    constexpr float kUlp = 0x1p-24f;
+    uint32_t const lane = threadIdx.x & 63u;
+    int const dim0 = g.dim[0], dim1 = g.dim[1], dim2 = g.dim[2];
+    uint32_t const a = lane >> 3, bl = lane & 7u;
+    if (IS2D)
+        pa.z = 0.0f;
+    // query point k, wave-uniform
+    auto query = [&](float v, uint32_t k) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), int(8u * k)));
+    };
+    if (HALF && s == 0)
+    {
+        // pairs within the cluster: lane (a, bl) with a < bl < na, no image
+        float const rx = __shfl(pa.x, int(8u * bl)) - pa.x, ry = __shfl(pa.y, int(8u * bl)) - pa.y;
+        float x = rx * rx + ry * ry;
+        if constexpr (!IS2D)
+        {
+            float const rz = __shfl(pa.z, int(8u * bl)) - pa.z;
+            x = x + rz * rz;
+        }
+        if (bl > a && bl < na)
+            est_exact<WAVE_HIST>(B, x, 2u);
+    }
+    // the cluster's points, in vector registers (24 more scalar ones would
+    // spill, and be read back with VALU instructions); NaN past na
+    float qx[8], qy[8], qz[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k)
+    {
+        qx[k] = k < na ? query(pa.x, k) : __builtin_nanf("");
+        qy[k] = query(pa.y, k);
+        qz[k] = IS2D ? 0.0f : query(pa.z, k);
+        asm("" : "+s"(qx[k]), "+s"(qy[k]), "+s"(qz[k]));
+    }
+    float const r_lim = __builtin_amdgcn_sqrtf(B.hi) * 1.0001f;
+    float const D = 0.5f * (b.L[0] + b.L[1] * (1.0f + fabsf(b.xy)) + b.L[2] * (1.0f + fabsf(b.xz) + fabsf(b.yz)));
+    float const eps_in = 7.0f * kUlp * B.hi + B.slack;
+    float const eps_edge = eps_in + 8.0f * kUlp * (r_lim * (D + r_lim));
+    float const eps_most = kEstEps / B.inv, x_last = float(kEstCells - 1) / B.inv, x_open = B.x_open;
+    __amdgpu_buffer_rsrc_t const rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float4*>(g.cpos), short(0), -1, kBufferWord3);
+    // The concatenated candidates of one kind: lane t's row holds the
+    // positions [beg, beg + len) of image `code`.
+    auto run = [&](uint32_t beg, uint32_t len, int code, auto shifted) {
+        constexpr bool SHIFTED = decltype(shifted)::value;
+        uint32_t const p = wave_exclusive_scan(len); // virtual start of row t's candidates
+        uint32_t const e = p + len;
+        uint32_t const sh = beg - p; // position = virtual index + sh within row t
+        uint32_t const tot = uint32_t(__builtin_amdgcn_readlane(int(e), 63));
+        if (tot == 0)
+            return;
+        uint64_t live = __builtin_amdgcn_ballot_w64(len > 0u); // rows not yet exhausted
+        int lcode = 13;
+        auto locate = [&](uint32_t v0) {
+            uint32_t const v = v0 + lane;
+            int const first = __builtin_ctzll(live);
+            uint32_t pos = v + uint32_t(__builtin_amdgcn_readlane(int(sh), first));
+            if (SHIFTED)
+                lcode = __builtin_amdgcn_readlane(code, first);
+            for (uint64_t m = live & (live - 1u); m; m &= m - 1u)
+            {
+                int const r = __builtin_ctzll(m);
+                uint32_t const sp = uint32_t(__builtin_amdgcn_readlane(int(p), r));
+                if (sp >= v0 + 64u)
+                    break;
+                uint32_t const p2 = v + uint32_t(__builtin_amdgcn_readlane(int(sh), r));
+                pos = v >= sp ? p2 : pos;
+                if (SHIFTED)
+                {
+                    int const c2 = __builtin_amdgcn_readlane(code, r);
+                    lcode = v >= sp ? c2 : lcode;
+                }
+            }
+            while (live && uint32_t(__builtin_amdgcn_readlane(int(e), __builtin_ctzll(live))) <= v0 + 64u)
+                live &= live - 1u;
+            return pos;
+        };
+        auto fetch = [&](uint32_t pos) {
+            return __builtin_amdgcn_raw_buffer_load_b128(rs, pos * uint32_t(sizeof(float4)), 0u, 0);
+        };
+        float const eps = SHIFTED ? eps_edge : eps_in;
+        float const hi_p = B.hi + eps;
+        bool const usable = eps <= eps_most;
+        auto cvn = fetch(locate(0u));
+        for (uint32_t v0 = 0; v0 < tot; v0 += 64u)
+        {
+            auto const cv = cvn;
+            int const im = lcode;
+            if (v0 + 64u < tot)
+                cvn = fetch(locate(v0 + 64u));
+            bool const exists = v0 + lane < tot;
+            float const cy = __uint_as_float(cv[1]);
+            float const cz = IS2D ? 0.0f : __uint_as_float(cv[2]);
+            float const cx = exists ? __uint_as_float(cv[0]) : __builtin_nanf(""); // fails every compare below
+            float ix = 0.0f, iy = 0.0f, iz = 0.0f;
+            if (SHIFTED)
+            {
+                ix = b.img[im][0];
+                iy = b.img[im][1];
+                iz = b.img[im][2];
+            }
+            float const vx = SHIFTED ? cx - ix : cx, vy = SHIFTED ? cy - iy : cy, vz = SHIFTED ? cz - iz : cz;
+            // estimate of query point k (entries past na: NaN)
+            auto estimate = [&](float ux, float uy, float uz) {
+                float const rx = vx - ux, ry = vy - uy;
+                if constexpr (IS2D)
+                    return __builtin_fmaf(rx, rx, ry * ry);
+                float const rz = vz - uz;
+                return __builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, rz * rz));
+            };
+            // its table cell; beyond the table (and for NaN) the last one
+            auto cell_of = [&](float x) { return est_cell(B, fminf(x, x_last)); };
+            float d_min = INFINITY, x_min = INFINITY; // nearest threshold, smallest estimate
+            if (usable)
+            {
+#pragma unroll
+                for (int k0 = 0; k0 < 8; k0 += 4)
+                {
+                    if (uint32_t(k0) >= na)
+                        break;
+                    float x[4];
+                    uint64_t cell[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                    {
+                        x[u] = estimate(qx[k0 + u], qy[k0 + u], qz[k0 + u]);
+                        cell[u] = cell_of(x[u]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                    {
+                        float const d = x[u] - __uint_as_float(uint32_t(cell[u]));
+                        d_min = fminf(d_min, fabsf(d));
+                        x_min = fminf(x_min, x[u]);
+                        if (fabsf(d) >= eps)
+                            est_atomic<WAVE_HIST>(B, est_word(cell[u], d), W);
+                    }
+                }
+            }
+            // Blocks with an open pair: the reference's arithmetic for those.
+            bool const some = usable ? d_min < eps || x_min < x_open : exists;
+            if (__builtin_amdgcn_ballot_w64(some))
+            {
+                for (uint32_t k = 0; k < na; ++k)
+                {
+                    float const ux = query(pa.x, k), uy = query(pa.y, k), uz = query(pa.z, k);
+                    bool open = some;
+                    if (usable)
+                    {
+                        float const x = estimate(ux, uy, uz);
+                        open = some && x < hi_p && !(fabsf(x - __uint_as_float(uint32_t(cell_of(x)))) >= eps);
+                    }
+                    if (!open)
+                        continue;
+                    float const rx = cx - (SHIFTED ? ux + ix : ux), ry = cy - (SHIFTED ? uy + iy : uy);
+                    float const rz = cz - (SHIFTED ? uz + iz : uz);
+                    float x = rx * rx + ry * ry;
+                    if constexpr (!IS2D)
+                        x = x + rz * rz;
+                    est_exact<WAVE_HIST>(B, x, SHIFTED ? 1u : W);
+                    if constexpr (SHIFTED && HALF)
+                    {
+                        // the other direction: point c as the query, the image reversed
+                        float const bx = ux - vx, by = uy - vy, bz = uz - vz;
+                        x = bx * bx + by * by;
+                        if constexpr (!IS2D)
+                            x = x + bz * bz;
+                        est_exact<WAVE_HIST>(B, x, 1u);
+                    }
+                }
+            }
+        }
+    };
+    // the cluster's extent
+    float xmn = qx[0], xmx = qx[0], ymn = qy[0], ymx = qy[0], zmn = qz[0], zmx = qz[0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k)
+    {
+        xmn = fminf(xmn, qx[k]);
+        xmx = fmaxf(xmx, qx[k]);
+        ymn = fminf(ymn, qy[k]);
+        ymx = fmaxf(ymx, qy[k]);
+        zmn = fminf(zmn, qz[k]);
+        zmx = fmaxf(zmx, qz[k]);
+    }
+    float const wx = g.cw[0] * 0.9999f, wy = g.cw[1] * 0.9999f, wz = g.cw[2] * 0.9999f;
+    bool const ortho = b.xy == 0.0f && b.xz == 0.0f && b.yz == 0.0f;
+    float const mgx = 1e-5f * b.L[0], mgy = 1e-5f * b.L[1], mgz = 1e-5f * b.L[2];
+    // u mod dim for -dim <= u < 2 dim: the shift in box lengths (2 when farther)
+    auto shift_of = [](int u, int dim) { return u < 0 ? (u >= -dim ? -1 : 2) : (u < dim ? 0 : u < 2 * dim ? 1 : 2); };
+    for (int r0 = 0; r0 < nrows; r0 += 64)
+    {
+        // lane t: stencil row r0 + t, cells u0 .. u1 (unwrapped; none if u1 < u0)
+        int u0 = 0, u1 = -1, sy = 0, sz = 0;
+        uint32_t rowbase = 0;
+        int const rt = r0 + int(lane);
+        if (rt < nrows && (split == 1u || uint32_t(rt) % split == s))
+        {
+            int const dz = rt / kRowsY - Rz, dy = rt % kRowsY - R;
+            int const ucz = cz0 + dz, ucy = cy0 + dy;
+            sz = shift_of(ucz, dim2);
+            sy = shift_of(ucy, dim1);
+            float gy = float(max(0, abs(dy) - 1)) * wy, gz = float(max(0, abs(dz) - 1)) * wz;
+            int xr = RX;
+            bool reach = sz != 2 && sy != 2;
+            int ux_lo = -dim0, ux_hi = 2 * dim0 - 1;
+            if (ortho)
+            {
+                // as in rows_body: the slab's gap to the cluster's extent
+                // (hardware square root and reciprocal: the margins of r_lim
+                // and mgx are a hundred times their error)
+                float const ys = b.lo[1] + float(ucy) * g.cw[1];
+                gy = fmaxf(gy, fmaxf(ys - ymx, ymn - (ys + g.cw[1])) - mgy);
+                if constexpr (!IS2D)
+                {
+                    float const zs = b.lo[2] + float(ucz) * g.cw[2];
+                    gz = fmaxf(gz, fmaxf(zs - zmx, zmn - (zs + g.cw[2])) - mgz);
+                }
+                float const rem = r_lim * r_lim - (gy * gy + gz * gz);
+                reach = reach && rem > 0.0f;
+                if (reach && wx > 0.0f)
+                {
+                    float const h = __builtin_amdgcn_sqrtf(rem) * 1.00001f;
+                    float const ix = __builtin_amdgcn_rcpf(g.cw[0]);
+                    xr = min(RX, int(h * ix * 1.0002f) + 1);
+                    ux_lo = int(fmaxf(floorf((xmn - h - mgx - b.lo[0]) * ix), float(-dim0)));
+                    ux_hi = int(fminf(floorf((xmx + h + mgx - b.lo[0]) * ix), float(2 * dim0 - 1)));
+                }
+            }
+            else
+                reach = reach && fmaxf(gy, gz) < r_lim;
+            if (reach)
+            {
+                rowbase = uint32_t((ucz - sz * dim2) * dim1 + (ucy - sy * dim1)) * uint32_t(dim0);
+                // shifts beyond one box length are not images the reference visits
+                u0 = max(max(cx_lo - xr, -dim0), ux_lo);
+                u1 = min(min(cx_hi + xr, 2 * dim0 - 1), ux_hi);
+            }
+        }
+        // the row's piece shifted by sx box lengths
+        auto piece = [&](int sx, uint32_t& beg, uint32_t& len) {
+            int const c0 = max(u0, sx * dim0) - sx * dim0, c1 = min(u1, sx * dim0 + dim0 - 1) - sx * dim0;
+            beg = len = 0u;
+            if (c0 <= c1)
+            {
+                beg = g.cstart[rowbase + uint32_t(c0)];
+                len = g.cstart[rowbase + uint32_t(c1) + 1u] - beg;
+            }
+        };
+        // AABB formula: r = p_j - (q_i + image), image = -shift
+        auto code_of = [&](int sx) { return (1 - sx) * 9 + (1 - sy) * 3 + (1 - sz); };
+        bool const plain = sy == 0 && sz == 0;
+        uint32_t beg, len;
+        piece(0, beg, len);
+        if (r0 == 0)
+            prefetch();
+        {
+            uint32_t ub = beg, ul = plain ? len : 0u;
+            if (HALF) // from the point after the cluster on
+            {
+                uint32_t const end = ub + ul;
+                ub = max(ub, A0 + na);
+                ul = end > ub ? end - ub : 0u;
+            }
+            run(ub, ul, 13, std::false_type{});
+        }
+        for (int sx = -1; sx <= (HALF ? 0 : 1); ++sx)
+        {
+            piece(sx, beg, len);
+            int const code = code_of(sx);
+            if (code == 13 || (HALF && code < 13))
+                len = 0u;
+            if (__builtin_amdgcn_ballot_w64(len > 0u))
+                run(beg, len, code, std::true_type{});
+        }
+    }
+}
+
+// A wave's cluster entries `item`, item + step, .. below `items` (entry =
+// item / split, its rows s = item mod split), estimated r_sq.  The next entry
+// and its points are loaded during the current one's pair work: a cluster's
+// start is otherwise a chain of dependent loads (entry, points, cell starts,
+// candidates) about as long as its pair work.
+template<int R, bool IS2D, bool HALF, bool WAVE_HIST, class Begin>
+__device__ inline void rows_est_items(const DevBox& b, const DevGrid& g, const DevGrid& gq,
+                                      const uint4* __restrict__ table, uint32_t item, uint32_t step, uint32_t items,
+                                      int RX, uint32_t split, Begin&& begin)
+{
+    uint32_t const a = (threadIdx.x & 63u) >> 3;
+    auto point = [&](const uint4& e) { return gq.cpos[e.y + min(a, e.z - 1u)]; };
+    bool const any = item < items;
+    uint4 e = any ? table[item / split] : make_uint4(0u, 0u, 1u, 0u);
+    float4 pa = any ? point(e) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    EstBins const B = begin();
+    for (; item < items; item += step)
+    {
+        uint32_t const s = item % split;
+        uint32_t const row = __builtin_amdgcn_readfirstlane(e.x);
+        uint32_t const A0 = __builtin_amdgcn_readfirstlane(e.y);
+        uint32_t const na = __builtin_amdgcn_readfirstlane(e.z);
+        uint32_t const cx = __builtin_amdgcn_readfirstlane(e.w);
+        float4 const q = pa;
+        bool const more = item + step < items;
+        if (more)
+            e = table[(item + step) / split];
+        rows_est<R, IS2D, HALF, WAVE_HIST>(b, g, q, int(row % uint32_t(g.dim[1])), int(row / uint32_t(g.dim[1])), A0,
+                                           na, int(cx & 0xffffu), int(cx >> 16), RX, s, split, B, [&]() {
+                                               if (more)
+                                                   pa = point(e);
+                                           });
+    }
+}
+
+// LDS: the cell table, then the histogram(s) of nbins + 2 words.
+__host__ __device__ constexpr size_t est_lds_bytes(uint32_t nbins, uint32_t hists)
+{
+    return sizeof(uint32_t) * (2 * size_t(kEstCells) + size_t(nbins + 2) * hists);
+}
+
+__device__ inline EstBins est_prologue(uint32_t* smem, const float* __restrict__ T, uint32_t nbins, uint32_t hists,
+                                       float vmin, float inv_width, float lo, float hi, float slack)
+{
+    uint32_t* const hist = smem + 2 * kEstCells;
+    uint32_t const base = lds_addr(hist);
+    const uint4* __restrict__ const src = reinterpret_cast<const uint4*>(T + est_table_start(nbins) + 4);
+    uint4* const dst = reinterpret_cast<uint4*>(smem);
+    for (uint32_t t = threadIdx.x; t < kEstCells / 2; t += blockDim.x)
+    {
+        uint4 v = src[t];
+        v.y += base;
+        v.w += base;
+        dst[t] = v;
+    }
+    for (uint32_t t = threadIdx.x; t < (nbins + 2) * hists; t += blockDim.x)
+        hist[t] = 0u;
+    __syncthreads();
+    uint32_t cells = lds_addr(smem) - (0x4b000000u << 3);
+    asm("" : "+s"(cells)); // a register, so that shift and sum are one instruction
+    return EstBins{cells, base, 0u, T[est_table_start(nbins)], T[est_table_start(nbins) + 1], T, nbins, vmin, inv_width,
+                   lo, hi, slack};
+}
+
+// Each workgroup takes kWaves * per_wave consecutive items (waves interleaved).
+template<int R, bool IS2D, bool HALF>
+__global__ __launch_bounds__(kBlock, 6) void rdf_est_kernel(DevBox b, DevGrid g, DevGrid gq,
+                                                            const uint4* __restrict__ table,
+                                                            const uint32_t* __restrict__ ncl_ptr, uint32_t split,
+                                                            uint32_t per_wave, int RX, float lo, float hi, float slack,
+                                                            const float* __restrict__ T, uint32_t nbins, float vmin,
+                                                            float inv_width, uint32_t* __restrict__ counts)
+{
+    extern __shared__ __align__(16) float smem[];
+    constexpr uint32_t kWaves = kBlock / 64;
+    uint32_t const first = fa::xcd_tile(blockIdx.x, gridDim.x) * (kWaves * per_wave), all = *ncl_ptr * split;
+    // The grid covers the largest possible cluster count.  Points outside the
+    // box have image offsets of their own: rdf_outside_kernel takes the system.
+    if (first >= all || *g.outside || (!HALF && *gq.outside))
+        return;
+    uint32_t* const words = reinterpret_cast<uint32_t*>(smem);
+    rows_est_items<R, IS2D, HALF, false>(b, g, gq, table, first + (threadIdx.x >> 6), kWaves,
+                                         min(all, first + kWaves * per_wave), RX, split,
+                                         [&]() { return est_prologue(words, T, nbins, 1, vmin, inv_width, lo, hi, slack); });
+    hist_epilogue<true>(words + 2 * kEstCells + 1, nbins, counts);
+}
+
+// The systems rdf_est_kernel leaves out: one thread per query point walks its
+// stencil with every point's own image offset, each ordered pair once.
+template<bool HALF>
+__global__ __launch_bounds__(kBlock) void rdf_outside_kernel(DevBox b, DevGrid g, DevGrid gq, uint32_t nq, int R,
+                                                             int RX, float lo, float hi, const float* __restrict__ T,
+                                                             uint32_t nbins, float vmin, float inv_width,
+                                                             uint32_t* __restrict__ counts)
+{
+    if (!*g.outside && (HALF || !*gq.outside))
+        return;
+    extern __shared__ uint32_t hist_only[];
+    for (uint32_t t = threadIdx.x; t < nbins; t += blockDim.x)
+        hist_only[t] = 0u;
+    __syncthreads();
+    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < nq; t += gridDim.x * blockDim.x)
+    {
+        float4 const q = gq.cpos[t];
+        uint32_t const qi = __float_as_uint(q.w);
+        fa::for_each_candidate<AABB_FORMULA>(
+            b, g, q.x, q.y, q.z, R, false,
+            [&](uint32_t j, float, float, float, float r_sq, int) {
+                if (!(HALF && j == qi) && r_sq >= lo && r_sq < hi)
+                    atomicAdd(&hist_only[bin_in_range(r_sq, T, nbins, vmin, inv_width)], 1u);
+            },
+            RX);
+    }
+    hist_epilogue<true>(hist_only, nbins, counts);
+}
+
 // The pair work of one cluster entry e = (frame-local row, start, count,
 // cx_lo | cx_hi << 16) for one wave (e is wave-uniform).
 template<int R, class Bins>
@@ -948,10 +1509,12 @@ __global__ void add_self_pairs_kernel(uint32_t* counts, uint32_t bin, uint32_t n
         counts[bin] += n;
 }
 
+struct EstRange;
 struct RowsArgs
 {
     fa_nq* nq;
     float qmax_sq, qmin_sq;
+    const EstRange* est;
     const float* T;
     uint32_t bins;
     float r_min, inv_width, q_r_max;
@@ -997,15 +1560,44 @@ struct RowsBuffers
 inline uint64_t rows_max_clusters(uint32_t n, uint32_t nrows) { return uint64_t(n) / 8 + nrows; }
 
 // The cluster table of a built grid, then the row-cluster kernel.
-int launch_rows(const DevBox& db, const DevGrid& g, const int dims[3], int R, int F, uint32_t n,
-                const RowsBuffers& B, float qmax_sq, float qmin_sq, const float* T, uint32_t bins, float r_min,
-                float inv_width, uint32_t* d_counts)
+// est: the estimate kernel's range (lo < hi), or its hi = 0 for the exact kernel.
+// gq: the query points' grid (of the same shape), nullptr for a self RDF;
+// n: the number of query points.
+struct EstRange
+{
+    float lo = 0.0f, hi = 0.0f, slack = 0.0f;
+};
+
+// Waves per cluster: clusters of a small system leave the chip idle (4096
+// points: 600 waves on 256 CUs x 32), so up to 8 waves share one.
+uint32_t rows_split(uint32_t n)
+{
+    uint32_t split = 1;
+    while (split < 8 && uint64_t(n) / 8 * split * 2 <= 8192)
+        split *= 2;
+    return split;
+}
+
+// Clusters per wave, one after the other: fewer workgroups copy the table and
+// add their histogram to the counts, and a cluster's first loads overlap its
+// predecessor's pair work.  1,048,576 points: one 0.78 ms, two 0.65, four 0.66,
+// eight 0.76 (the last waves run longer); one while two would leave less than
+// two rounds of resident waves (6 x 1024).
+uint32_t rows_per_wave(uint64_t items)
+{
+    return items >= 4 * 6144 ? 2 : 1;
+}
+
+int launch_rows(const DevBox& db, const DevGrid& g, const DevGrid* gq, const int dims[3], int R, int F, uint32_t n,
+                const RowsBuffers& B, float qmax_sq, float qmin_sq, const EstRange& est, const float* T, uint32_t bins,
+                float r_min, float inv_width, uint32_t* d_counts)
 {
     hipStream_t s = fa::stream();
+    const uint32_t* const qstart = gq ? gq->cstart : g.cstart;
     uint32_t const nrows = uint32_t(dims[1]) * uint32_t(dims[2]);
     uint64_t const max_clusters = rows_max_clusters(n, nrows);
     unsigned const rblocks = (nrows + kBlock - 1) / kBlock;
-    FA_KLAUNCH(row_cluster_count_kernel, dim3(rblocks), dim3(kBlock), 0, s, g.cstart, uint32_t(dims[0]), nrows,
+    FA_KLAUNCH(row_cluster_count_kernel, dim3(rblocks), dim3(kBlock), 0, s, qstart, uint32_t(dims[0]), nrows,
                B.nclus);
     if (B.scan_tmp)
     {
@@ -1015,8 +1607,49 @@ int launch_rows(const DevBox& db, const DevGrid& g, const int dims[3], int R, in
     else if (int rc = fa::exclusive_scan_u32(B.nclus, B.cl_off, nrows, nullptr))
         return rc;
     unsigned const tblocks = unsigned((max_clusters + kBlock - 1) / kBlock);
-    FA_KLAUNCH(row_cluster_table_kernel, dim3(tblocks), dim3(kBlock), 0, s, g.cstart, uint32_t(dims[0]), nrows,
+    FA_KLAUNCH(row_cluster_table_kernel, dim3(tblocks), dim3(kBlock), 0, s, qstart, uint32_t(dims[0]), nrows,
                B.cl_off, uint32_t(max_clusters), B.table);
+    if (est.hi > 0.0f)
+    {
+        uint32_t const split = rows_split(n);
+        uint32_t const per_wave = rows_per_wave(uint64_t(n) / 8 * split);
+        uint64_t const per_block = uint64_t(kBlock / 64) * per_wave;
+        unsigned const eblocks = unsigned((max_clusters * split + per_block - 1) / per_block);
+        size_t const lds = est_lds_bytes(bins, 1);
+        auto go = [&](auto kern, const DevGrid& query_grid) {
+            FA_PROF_BEGIN("rdf_est_kernel");
+            hipLaunchKernelGGL(kern, dim3(eblocks), dim3(kBlock), lds, s, db, g, query_grid, B.table, B.cl_off + nrows,
+                               split, per_wave, R * F, est.lo, est.hi, est.slack, T, bins, r_min, inv_width, d_counts);
+            FA_PROF_END();
+        };
+#define FA_EST(RR)                                                                                                  \
+    case RR:                                                                                                        \
+        if (gq)                                                                                                     \
+            db.is2D ? go(rdf_est_kernel<RR, true, false>, *gq) : go(rdf_est_kernel<RR, false, false>, *gq);         \
+        else                                                                                                        \
+            db.is2D ? go(rdf_est_kernel<RR, true, true>, g) : go(rdf_est_kernel<RR, false, true>, g);               \
+        break;
+        switch (R)
+        {
+            FA_EST(2)
+            FA_EST(3)
+            FA_EST(4)
+        default:
+            return fa::fail(FA_ERR_RUNTIME, "unsupported RDF cell ratio");
+        }
+#undef FA_EST
+        FA_HIP(hipGetLastError());
+        auto outside = [&](auto kern, const DevGrid& query_grid) {
+            FA_PROF_BEGIN("rdf_outside_kernel");
+            hipLaunchKernelGGL(kern, dim3(std::min<unsigned>((n + kBlock - 1) / kBlock, 2048u)), dim3(kBlock),
+                               sizeof(uint32_t) * bins, s, db, g, query_grid, n, R, R * F, est.lo, est.hi, T, bins,
+                               r_min, inv_width, d_counts);
+            FA_PROF_END();
+        };
+        gq ? outside(rdf_outside_kernel<false>, *gq) : outside(rdf_outside_kernel<true>, g);
+        FA_HIP(hipGetLastError());
+        return FA_OK;
+    }
     unsigned const wblocks = unsigned((max_clusters + kBlock / 64 - 1) / (kBlock / 64));
     bool const lds = bins <= kMaxLdsBins;
     size_t const shmem = lds ? sizeof(float) * lds_table_floats(bins) + sizeof(uint32_t) * bins : 0;
@@ -1040,6 +1673,25 @@ int launch_rows(const DevBox& db, const DevGrid& g, const int dims[3], int R, in
 #undef FA_ROWS
     FA_HIP(hipGetLastError());
     return FA_OK;
+}
+
+// The range the estimate kernel bins, when it applies: an estimate table, and
+// a query range that is the histogram's up to rounding (the two ends may
+// differ by ulps, which the error bound takes in as `slack`).  Other ranges
+// (a query radius below the histogram's) cut bins apart and take the exact
+// kernel.
+EstRange est_range(bool has_table, float first, float last, float qmax_sq, float qmin_sq)
+{
+    EstRange r;
+    float const lo = std::max(qmin_sq, first), hi = std::min(qmax_sq, last);
+    float const slack = (last - hi) + (lo - first);
+    if (has_table && hi > lo && slack <= 4.0e-7f * last)
+    {
+        r.lo = lo;
+        r.hi = hi;
+        r.slack = slack;
+    }
+    return r;
 }
 
 // Self RDF through the row-cluster kernel with cells at least r_max / R wide
@@ -1066,8 +1718,44 @@ int run_rows(const RowsArgs& a, RowVariant rv, uint32_t* d_counts, bool* handled
     B.nclus = static_cast<uint32_t*>(tmp);
     B.cl_off = B.nclus + (nrows + 1);
     B.table = reinterpret_cast<uint4*>(static_cast<char*>(tmp) + ((2 * rb + 15) & ~size_t(15)));
-    return launch_rows(nq->cur->dbox, nq->cur->dev(), dims, rv.R, F, nq->n, B, a.qmax_sq, a.qmin_sq, a.T, a.bins,
-                       a.r_min, a.inv_width, d_counts);
+    return launch_rows(nq->cur->dbox, nq->cur->dev(), nullptr, dims, rv.R, F, nq->n, B, a.qmax_sq, a.qmin_sq, *a.est,
+                       a.T, a.bins, a.r_min, a.inv_width, d_counts);
+}
+
+// RDF of distinct query points (AABB formula, no index exclusion): the query
+// points get a grid of the points' shape and are taken as row clusters of it,
+// against the points' rows.  One cell shape, (R, F) = (2, 8), the one the tuner
+// picks for self RDFs at 10 to 500 neighbours.  The thread-per-query kernel
+// below walks its candidates one by one, each a scattered load and an LDS
+// atomic of its own: 65,000 points and 35,000 query points, r_max = 5:
+// 1.29 -> 0.06 ms.
+int run_cross_rows(fa_nq* nq, const float* d_query, uint32_t n_query, float q_r_max, float qmax_sq, float qmin_sq,
+                   const EstRange& est, const float* T, uint32_t bins, float r_min, float inv_width,
+                   uint32_t* d_counts, bool* handled)
+{
+    *handled = false;
+    RowVariant const rv{2, 8};
+    int dims[3], F = 1;
+    if (uint64_t(n_query) + fa::kCposPad > (1ull << 28) || !rows_grid_dims(nq->box, nq->n, q_r_max, rv, dims, &F))
+        return FA_OK;
+    if (int rc = fa::ensure_grid(nq, dims))
+        return rc;
+    fa::Grid qgrid; // its buffers return to the allocator's cache, ordered on the stream
+    if (int rc = fa::build_grid(qgrid, nq->box, d_query, n_query, dims))
+        return rc;
+    *handled = true;
+    uint32_t const nrows = uint32_t(dims[1]) * uint32_t(dims[2]);
+    size_t const rb = sizeof(uint32_t) * (size_t(nrows) + 1);
+    void* tmp = nullptr;
+    if (int rc = fa::scratch(13, 2 * rb + sizeof(uint4) * rows_max_clusters(n_query, nrows) + 256, &tmp))
+        return rc;
+    RowsBuffers B{};
+    B.nclus = static_cast<uint32_t*>(tmp);
+    B.cl_off = B.nclus + (nrows + 1);
+    B.table = reinterpret_cast<uint4*>(static_cast<char*>(tmp) + ((2 * rb + 15) & ~size_t(15)));
+    DevGrid const gq = qgrid.dev();
+    return launch_rows(nq->cur->dbox, nq->cur->dev(), &gq, dims, rv.R, F, n_query, B, qmax_sq, qmin_sq, est, T, bins,
+                       r_min, inv_width, d_counts);
 }
 
 // ------------------------------------------------------------------ batches
@@ -1218,6 +1906,123 @@ __global__ __launch_bounds__(kBlock) void brdf_rows_kernel(fa::BatchGrid G, cons
         flush_wave_hist(wh, nbins, counts + size_t(cur) * nbins);
 }
 
+// The batched RDF over estimated r_sq (see rows_est): the queues of
+// brdf_rows_kernel, two clusters per chunk.  A chunk's entries and points are
+// loaded together, and the next chunk is taken from the queue before the
+// current one's pair work, so that neither the queue's atomic nor the loads
+// are waited for cluster by cluster.  Frames with points outside their box are
+// left to brdf_outside_kernel.
+template<int R>
+__global__ __launch_bounds__(kBlock, 6) void brdf_est_kernel(fa::BatchGrid G, const uint4* __restrict__ table,
+                                                             const uint32_t* __restrict__ cl_frame,
+                                                             const uint32_t* __restrict__ ncl_ptr,
+                                                             uint32_t* __restrict__ queue, float lo, float hi,
+                                                             float slack, const float* __restrict__ T, uint32_t nbins,
+                                                             float vmin, float inv_width,
+                                                             uint32_t* __restrict__ counts)
+{
+    static_assert(kChunk == 2, "two entries per chunk");
+    extern __shared__ __align__(16) float smem[];
+    constexpr uint32_t kWaves = kBlock / 64;
+    uint32_t const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    uint32_t* const words = reinterpret_cast<uint32_t*>(smem);
+    EstBins B = est_prologue(words, T, nbins, kWaves, vmin, inv_width, lo, hi, slack);
+    B.wave_off = wave * (nbins + 2) * uint32_t(sizeof(uint32_t));
+    uint32_t* const wh = words + 2 * kEstCells + wave * (nbins + 2) + 1;
+    uint32_t const ncl = *ncl_ptr;
+    uint32_t cur = 0xffffffffu;
+    uint32_t const x0 = blockIdx.x % fa::kXcds;
+    uint32_t xi = 0; // queue (x0 + xi) mod kXcds: the XCD's own range first, then the others'
+    auto take = [&]() {
+        uint32_t off = 0;
+        if (lane == 0 && xi < fa::kXcds)
+            off = atomicAdd(&queue[(x0 + xi) % fa::kXcds], kChunk);
+        return off;
+    };
+    uint32_t off = take();
+    while (xi < fa::kXcds)
+    {
+        uint32_t const x = (x0 + xi) % fa::kXcds;
+        uint32_t const r_lo = uint32_t((uint64_t(ncl) * x) / fa::kXcds);
+        uint32_t const r_hi = uint32_t((uint64_t(ncl) * (x + 1)) / fa::kXcds);
+        uint32_t const base = r_lo + __builtin_amdgcn_readfirstlane(off);
+        if (base >= r_hi)
+        {
+            ++xi; // this range is done: help the next XCD's
+            off = take();
+            continue;
+        }
+        off = take();
+        uint32_t const have = min(kChunk, r_hi - base);
+        uint4 const e0 = table[base], e1 = table[base + have - 1u];
+        uint32_t const f0 = __builtin_amdgcn_readfirstlane(cl_frame[base]),
+                       f1 = __builtin_amdgcn_readfirstlane(cl_frame[base + have - 1u]);
+        uint32_t const a = lane >> 3;
+        float4 const p0 = G.cpos[e0.y + min(a, e0.z - 1u)], p1 = G.cpos[e1.y + min(a, e1.z - 1u)];
+        for (uint32_t k = 0; k < have; ++k)
+        {
+            uint32_t const f = k ? f1 : f0;
+            const fa::BatchFrame& F = G.frames[f];
+            if (F.any_outside)
+                continue;
+            if (f != cur)
+            {
+                if (cur != 0xffffffffu)
+                    flush_wave_hist(wh, nbins, counts + size_t(cur) * nbins);
+                cur = f;
+            }
+            uint32_t const row = __builtin_amdgcn_readfirstlane(k ? e1.x : e0.x);
+            uint32_t const A0 = __builtin_amdgcn_readfirstlane(k ? e1.y : e0.y);
+            uint32_t const na = __builtin_amdgcn_readfirstlane(k ? e1.z : e0.z);
+            uint32_t const cx = __builtin_amdgcn_readfirstlane(k ? e1.w : e0.w);
+            float4 const pa = k ? p1 : p0;
+            DevGrid const g = fa::frame_grid(F, G);
+            int const cy = int(row % uint32_t(F.dim[1])), cz = int(row / uint32_t(F.dim[1]));
+            if (F.box.is2D)
+                rows_est<R, true, true, true>(F.box, g, pa, cy, cz, A0, na, int(cx & 0xffffu), int(cx >> 16), F.rx, 0u,
+                                              1u, B, [] {});
+            else
+                rows_est<R, false, true, true>(F.box, g, pa, cy, cz, A0, na, int(cx & 0xffffu), int(cx >> 16), F.rx,
+                                               0u, 1u, B, [] {});
+        }
+    }
+    if (cur != 0xffffffffu)
+        flush_wave_hist(wh, nbins, counts + size_t(cur) * nbins);
+}
+
+// Frames with points outside their box: one workgroup per 256-point tile, one
+// thread per point (see rdf_outside_kernel).
+template<int R>
+__global__ __launch_bounds__(kBlock) void brdf_outside_kernel(fa::BatchGrid G, const uint32_t* __restrict__ tile_frame,
+                                                              float lo, float hi, const float* __restrict__ T,
+                                                              uint32_t nbins, float vmin, float inv_width,
+                                                              uint32_t* __restrict__ counts)
+{
+    uint32_t const f = tile_frame[blockIdx.x];
+    const fa::BatchFrame& F = G.frames[f];
+    if (!F.any_outside)
+        return;
+    extern __shared__ uint32_t hist_only[];
+    for (uint32_t t = threadIdx.x; t < nbins; t += blockDim.x)
+        hist_only[t] = 0u;
+    __syncthreads();
+    uint32_t const local = (blockIdx.x - F.tile_base) * fa::kTile + threadIdx.x;
+    if (local < F.n)
+    {
+        DevGrid const g = fa::frame_grid(F, G);
+        float4 const q = G.cpos[F.pt_base + local];
+        uint32_t const qi = __float_as_uint(q.w);
+        fa::for_each_candidate<AABB_FORMULA>(
+            F.box, g, q.x, q.y, q.z, R, false,
+            [&](uint32_t j, float, float, float, float r_sq, int) {
+                if (j != qi && r_sq >= lo && r_sq < hi)
+                    atomicAdd(&hist_only[bin_in_range(r_sq, T, nbins, vmin, inv_width)], 1u);
+            },
+            F.rx);
+    }
+    hist_epilogue<true>(hist_only, nbins, counts + size_t(f) * nbins);
+}
+
 int grid_blocks(uint64_t work)
 {
     uint64_t const b = (work + kBlock - 1) / kBlock;
@@ -1235,7 +2040,8 @@ int rdf_row_variant_count()
 // Batched self RDF with cells at least r_max / R wide (R in 2..4): counts has
 // n_frames x bins entries.  Bins beyond 2048 are not supported here (each wave
 // keeps a private LDS histogram).
-int batch_rdf(const BatchGrid& G, int R, float r_max, uint32_t bins, const BatchRdfScratch& S, uint32_t* d_counts)
+int batch_rdf(const BatchGrid& G, const uint32_t* d_tile_frame, uint32_t ntiles, int R, float r_max, uint32_t bins,
+              const BatchRdfScratch& S, uint32_t* d_counts)
 {
     hipStream_t s = stream();
     if (bins == 0 || bins > 2048)
@@ -1264,6 +2070,32 @@ int batch_rdf(const BatchGrid& G, int R, float r_max, uint32_t bins, const Batch
         FA_HIP(hipGetDevice(&dev));
         FA_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
     }
+    if (S.est_hi > 0.0f)
+    {
+        // estimated r_sq: 6 workgroups per CU (its registers), see brdf_est_kernel
+        unsigned const eblocks = unsigned(std::max(1, n_cu) * 6);
+        size_t const lds = est_lds_bytes(bins, kBlock / 64);
+#define FA_BEST(RR)                                                                                                 \
+    case RR:                                                                                                        \
+        FA_KLAUNCH(brdf_est_kernel<RR>, dim3(eblocks), dim3(kBlock), lds, s, G, S.table, cl_frame,                  \
+                   S.cl_off + G.total_rows, S.queue, S.est_lo, S.est_hi, S.est_slack, T, bins, 0.0f, inv_width,     \
+                   d_counts);                                                                                       \
+        if (ntiles)                                                                                                 \
+            FA_KLAUNCH(brdf_outside_kernel<RR>, dim3(ntiles), dim3(kBlock), sizeof(uint32_t) * bins, s, G,          \
+                       d_tile_frame, S.est_lo, S.est_hi, T, bins, 0.0f, inv_width, d_counts);                       \
+        break;
+        switch (R)
+        {
+            FA_BEST(2)
+            FA_BEST(3)
+            FA_BEST(4)
+        default:
+            return fail(FA_ERR_INVALID, "unsupported RDF cell ratio");
+        }
+#undef FA_BEST
+        FA_HIP(hipGetLastError());
+        return FA_OK;
+    }
     unsigned const blocks = unsigned(std::max(1, n_cu) * 8);
     size_t const shmem = sizeof(float) * lds_table_floats(bins) + sizeof(uint32_t) * bins * (kBlock / 64);
     float const qmax_sq = r_max * r_max;
@@ -1285,9 +2117,14 @@ int batch_rdf(const BatchGrid& G, int R, float r_max, uint32_t bins, const Batch
     return FA_OK;
 }
 
-int thresholds_for(uint32_t bins, float r_max, float* d_T)
+int thresholds_for(uint32_t bins, float r_max, float* d_T, BatchRdfScratch& S)
 {
     std::vector<float> const tab = build_table(bins, 0.0f, r_max);
+    bool const table = bins <= kEstMaxBins && tab[est_table_start(bins)] > 0.0f;
+    EstRange const r = est_range(table, tab[0], tab[bins], r_max * r_max, 0.0f);
+    S.est_lo = r.lo;
+    S.est_hi = r.hi;
+    S.est_slack = r.slack;
     FA_HIP(hipMemcpy(d_T, tab.data(), sizeof(float) * tab.size(), hipMemcpyHostToDevice));
     return FA_OK;
 }
@@ -1310,7 +2147,9 @@ namespace {
 constexpr size_t kNoAllocBytes = size_t(64) << 20;
 constexpr uint32_t kNoAllocMaxPoints = 1u << 20;
 constexpr size_t kNoAllocTableBytes = size_t(32) << 10; // table_floats(kMaxLdsBins) floats
-static_assert(sizeof(float) * table_floats(kMaxLdsBins) <= kNoAllocTableBytes, "bin table region too small");
+static_assert(sizeof(float) * table_floats(kMaxLdsBins) <= kNoAllocTableBytes &&
+                  sizeof(float) * table_floats(kEstMaxBins) <= kNoAllocTableBytes,
+              "bin table region too small");
 constexpr int kNoAllocMaxDevices = 64;
 } // namespace
 
@@ -1328,6 +2167,8 @@ struct NoAllocDevice
     bool table_valid = false;
     uint32_t bins = 0;
     float r_min = 0.0f, r_max = 0.0f;
+    float first = 0.0f, last = 0.0f; // T[0], T[bins]
+    bool est = false;                // an estimate table follows
 };
 NoAllocDevice g_noalloc[kNoAllocMaxDevices];
 
@@ -1360,13 +2201,14 @@ int fa_rdf_bin_table(uint32_t bins, float r_min, float r_max, float* out, uint64
     if (bins == 0 || !(r_max > r_min))
         return fa::fail(FA_ERR_INVALID, "bin table needs bins > 0 and r_max > r_min");
     std::vector<float> const tab = build_table(bins, r_min, r_max);
+    size_t const n = exact_table_floats(bins);
     if (out)
     {
-        if (cap < tab.size())
+        if (cap < n)
             return fa::fail(FA_ERR_INVALID, "output too small for the bin table");
-        std::memcpy(out, tab.data(), sizeof(float) * tab.size());
+        std::memcpy(out, tab.data(), sizeof(float) * n);
     }
-    return int(tab.size());
+    return int(n);
 }
 
 int fa_rdf_accumulate_query(fa_nq* nq, const float* d_query_points, uint32_t n_query, float q_r_max, float q_r_min,
@@ -1388,6 +2230,7 @@ int fa_rdf_accumulate_query(fa_nq* nq, const float* d_query_points, uint32_t n_q
     float* T = nullptr;
     if (int rc = thresholds(bins, r_min, r_max, &T))
         return rc;
+    EstRange const est = est_range(g_thr.est, g_thr.first, g_thr.last, qmax_sq, qmin_sq);
     bool const lds = bins <= kMaxLdsBins;
     size_t const shmem = lds ? sizeof(float) * lds_table_floats(bins) + sizeof(uint32_t) * bins : 0;
     bool const self = (d_query_points == nq->d_points) && (n_query == nq->n);
@@ -1395,7 +2238,7 @@ int fa_rdf_accumulate_query(fa_nq* nq, const float* d_query_points, uint32_t n_q
     if (self && nq->kind == FA_NQ_AABB)
     {
         // row-cluster kernel; the cell size (r_max / R) is picked by the autotuner
-        RowsArgs ra{nq, qmax_sq, qmin_sq, T, bins, r_min, inv_width, q_r_max};
+        RowsArgs ra{nq, qmax_sq, qmin_sq, &est, T, bins, r_min, inv_width, q_r_max};
         double const density = double(nq->n) / double(fa::box_volume(nq->box));
         int const key = fa::tune_key(density, q_r_max);
         int variant = fa::tuned_variant(fa::TUNE_RDF_SELF, key);
@@ -1439,6 +2282,15 @@ int fa_rdf_accumulate_query(fa_nq* nq, const float* d_query_points, uint32_t n_q
             }
             return FA_OK;
         }
+    }
+    if (!self && nq->kind == FA_NQ_AABB && !exclude_ii && est.hi > 0.0f)
+    {
+        bool handled = false;
+        if (int rc = run_cross_rows(nq, d_query_points, n_query, q_r_max, qmax_sq, qmin_sq, est, T, bins, r_min,
+                                    inv_width, d_counts, &handled))
+            return rc;
+        if (handled)
+            return FA_OK;
     }
     int const R = 1;
     int dims[3];
@@ -1566,6 +2418,9 @@ int fa_rdf_accumulate_self_noalloc(const fa_box* box, const float* d_points, uin
         std::vector<float> const tab = build_table(bins, r_min, r_max);
         FA_HIP(hipMemcpyAsync(T, tab.data(), sizeof(float) * tab.size(), hipMemcpyHostToDevice, s));
         D.table_valid = true;
+        D.first = tab[0];
+        D.last = tab[bins];
+        D.est = bins <= kEstMaxBins && tab[est_table_start(bins)] > 0.0f;
         D.bins = bins;
         D.r_min = r_min;
         D.r_max = r_max;
@@ -1604,8 +2459,9 @@ int fa_rdf_accumulate_self_noalloc(const fa_box* box, const float* d_points, uin
     B.scan_bytes = scan_bytes;
     float const width = (r_max - r_min) / float(bins);
     float const inv_width = 1.0f / width;
-    return launch_rows(db, g, dims, rv.R, F, n, B, q_r_max * q_r_max, q_r_min * q_r_min, T, bins, r_min, inv_width,
-                       d_counts);
+    EstRange const est = est_range(D.est, D.first, D.last, q_r_max * q_r_max, q_r_min * q_r_min);
+    return launch_rows(db, g, nullptr, dims, rv.R, F, n, B, q_r_max * q_r_max, q_r_min * q_r_min, est, T, bins, r_min,
+                       inv_width, d_counts);
 }
 
 int fa_rdf_accumulate_nlist(const fa_nlist* nl, uint32_t bins, float r_min, float r_max, uint32_t* d_counts)

@@ -54,3 +54,68 @@ def test_solid_bonds_lane_groups(oracle, l, n, normalize):
     if not np.any(np.abs(ref["ql_ij"] - 0.3) < 1e-6):
         npt.assert_array_equal(sl.num_connections, ref["num_connections"])
         npt.assert_array_equal(sl.cluster_idx, ref["cluster_idx"])
+
+
+BOXES = {
+    "cube": Box.cube(16),
+    "triclinic": Box(12.0, 13.0, 14.0, 0.3, -0.2, 0.25),
+    "square": Box.square(24.0),
+    "flat": Box(30.0, 9.0, 12.0),
+    # across the edge of a box this large the estimate's bound exceeds its table: every pair exact
+    "large": Box.cube(900.0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(BOXES))
+@pytest.mark.parametrize("n", [2, 9, 513, 4096])
+@pytest.mark.parametrize("bins,r_max,r_min", [(100, 4.0, 0.0), (37, 2.3, 0.5), (512, 4.2, 0.0), (513, 4.0, 0.0),
+                                              (1, 3.0, 0.0)])
+def test_rdf_estimate_borders(oracle, name, n, bins, r_max, r_min):
+    """Bin counts bit for bit, self and with distinct query points, on both
+    sides of the estimate table's largest bin count, over few and many
+    clusters, dense and nearly empty boxes."""
+    box = BOXES[name]
+    rng = np.random.default_rng(n + bins)
+    pts = np.ascontiguousarray(box.make_absolute(rng.random((n, 3)).astype(np.float32)), np.float32)
+    q = np.ascontiguousarray(box.wrap(pts[::2] + np.float32(0.07)), np.float32)
+    if box.is2D:
+        pts[:, 2] = q[:, 2] = 0
+    rdf = freud_amd.density.RDF(bins, r_max, r_min=r_min)
+    ref = oracle.rdf_accumulate(_bt(box), pts, pts, bins, r_max, r_min=r_min, exclude_ii=True, nthreads=4)
+    npt.assert_array_equal(rdf.compute((box, pts)).bin_counts, ref)
+    ref = oracle.rdf_accumulate(_bt(box), pts, q, bins, r_max, r_min=r_min, exclude_ii=False, nthreads=4)
+    npt.assert_array_equal(rdf.compute((box, pts), query_points=q).bin_counts, ref)
+
+
+@pytest.mark.parametrize("which", ["points", "query_points", "both"])
+def test_rdf_points_outside_the_box(oracle, which):
+    """Systems with points (or query points) outside the box leave the
+    estimate kernel to the general walk."""
+    box = Box.cube(14.0)
+    rng = np.random.default_rng(3)
+    pts = ((rng.random((1500, 3)) - 0.5) * 14).astype(np.float32)
+    q = ((rng.random((700, 3)) - 0.5) * 14).astype(np.float32)
+    if which != "query_points":
+        pts[::7, 0] += np.float32(14.0)
+    if which != "points":
+        q[::5, 2] -= np.float32(14.0)
+    rdf = freud_amd.density.RDF(60, 3.0)
+    ref = oracle.rdf_accumulate(_bt(box), pts, q, 60, 3.0, exclude_ii=False, nthreads=4)
+    npt.assert_array_equal(rdf.compute((box, pts), query_points=q).bin_counts, ref)
+    ref = oracle.rdf_accumulate(_bt(box), pts, pts, 60, 3.0, exclude_ii=True, nthreads=4)
+    npt.assert_array_equal(rdf.compute((box, pts)).bin_counts, ref)
+
+
+def test_rdf_query_ranges_inside_the_histogram(oracle):
+    """A query radius inside the histogram's range cuts bins apart (exact
+    kernel); index exclusion with distinct query points (general kernel)."""
+    box, pts = _uniform(3000, seed=4)
+    q = np.ascontiguousarray(box.wrap(pts + np.float32(0.2)), np.float32)
+    rdf = freud_amd.density.RDF(80, 4.0)
+    for nb in (dict(r_max=2.71), dict(r_max=4.0, r_min=1.3), dict(r_max=4.0, exclude_ii=True)):
+        for query in (None, q):
+            ex = nb.get("exclude_ii", query is None)
+            nl = oracle.query(_bt(box), pts, pts if query is None else query, dict(nb, exclude_ii=ex), nthreads=4)
+            ref = oracle.rdf_bin(nl["distances"], 80, 0.0, 4.0)
+            got = rdf.compute((box, pts), query_points=query, neighbors=dict(nb)).bin_counts
+            npt.assert_array_equal(got, ref)
