@@ -670,8 +670,10 @@ int spatial_order(const fa_box& box, const float* d_points, uint32_t n, const ui
 // d_out[0] = 0, d_out[t + 1] = sum of d_in[0..t]; *total (if given) = the 64-bit
 // sum, read back with one synchronisation.  If d_extra is given, the n_extra
 // (1 or 2) u32 it points to are copied to h_extra in the same synchronisation.
+// d_segments (if given): d_out[t] where d_in[t] != 0, else 0.
 int exclusive_scan_u32(const uint32_t* d_in, uint32_t* d_out, uint32_t n, uint64_t* total,
-                       const uint32_t* d_extra = nullptr, uint32_t* h_extra = nullptr, int n_extra = 1);
+                       const uint32_t* d_extra = nullptr, uint32_t* h_extra = nullptr, int n_extra = 1,
+                       uint32_t* d_segments = nullptr);
 // The same scan for code that may be captured into a HIP graph: no memset, no
 // host synchronisation; `tmp` holds scan_tmp_bytes(n) bytes.
 size_t scan_tmp_bytes(uint32_t n);

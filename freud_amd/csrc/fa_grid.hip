@@ -2,6 +2,7 @@
 // freud's LinkCell / CellQuery cell lists, freud/locality/LinkCell.cc:316-367,
 // freud/locality/CellQuery.cc): counting sort of the points into cells, stored
 // as cell-ordered float4 (x, y, z, bits(j)) for coalesced stencil reads.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -72,6 +73,14 @@ __global__ void grid_assign_kernel(fa::DevBox b, const float* __restrict__ pts, 
     uint32_t const rank = wave_aggregated_increment(counts, cell, valid);
     if (valid && rank_of_point)
         rank_of_point[i] = rank;
+}
+
+__global__ void grid_clear_kernel(uint32_t* __restrict__ counts, uint32_t n, int* __restrict__ any_outside)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *any_outside = 0;
+    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x)
+        counts[t] = 0u;
 }
 
 __global__ void grid_scatter_kernel(const float* __restrict__ pts, uint32_t n,
@@ -365,8 +374,9 @@ int build_grid(Grid& g, const fa_box& box, const float* d_points, uint32_t n, co
         if (int rc = device_alloc((void**) &g.outside, 256))
             return rc;
     int* d_any = g.outside;
-    FA_HIP(hipMemsetAsync(counts, 0, cb, s));
-    FA_HIP(hipMemsetAsync(d_any, 0, sizeof(int), s));
+    // one small kernel clears the counters and the flag
+    FA_KLAUNCH(grid_clear_kernel, dim3(unsigned(std::min<uint64_t>((ncell64 + 1023) / 1024, 2048))), dim3(256), 0, s,
+               counts, ncell, d_any);
     unsigned const blocks = (n + 255) / 256;
     if (n)
     {

@@ -1634,7 +1634,8 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
         self ? walk(ball_walk_kernel<LINKCELL_FORMULA, true>) : walk(ball_walk_kernel<LINKCELL_FORMULA, false>);
     FA_HIP(hipGetLastError());
     uint64_t total = 0;
-    if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total))
+    if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total, nullptr, nullptr, 1,
+                                        out->segments))
         return rc;
     if (total > 0xffffffffull)
         return fa::fail(FA_ERR_RUNTIME, "NeighborList would exceed 2^32 bonds");
@@ -1687,7 +1688,7 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
         FA_HIP(hipGetLastError());
     }
 #undef FA_BALL_EMIT
-    return fa::nlist_finish_counts(out);
+    return FA_OK;
 }
 
 // Radius of the last ball of the reference's expanding kNN search
@@ -1758,7 +1759,6 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
     uint32_t* flagged = nflag + 16;
     uint32_t* pos = flagged + n_query + 48;
     uint32_t* refine = pos + n_query + 16;
-    FA_HIP(hipMemsetAsync(nflag, 0, 2 * sizeof(uint32_t), s));
     float npd[3];
     fa::nearest_plane_distance(nq->box, npd);
     float min_pd = std::min(npd[0], npd[1]);
@@ -1792,7 +1792,8 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
             for (int d = 0; d < (nq->box.is2D ? 2 : 3); ++d)
                 wmin = std::min(wmin, npd[d] / float(dims[d]));
             int const rmax_ring = std::max(dims[0], std::max(dims[1], dims[2])) * 2 + 2;
-            FA_HIP(hipMemsetAsync(nflag, 0, 2 * sizeof(uint32_t), s));
+            if (int rc = fa::zero_u32(nflag, 2))
+                return rc;
 #define FA_KNN_LAUNCH(KM)                                                                                     \
     launch_knn_aabb<KM>(*dbp, nq->cur->dev(), qpts, n_query, k, rlim, a.r_min, a.exclude_ii, wmin, min_pd / 2.0f, \
                         rmax_ring, stage, out->counts, sel, flagged, nflag, refine, nrefine, nq->d_points, nq->n, pos)
@@ -1950,7 +1951,7 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
     uint64_t total = 0;
     uint32_t h_counts[2] = {0, 0}; // flagged, handed back
     if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total,
-                                        nq->kind == FA_NQ_AABB ? nflag : nullptr, h_counts, 2))
+                                        nq->kind == FA_NQ_AABB ? nflag : nullptr, h_counts, 2, out->segments))
         return rc;
     h_nflag = h_counts[0];
     // The staged search pays a serial ring walk for each handed-back point; on
@@ -1981,7 +1982,8 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
                        static_cast<uint64_t*>(work), out->counts, sel, pos);
             FA_HIP(hipGetLastError());
         }
-        if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total))
+        if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total, nullptr, nullptr, 1,
+                                            out->segments))
             return rc;
     }
     if (int rc = fa::nlist_reserve(out, total, n_query))
@@ -2031,7 +2033,7 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
                     : launch(knn_write_kernel<LINKCELL_FORMULA, false, false, true>);
     }
     FA_HIP(hipGetLastError());
-    return fa::nlist_finish_counts(out);
+    return FA_OK;
 }
 
 } // namespace

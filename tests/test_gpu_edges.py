@@ -119,3 +119,33 @@ def test_rdf_query_ranges_inside_the_histogram(oracle):
             ref = oracle.rdf_bin(nl["distances"], 80, 0.0, 4.0)
             got = rdf.compute((box, pts), query_points=query, neighbors=dict(nb)).bin_counts
             npt.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("bonds", [1, 4096, 8191, 8192, 8193, 70001, (1 << 22) + 5])
+def test_scan_sizes_through_filter(bonds):
+    """The count scan at its tile, single-workgroup and library borders:
+    filtering a list compacts it by a scan over its bonds, its segments by one
+    over its points."""
+    rng = np.random.default_rng(bonds)
+    n = max(1, bonds // 7)
+    i = np.sort(rng.integers(0, n, bonds)).astype(np.uint32)
+    j = rng.integers(0, n, bonds).astype(np.uint32)
+    v = rng.random((bonds, 3)).astype(np.float32)
+    nl = freud_amd.locality.NeighborList.from_arrays(n, n, i, j, v)
+    keep = rng.random(bonds) < 0.6
+    nl.filter(keep)
+    npt.assert_array_equal(nl[:], np.stack([i[keep], j[keep]], 1))
+    npt.assert_array_equal(nl.vectors, v[keep])
+    npt.assert_array_equal(nl.neighbor_counts, np.bincount(i[keep], minlength=n))
+
+
+@pytest.mark.parametrize("n", [2, 4096, 8192, 8193, 40001])
+def test_query_segments(n):
+    """Offsets, counts and segments (0 for points without bonds) of a query."""
+    box, pts = _uniform(n, density=0.3, seed=n)
+    for args in (dict(r_max=1.0, exclude_ii=True), dict(num_neighbors=1, r_max=0.9, exclude_ii=True)):
+        nl = freud_amd.AABBQuery(box, pts).query(pts, args).toNeighborList()
+        counts = np.bincount(nl[:][:, 0], minlength=n)
+        npt.assert_array_equal(nl.neighbor_counts, counts)
+        start = np.cumsum(counts) - counts
+        npt.assert_array_equal(nl.segments, np.where(counts > 0, start, 0))
