@@ -30,6 +30,10 @@ using fa::LINKCELL_FORMULA;
 constexpr int kBlock = 256;
 constexpr int kKeyBytes = 32768; // largest LDS key staging per block
 // keys per point that the one-walk ball query stages in LDS (32 KB per block)
+// query points up to which a ball query, and a kNN query (whose per-thread
+// search the tuner fits to larger systems), takes one wave per point
+constexpr uint32_t kWaveQueries = 32768;
+constexpr uint32_t kWaveKnnQueries = 8192;
 constexpr uint32_t kWalkMaxSlots = kKeyBytes / (kBlock * sizeof(uint32_t));
 extern __shared__ __align__(16) unsigned char fa_dyn_lds[];
 
@@ -843,6 +847,294 @@ __global__ __launch_bounds__(kBlock) void knn_stage_kernel(DevBox b, DevGrid g, 
         sel[uint64_t(p0) * k + t] = s_out[t];
 }
 
+// ------------------------------------------------------------------ one wave per query point
+// Small systems (up to kWaveQueries query points) leave most of the chip idle
+// with a thread per query point, and a thread's walk is one dependent load
+// after another: 4,096 points are 64 waves on 1,024 SIMDs.  Here a wave takes
+// one query point: lane t resolves stencil cell t, the cells' points are
+// concatenated and evaluated 64 at a time, and what is kept is ranked by
+// comparing every key with every other.  The candidates, their arithmetic and
+// the selected order are those of the per-thread kernels.
+// 4,096 points, k = 12: search 154 -> 19 us; 20,000 points, r_max = 1.5:
+// walk 47 -> 37 us, emission 93 -> 9 us.  At 100,000 points the per-thread
+// kernels are the faster ones.
+constexpr uint32_t kWaveKeys = 256; // keys a wave keeps (2 KB of LDS)
+constexpr uint32_t kWaves = kBlock / 64;
+
+// Calls f(valid, j, code, r_sq) with all lanes for 64 candidates at a time of
+// the stencil of half-width R around q (AABB formula), as for_each_candidate
+// visits them; lanes without a candidate get valid = false.
+template<typename F>
+__device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float qx, float qy, float qz, int R, F&& f)
+{
+    int c[3], w[3];
+    fa::cell_of(b, g.dim, qx, qy, qz, c, w);
+    float const qzz = b.is2D ? 0.0f : qz;
+    int const side = 2 * R + 1, Rz = b.is2D ? 0 : R;
+    int const ncell = side * side * (2 * Rz + 1);
+    bool const outside = *g.outside;
+    uint32_t const lane = threadIdx.x & 63u;
+    for (int c0 = 0; c0 < ncell; c0 += 64)
+    {
+        uint32_t beg = 0u, len = 0u;
+        int shift = 0; // image offset of the cell per axis, 10 bits each (biased by 512)
+        int const t = c0 + int(lane);
+        if (t < ncell)
+        {
+            int const d[3] = {t % side - R, (t / side) % side - R, t / (side * side) - Rz};
+            int cell[3], nb[3];
+            bool in = true;
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+            {
+                int const u = c[k] + d[k], s = fa::floor_div(u, g.dim[k]);
+                cell[k] = u - s * g.dim[k];
+                nb[k] = -w[k] - s;
+                in = in && (outside ? nb[k] >= -500 && nb[k] <= 500 : nb[k] >= -1 && nb[k] <= 1);
+            }
+            if (in)
+            {
+                uint32_t const id = uint32_t((cell[2] * g.dim[1] + cell[1]) * g.dim[0] + cell[0]);
+                beg = g.cstart[id];
+                len = g.cstart[id + 1] - beg;
+                shift = (nb[0] + 512) | ((nb[1] + 512) << 10) | ((nb[2] + 512) << 20);
+            }
+        }
+        uint32_t e = len; // inclusive scan over the lanes
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1)
+        {
+            uint32_t const y = __shfl_up(e, d);
+            if (lane >= uint32_t(d))
+                e += y;
+        }
+        uint32_t const p = e - len, sh = beg - p;
+        uint32_t const tot = uint32_t(__builtin_amdgcn_readlane(int(e), 63));
+        uint64_t live = __builtin_amdgcn_ballot_w64(len > 0u);
+        for (uint32_t v0 = 0; v0 < tot; v0 += 64u)
+        {
+            uint32_t const v = v0 + lane;
+            uint32_t pos = 0u;
+            int code3 = 0;
+            for (uint64_t m = live; m; m &= m - 1u)
+            {
+                int const r = __builtin_ctzll(m);
+                uint32_t const sp = uint32_t(__builtin_amdgcn_readlane(int(p), r));
+                if (sp >= v0 + 64u)
+                    break;
+                uint32_t const p2 = v + uint32_t(__builtin_amdgcn_readlane(int(sh), r));
+                int const s2 = __builtin_amdgcn_readlane(shift, r);
+                pos = v >= sp ? p2 : pos;
+                code3 = v >= sp ? s2 : code3;
+                if (uint32_t(__builtin_amdgcn_readlane(int(e), r)) <= v0 + 64u)
+                    live &= ~(uint64_t(1) << r);
+            }
+            bool valid = v < tot;
+            float4 const pj = g.cpos[valid ? pos : 0u];
+            int n0 = (code3 & 1023) - 512, n1 = ((code3 >> 10) & 1023) - 512, n2 = ((code3 >> 20) & 1023) - 512;
+            if (outside)
+            {
+                int wj[3];
+                fa::unpack_wrap(g.wrapc[valid ? pos : 0u], wj);
+                n0 += wj[0];
+                n1 += wj[1];
+                n2 = b.is2D ? 0 : n2 + wj[2];
+            }
+            valid = valid && n0 >= -1 && n0 <= 1 && n1 >= -1 && n1 <= 1 && n2 >= -1 && n2 <= 1;
+            int const code = valid ? (n0 + 1) * 9 + (n1 + 1) * 3 + (n2 + 1) : 13;
+            float const pz = b.is2D ? 0.0f : pj.z;
+            float const rx = pj.x - (qx + b.img[code][0]);
+            float const ry = pj.y - (qy + b.img[code][1]);
+            float const rz = pz - (qzz + b.img[code][2]);
+            f(valid, __float_as_uint(pj.w), code, (rx * rx + ry * ry) + rz * rz);
+        }
+    }
+}
+
+// Appends the key of every lane with `take` to the wave's list (beyond
+// kWaveKeys they are counted only).
+__device__ inline void wave_append(uint64_t* keys, uint32_t& n, bool take, uint64_t key)
+{
+    uint64_t const m = __builtin_amdgcn_ballot_w64(take);
+    uint32_t const at = n + __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+    if (take && at < kWaveKeys)
+        keys[at] = key;
+    n += uint32_t(__builtin_popcountll(m));
+}
+
+// Calls f(rank, key) for the wave's n <= kWaveKeys distinct keys, in any order.
+template<typename F> __device__ inline void wave_rank(const uint64_t* keys, uint32_t n, F&& f)
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the lanes' appends are visible to the wave
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t t0 = 0; t0 < n; t0 += 64u)
+    {
+        uint32_t const t = t0 + (threadIdx.x & 63u);
+        uint64_t const own = t < n ? keys[t] : 0u;
+        uint32_t rank = 0;
+        for (uint32_t m = 0; m < n; ++m)
+            rank += keys[m] < own ? 1u : 0u;
+        if (t < n)
+            f(rank, own);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the list may be written again
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Ball query, one wave per query position: the point's keys (j << 5 | image
+// code) in NeighborList order into rows[i * C ..], its bond count, and a mark
+// when some point has more than C bonds (the caller then runs the per-thread
+// query).
+template<bool BYDIST, bool SELF>
+__global__ __launch_bounds__(kBlock) void ball_wave_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
+                                                           uint32_t nq, float r_max_sq, float r_min_sq, int exclude_ii,
+                                                           int R, uint32_t C, uint32_t* __restrict__ counts,
+                                                           uint32_t* __restrict__ rows, uint32_t* __restrict__ over)
+{
+    __shared__ uint64_t s_keys[kWaves][kWaveKeys];
+    uint32_t const wave = threadIdx.x >> 6;
+    uint32_t const p = fa::xcd_tile(blockIdx.x, gridDim.x) * kWaves + wave;
+    if (p >= nq)
+        return;
+    float qx, qy, qz;
+    uint32_t const i = query_at<SELF>(g, qpts, p, qx, qy, qz);
+    uint64_t* const keys = s_keys[wave];
+    uint32_t n = 0;
+    wave_candidates(b, g, qx, qy, qz, R, [&](bool valid, uint32_t j, int code, float r_sq) {
+        bool const take = valid && r_sq < r_max_sq && r_sq >= r_min_sq && !(exclude_ii && j == i);
+        uint64_t const jc = (uint64_t(j) << 5) | uint32_t(code);
+        wave_append(keys, n, take, BYDIST ? (uint64_t(float_order_bits(sqrtf(r_sq))) << 32) | jc : jc);
+    });
+    if ((threadIdx.x & 63u) == 0)
+    {
+        counts[i] = n;
+        if (n > C)
+            *over = 1u; // every writer stores the same value
+    }
+    if (n <= C)
+        wave_rank(keys, n, [&](uint32_t rank, uint64_t key) { rows[uint64_t(i) * C + rank] = uint32_t(key); });
+}
+
+// Emission for ball_wave_kernel: 16 lanes per query point write its bonds from
+// its sorted keys (stride C).
+template<int FORMULA>
+__global__ __launch_bounds__(kBlock) void wave_emit_kernel(DevBox b, const float* __restrict__ qpts, uint32_t nq,
+                                                           const float* __restrict__ pts,
+                                                           const uint32_t* __restrict__ rows, uint32_t C,
+                                                           const uint32_t* __restrict__ offsets,
+                                                           uint32_t* __restrict__ nb_out, float* __restrict__ d_out,
+                                                           float* __restrict__ w_out, float* __restrict__ v_out)
+{
+    uint32_t const i = (blockIdx.x * kBlock + threadIdx.x) / 16u;
+    if (i >= nq)
+        return;
+    uint32_t const e0 = offsets[i], n = offsets[i + 1] - e0;
+    float const qx = qpts[3 * i], qy = qpts[3 * i + 1], qz = qpts[3 * i + 2];
+    for (uint32_t m = threadIdx.x & 15u; m < n; m += 16u)
+        write_bond_at<FORMULA, false>(b, qx, qy, qz, pts, i, uint64_t(rows[uint64_t(i) * C + m]), uint64_t(e0) + m,
+                                      nb_out, d_out, w_out, v_out);
+}
+
+// kNN, one wave per query position (see the ring search for what is selected):
+// the stencil of half-width 1, then 2, .., is searched until k distances lie
+// inside the radius it covers, or it covers rlim.  Positions whose stencils hold more
+// than the wave's keys, or need more than three, are handed back to the ring
+// search, and answers reaching half the smallest plane distance are flagged for
+// the exhaustive one, as there.
+template<bool SELF>
+__global__ __launch_bounds__(kBlock) void knn_wave_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
+                                                          uint32_t nq, uint32_t k, float rlim_sq, float rlim,
+                                                          float rmin_thr, int exclude_ii, float wmin,
+                                                          float half_min_plane, uint32_t* __restrict__ counts,
+                                                          uint64_t* __restrict__ sel, uint32_t* __restrict__ flagged,
+                                                          uint32_t* __restrict__ nflag, uint32_t* __restrict__ refine,
+                                                          uint32_t* __restrict__ nrefine, uint32_t* __restrict__ pos)
+{
+    __shared__ uint64_t s_keys[kWaves][kWaveKeys];
+    uint32_t const wave = threadIdx.x >> 6;
+    bool const lead = (threadIdx.x & 63u) == 0;
+    uint32_t const p = fa::xcd_tile(blockIdx.x, gridDim.x) * kWaves + wave;
+    if (p >= nq)
+        return;
+    float qx, qy, qz;
+    uint32_t const i = query_at<SELF>(g, qpts, p, qx, qy, qz);
+    if (SELF && lead)
+        pos[i] = p;
+    uint64_t* const keys = s_keys[wave];
+    uint32_t n = 0;
+    bool done = false;
+    for (int R = 1; R <= 3 && !done; ++R)
+    {
+        float const complete = float(R) * wmin * (1.0f - 1e-4f);
+        n = 0; // keys with d < complete
+        wave_candidates(b, g, qx, qy, qz, R, [&](bool valid, uint32_t j, int code, float r_sq) {
+            bool take = valid && r_sq < rlim_sq && r_sq >= rmin_thr && !(exclude_ii && j == i);
+            uint64_t const key = knn_key(r_sq, (j << 5) | uint32_t(code));
+            take = take && knn_key_distance(key) < complete;
+            wave_append(keys, n, take, key);
+        });
+        if (n > kWaveKeys)
+            break;
+        done = n >= k || complete >= rlim; // inside `complete` nothing is missing
+        if (!done && complete >= half_min_plane && rlim > half_min_plane)
+            break; // longer searches, and the exhaustive flag, are the ring search's
+    }
+    if (!done)
+    {
+        if (lead)
+            refine[atomicAdd(nrefine, 1u)] = p;
+        return;
+    }
+    uint32_t const kept = min(n, k);
+    float last = 0.0f;
+    wave_rank(keys, n, [&](uint32_t rank, uint64_t key) {
+        if (rank < kept)
+            sel[uint64_t(p) * k + rank] = key;
+        if (rank + 1u == kept)
+            last = knn_key_distance(key);
+    });
+    // two images of one point are at least a plane distance apart (see the ring search)
+    bool const flag = __builtin_amdgcn_ballot_w64(rlim > half_min_plane && last >= half_min_plane) != 0;
+    if (lead)
+    {
+        if (flag)
+            flagged[atomicAdd(nflag, 1u)] = p;
+        counts[i] = flag ? 0u : kept;
+    }
+}
+
+// Emission of a small system's kNN result: 16 lanes per query point rank its
+// selected keys in the NeighborList order and write the bonds.
+template<bool BYDIST, bool SELF>
+__global__ __launch_bounds__(kBlock) void knn_rank_emit_kernel(DevBox b, const float* __restrict__ qpts, uint32_t nq,
+                                                               const float* __restrict__ pts, uint32_t k,
+                                                               const uint64_t* __restrict__ sel,
+                                                               const uint32_t* __restrict__ pos,
+                                                               const uint32_t* __restrict__ offsets,
+                                                               uint32_t* __restrict__ nb_out,
+                                                               float* __restrict__ d_out, float* __restrict__ w_out,
+                                                               float* __restrict__ v_out)
+{
+    uint32_t const i = (blockIdx.x * kBlock + threadIdx.x) / 16u;
+    if (i >= nq)
+        return;
+    uint32_t const e0 = offsets[i], n = offsets[i + 1] - e0;
+    const uint64_t* const row = sel + uint64_t(SELF ? pos[i] : i) * k;
+    auto key_of = [&](uint64_t sk) -> uint64_t {
+        uint64_t const jc = uint32_t(sk);
+        return BYDIST ? (uint64_t(float_order_bits(knn_key_distance(sk))) << 32) | jc : jc;
+    };
+    float const qx = qpts[3 * i], qy = qpts[3 * i + 1], qz = qpts[3 * i + 2];
+    for (uint32_t m = threadIdx.x & 15u; m < n; m += 16u)
+    {
+        uint64_t const own = key_of(row[m]);
+        uint32_t rank = 0;
+        for (uint32_t t = 0; t < n; ++t)
+            rank += key_of(row[t]) < own ? 1u : 0u;
+        write_bond_at<AABB_FORMULA, BYDIST>(b, qx, qy, qz, pts, i, own, uint64_t(e0) + rank, nb_out, d_out, w_out, v_out);
+    }
+}
+
 // LinkCell formula kNN (LinkCell.cc:575-679): every point in cells within
 // max_range - 1 Chebyshev shells of the reference's grid, each cell once.
 template<int KMAX>
@@ -1558,6 +1850,44 @@ int launch_knn_aabb(const fa::DevBox& db, const DevGrid& g, const float* qpts, u
     return FA_OK;
 }
 
+// The wave-per-query search, then the ring search over what it hands back.
+int launch_knn_wave(const fa::DevBox& db, const DevGrid& g, const float* qpts, uint32_t nq, uint32_t k, float rlim,
+                    float r_min, int exclude_ii, float wmin, float hmp, int rmax_ring, uint32_t* counts, uint64_t* sel,
+                    uint32_t* flagged, uint32_t* nflag, uint32_t* refine, uint32_t* nrefine, const float* self_points,
+                    uint32_t self_n, uint32_t* pos)
+{
+    bool const self = (qpts == self_points) && (nq == self_n);
+    float const rlim_sq = rlim * rlim, rmin_thr = sqrt_threshold(r_min);
+    FA_PROF_BEGIN("knn_wave_kernel");
+    auto search = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((nq + kWaves - 1) / kWaves), dim3(kBlock), 0, fa::stream(), db, g, qpts, nq, k,
+                           rlim_sq, rlim, rmin_thr, exclude_ii, wmin, hmp, counts, sel, flagged, nflag, refine, nrefine,
+                           pos);
+    };
+    self ? search(knn_wave_kernel<true>) : search(knn_wave_kernel<false>);
+    FA_PROF_END();
+    FA_HIP(hipGetLastError());
+    FA_PROF_BEGIN("knn_refine_kernel");
+    auto rest = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((nq + kBlock - 1) / kBlock), dim3(kBlock), 0, fa::stream(), db, g, qpts, nq, k,
+                           rlim_sq, rlim, rmin_thr, exclude_ii, wmin, hmp, rmax_ring, counts, sel, flagged, nflag, pos,
+                           refine, nrefine);
+    };
+#define FA_KNN_REST(KM) (self ? rest(knn_aabb_kernel<KM, true, true>) : rest(knn_aabb_kernel<KM, false, true>))
+    if (k <= 8)
+        FA_KNN_REST(8);
+    else if (k <= 16)
+        FA_KNN_REST(16);
+    else if (k <= 32)
+        FA_KNN_REST(32);
+    else
+        FA_KNN_REST(64);
+#undef FA_KNN_REST
+    FA_PROF_END();
+    FA_HIP(hipGetLastError());
+    return FA_OK;
+}
+
 template<int KMAX>
 int launch_knn_lc(const fa::DevBox& db, const DevGrid& g, const float* qpts, uint32_t nq, uint32_t k, float r_max,
                   float r_min, int exclude_ii, int R, uint32_t* counts, uint64_t* sel)
@@ -1585,6 +1915,62 @@ uint32_t ball_row_slots(const fa_nq* nq, float r_max)
     return uint32_t(std::max(c, 8.0));
 }
 
+// Key slots per point of the wave-per-query ball query: twice the expected
+// bonds and some; 0 (not used) where more than a third of a wave's keys are
+// expected, and its ranking, quadratic in the bonds, would dominate.
+uint32_t ball_wave_slots(const fa_nq* nq, float r_max)
+{
+    double const vol = std::max(double(fa::box_volume(nq->box)), 1e-30);
+    double const dens = double(nq->n) / vol;
+    double const r = double(r_max);
+    double const expect = nq->box.is2D ? dens * M_PI * r * r : dens * (4.0 / 3.0) * M_PI * r * r * r;
+    return expect > kWaveKeys / 3 ? 0u : uint32_t(std::min<double>(kWaveKeys, 2.0 * expect + 32.0));
+}
+
+// The ball query of a small system on nq->cur.  handled = false: some point
+// has more bonds than slots (nothing but counts has been written).
+int run_ball_wave(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args& a, int by_distance, bool self,
+                  uint32_t C, fa_nlist* out, bool* handled)
+{
+    *handled = false;
+    hipStream_t s = fa::stream();
+    DevGrid const g = nq->cur->dev();
+    fa::DevBox const& db = nq->cur->dbox;
+    float const r_max_sq = a.r_max * a.r_max, r_min_sq = a.r_min * a.r_min;
+    void* tmp = nullptr;
+    if (int rc = fa::scratch(21, sizeof(uint32_t) * (size_t(n_query) * C + 64), &tmp))
+        return rc;
+    uint32_t* const over = static_cast<uint32_t*>(tmp);
+    uint32_t* const rows = over + 64;
+    if (int rc = fa::zero_u32(over, 1))
+        return rc;
+    auto walk = [&](auto kern) {
+        FA_PROF_BEGIN("ball_wave_kernel");
+        hipLaunchKernelGGL(kern, dim3((n_query + kWaves - 1) / kWaves), dim3(kBlock), 0, s, db, g, qpts, n_query,
+                           r_max_sq, r_min_sq, a.exclude_ii, 1, C, out->counts, rows, over);
+        FA_PROF_END();
+    };
+    if (self)
+        by_distance ? walk(ball_wave_kernel<true, true>) : walk(ball_wave_kernel<false, true>);
+    else
+        by_distance ? walk(ball_wave_kernel<true, false>) : walk(ball_wave_kernel<false, false>);
+    FA_HIP(hipGetLastError());
+    uint64_t total = 0;
+    uint32_t h_over = 0;
+    if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total, over, &h_over, 1, out->segments))
+        return rc;
+    if (h_over)
+        return FA_OK;
+    if (int rc = fa::nlist_reserve(out, total, n_query))
+        return rc;
+    out->num_bonds = total;
+    FA_KLAUNCH(wave_emit_kernel<AABB_FORMULA>, dim3((n_query * 16u + kBlock - 1) / kBlock), dim3(kBlock), 0, s, db, qpts,
+               n_query, nq->d_points, rows, C, out->offsets, out->neighbors, out->distances, out->weights, out->vectors);
+    FA_HIP(hipGetLastError());
+    *handled = true;
+    return FA_OK;
+}
+
 int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args& a, int by_distance, fa_nlist* out)
 {
     hipStream_t s = fa::stream();
@@ -1601,6 +1987,17 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
     unsigned const blocks = (n_query + kBlock - 1) / kBlock;
     // query points == the grid's points: the walk takes them in cell order
     bool const self = (qpts == nq->d_points) && (n_query == nq->n);
+    if (nq->kind == FA_NQ_AABB && n_query && n_query <= kWaveQueries)
+    {
+        // small systems: one wave per query point, unless bonds are many
+        uint32_t const Cw = ball_wave_slots(nq, a.r_max);
+        bool handled = false;
+        if (Cw)
+            if (int rc = run_ball_wave(nq, qpts, n_query, a, by_distance, self, Cw, out, &handled))
+                return rc;
+        if (handled)
+            return FA_OK;
+    }
     fa::CQGrid const cq = nq->kind == FA_NQ_CELLQUERY ? fa::cq_grid_for(nq->box, a.r_max) : fa::CQGrid{};
     uint32_t const C = ball_row_slots(nq, a.r_max);
     uint32_t* rows = nullptr;
@@ -1836,7 +2233,29 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
         }
         int rc = FA_OK;
         int const key = fa::tune_key(dens, rk) * 128 + int(std::min<uint32_t>(k, 127u));
-        if (k <= 64 && reuse >= 0)
+        if (k <= kWaveKeys / 4 && n_query <= kWaveKnnQueries)
+        {
+            // small systems: one wave per query point, cells as wide as the
+            // radius that holds k + 5 sqrt(k) + 8 points, so that one stencil
+            // nearly always holds the answer
+            double const lam = k + 5.0 * std::sqrt(double(k)) + 8.0;
+            double const wcell = nq->box.is2D ? std::sqrt(lam / (M_PI * dens)) : std::cbrt(3.0 * lam / (4.0 * M_PI * dens));
+            int dims[3];
+            fa::grid_dims_for(nq->box, nq->n, float(std::max(wcell, 1e-6)), 1, dims);
+            if (int rc2 = fa::ensure_grid(nq, dims))
+                return rc2;
+            dbp = &nq->cur->dbox;
+            if (int rc2 = fa::zero_u32(nflag, 2))
+                return rc2;
+            float wmin = std::numeric_limits<float>::infinity();
+            for (int d = 0; d < (nq->box.is2D ? 2 : 3); ++d)
+                wmin = std::min(wmin, npd[d] / float(dims[d]));
+            int const rmax_ring = std::max(dims[0], std::max(dims[1], dims[2])) * 2 + 2;
+            rc = launch_knn_wave(*dbp, nq->cur->dev(), qpts, n_query, k, rlim, a.r_min, a.exclude_ii, wmin,
+                                 min_pd / 2.0f, rmax_ring, out->counts, sel, flagged, nflag, refine, nrefine,
+                                 nq->d_points, nq->n, pos);
+        }
+        else if (k <= 64 && reuse >= 0)
         {
             int const dims[3] = {nq->grid_dims[reuse][0], nq->grid_dims[reuse][1], nq->grid_dims[reuse][2]};
             int mode = stage_params.C ? fa::tuned_variant(fa::TUNE_KNN_REUSE, key) : 0;
@@ -2004,7 +2423,21 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
                            key_cap);
         FA_PROF_END();
     };
-    if (nq->kind == FA_NQ_AABB)
+    if (nq->kind == FA_NQ_AABB && n_query <= kWaveQueries && k <= 64)
+    {
+        auto emit = [&](auto kern) {
+            FA_PROF_BEGIN("knn_rank_emit_kernel");
+            hipLaunchKernelGGL(kern, dim3((n_query * 16u + kBlock - 1) / kBlock), dim3(kBlock), 0, s, *dbp, qpts, n_query,
+                               nq->d_points, k, sel, pos, out->offsets, out->neighbors, out->distances, out->weights,
+                               out->vectors);
+            FA_PROF_END();
+        };
+        if (self)
+            by_distance ? emit(knn_rank_emit_kernel<true, true>) : emit(knn_rank_emit_kernel<false, true>);
+        else
+            by_distance ? emit(knn_rank_emit_kernel<true, false>) : emit(knn_rank_emit_kernel<false, false>);
+    }
+    else if (nq->kind == FA_NQ_AABB)
     {
         // self queries of points stored in random order write in processing order
         bool index_order = true;

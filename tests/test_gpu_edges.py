@@ -149,3 +149,49 @@ def test_query_segments(n):
         npt.assert_array_equal(nl.neighbor_counts, counts)
         start = np.cumsum(counts) - counts
         npt.assert_array_equal(nl.segments, np.where(counts > 0, start, 0))
+
+
+def _assert_same(nl, ref):
+    npt.assert_array_equal(nl[:], ref["ij"])
+    npt.assert_array_equal(nl.distances, ref["distances"])
+    npt.assert_array_equal(nl.vectors, ref["vectors"])
+
+
+@pytest.mark.parametrize("name", ["cube", "triclinic", "square", "flat"])
+@pytest.mark.parametrize("n", [2, 65, 1500, 8193])
+@pytest.mark.parametrize("outside", [False, True])
+def test_wave_queries(oracle, name, n, outside):
+    """One wave per query point, up to its largest kNN size and past it: ball
+    and nearest queries against the oracle, self and with distinct query
+    points, in every order, with points inside and outside the box, in boxes
+    of a few cells and of many."""
+    box = BOXES[name]
+    rng = np.random.default_rng(n)
+    pts = np.ascontiguousarray(box.make_absolute(rng.random((n, 3)).astype(np.float32)), np.float32)
+    q = np.ascontiguousarray(box.wrap(pts[::3] + np.float32(0.31)), np.float32)
+    if outside:
+        pts[::5, 0] += np.float32(box.Lx)
+        q[::4, 1] -= np.float32(box.Ly)
+    if box.is2D:
+        pts[:, 2] = q[:, 2] = 0
+    nq = freud_amd.AABBQuery(box, pts)
+    r = min(1.4, (60 * box.volume / n / 4.2) ** (1 / 3)) if not box.is2D else 1.2
+    for args in (dict(r_max=r, exclude_ii=True), dict(r_max=r, r_min=0.4 * r), dict(num_neighbors=5, exclude_ii=True),
+                 dict(num_neighbors=17, r_max=2.0), dict(num_neighbors=1, r_min=0.3)):
+        for points in (pts, q):
+            for by_distance in (False, True):
+                ref = oracle.query(_bt(box), pts, points, args, sort_by_distance=by_distance, nthreads=4)
+                nl = nq.query(points, args).toNeighborList(sort_by_distance=by_distance)
+                _assert_same(nl, ref)
+
+
+def test_wave_ball_query_falls_back_on_clumps(oracle):
+    """A clump with more bonds per point than a wave keeps: the per-thread
+    query takes the call."""
+    box = Box.cube(20.0)
+    rng = np.random.default_rng(8)
+    pts = ((rng.random((1500, 3)) - 0.5) * 20).astype(np.float32)
+    pts[:600] = (rng.standard_normal((600, 3)) * 0.3).astype(np.float32)
+    for args in (dict(r_max=1.5, exclude_ii=True), dict(num_neighbors=12, exclude_ii=True)):
+        ref = oracle.query(_bt(box), pts, pts, args, nthreads=4)
+        _assert_same(freud_amd.AABBQuery(box, pts).query(pts, args).toNeighborList(), ref)
