@@ -35,16 +35,25 @@ constexpr int kKeyBytes = 32768; // largest LDS key staging per block
 constexpr uint32_t kWaveQueries = 32768;
 constexpr uint32_t kWaveKnnQueries = 8192;
 constexpr uint32_t kWalkMaxSlots = kKeyBytes / (kBlock * sizeof(uint32_t));
+// keys per point that the dense ball query sorts in registers
+constexpr uint32_t kDenseSlots = 48;
 extern __shared__ __align__(16) unsigned char fa_dyn_lds[];
 
-// Dynamic LDS bytes for a fill block's keys: 1.3 x the mean bonds of kBlock
-// query points, between 4 KB and kKeyBytes.
-size_t fill_key_bytes(uint64_t bonds, uint64_t points, size_t key_size)
+
+// Dynamic LDS bytes for a fill block's keys: 1.3 x the mean bonds of its query
+// points, between 4 KB and kKeyBytes.
+size_t fill_key_bytes(uint64_t bonds, uint64_t points, size_t key_size, uint32_t block_points = kBlock)
 {
     double const per = points ? double(bonds) / double(points) : 0.0;
-    double const want = std::ceil(per * kBlock * 1.3) * double(key_size);
+    double const want = std::ceil(per * block_points * 1.3) * double(key_size);
     size_t const b = size_t(std::min(std::max(want, 4096.0), double(kKeyBytes)));
     return (b + 15) & ~size_t(15);
+}
+
+// LDS of kb bytes of keys and one owner byte per key.
+size_t owner_lds(size_t kb, size_t key_size)
+{
+    return kb + ((kb / key_size + 15) & ~size_t(15));
 }
 
 __device__ inline uint32_t float_order_bits(float v)
@@ -128,6 +137,64 @@ template<typename K> __device__ inline void insertion_sort(K* a, uint32_t n)
     }
 }
 
+// Batcher's odd-even merge sort of N registers (K. E. Batcher, 1968): every
+// lane sorts its own keys without a branch or a memory access.  191
+// comparators for 32 keys; an insertion sort in LDS runs the longest lane's
+// ~400 dependent steps.
+template<int N> __device__ inline void register_sort(uint32_t (&v)[N])
+{
+#pragma unroll
+    for (int p = 1; p < N; p *= 2)
+    {
+#pragma unroll
+        for (int k = p; k >= 1; k /= 2)
+        {
+#pragma unroll
+            for (int j = k % p; j + k < N; j += 2 * k)
+            {
+#pragma unroll
+                for (int i = 0; i < k; ++i)
+                {
+                    if (j + i + k < N && (j + i) / (2 * p) == (j + i + k) / (2 * p))
+                    {
+                        uint32_t const a = v[j + i], b = v[j + i + k];
+                        v[j + i] = min(a, b);
+                        v[j + i + k] = max(a, b);
+                    }
+                }
+            }
+        }
+    }
+}
+
+template<int N> __device__ inline void register_sort_keys(uint32_t* a, uint32_t n)
+{
+    uint32_t v[N];
+#pragma unroll
+    for (int m = 0; m < N; ++m)
+        v[m] = uint32_t(m) < n ? a[m] : ~0u;
+    register_sort<N>(v);
+#pragma unroll
+    for (int m = 0; m < N; ++m)
+        if (uint32_t(m) < n)
+            a[m] = v[m];
+}
+
+// Sorts the n keys at `a` (LDS) of each of the caller's lanes: 32-bit keys in
+// registers, as many as the wave's longest list needs (up to 32), others and
+// longer lists by insertion.
+template<typename K> __device__ inline void sort_keys(K* a, uint32_t n)
+{
+    if constexpr (sizeof(K) == sizeof(uint32_t))
+    {
+        if (!__builtin_amdgcn_ballot_w64(n > 16u))
+            return register_sort_keys<16>(a, n);
+        if (!__builtin_amdgcn_ballot_w64(n > 32u))
+            return register_sort_keys<32>(a, n);
+    }
+    insertion_sort(a, n);
+}
+
 // Writes the bond of query point i (at qx, qy, qz) given its key, at bond
 // index bidx.
 // NT: non-temporal stores, for a block's contiguous range of the
@@ -172,39 +239,82 @@ __device__ inline void write_bond(const DevBox& b, const float* __restrict__ qpt
                                    w_out, v_out);
 }
 
-// The point lo (< nloc) of a block whose key segment [s_off[lo], s_off[lo + 1])
-// holds element t < s_off[nloc].
-__device__ inline uint32_t segment_of(const uint32_t* s_off, uint32_t nloc, uint32_t t)
+// Marks the owner (point lo of the block) of each of its key slots: one pass of
+// short byte writes instead of a binary search over the offsets per key and
+// pass.  Every thread tid < nloc calls it with its own range.
+__device__ inline void mark_owner(uint8_t* own, uint32_t beg, uint32_t cnt)
 {
-    uint32_t lo = 0, hi = nloc;
-    while (hi - lo > 1)
-    {
-        uint32_t const mid = (lo + hi) >> 1;
-        if (s_off[mid] <= t)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
+    for (uint32_t m = 0; m < cnt; ++m)
+        own[beg + m] = uint8_t(threadIdx.x);
 }
 
 // Block-cooperative store of a block's bonds: keys[t] for t < total belong to
-// the block's query points in processing order (exclusive offsets s_off,
-// point indices s_i, positions s_q); bond t of point lo goes to
-// offsets[s_i[lo]] + t - s_off[lo].
-template<int FORMULA, bool BYDIST, typename K, bool NT = false>
+// the block's query points in processing order (owners own[t], exclusive
+// offsets s_off, point indices s_i, positions s_q); bond t of point lo goes to
+// offsets[s_i[lo]] + t - s_off[lo], which is first + t when the block's points
+// are consecutive (INDEX).  A wave's 64 bond vectors go through LDS, so that
+// every store instruction writes whole lines (three strided dword stores per
+// bond write each line three times).
+template<int FORMULA, bool BYDIST, typename K, bool INDEX>
 __device__ inline void store_block_bonds(const DevBox& b, const float* s_q, const float* __restrict__ pts,
-                                         const K* keys, uint32_t total, uint32_t nloc, const uint32_t* s_off,
-                                         const uint32_t* s_i, const uint32_t* __restrict__ offsets,
+                                         const K* keys, const uint8_t* own, uint32_t total, const uint32_t* s_off,
+                                         const uint32_t* s_i, const uint32_t* __restrict__ offsets, uint32_t first,
                                          uint32_t* __restrict__ nb_out, float* __restrict__ d_out,
                                          float* __restrict__ w_out, float* __restrict__ v_out)
 {
-    for (uint32_t t = threadIdx.x; t < total; t += kBlock)
+    __shared__ float s_v[kBlock / 64][192];
+    __shared__ uint32_t s_b[kBlock / 64][64];
+    uint32_t const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    for (uint32_t t0 = threadIdx.x - lane; t0 < total; t0 += kBlock)
     {
-        uint32_t const lo = segment_of(s_off, nloc, t);
-        uint32_t const i = s_i[lo];
-        write_bond_at<FORMULA, BYDIST, NT>(b, s_q[3 * lo], s_q[3 * lo + 1], s_q[3 * lo + 2], pts, i, uint64_t(keys[t]),
-                                       uint64_t(offsets[i]) + (t - s_off[lo]), nb_out, d_out, w_out, v_out);
+        uint32_t const t = t0 + lane, have = min(64u, total - t0);
+        if (t < total)
+        {
+            uint32_t const lo = own[t], i = s_i[lo];
+            uint32_t const jc = uint32_t(keys[t]), j = jc >> 5;
+            uint32_t const bidx = INDEX ? first + t : offsets[i] + (t - s_off[lo]);
+            float rx, ry, rz;
+            fa::bond_vector<FORMULA>(b, s_q[3 * lo], s_q[3 * lo + 1], s_q[3 * lo + 2], pts[3 * j], pts[3 * j + 1],
+                                     pts[3 * j + 2], int(jc & 31u), rx, ry, rz);
+            float const d = sqrtf((rx * rx + ry * ry) + rz * rz);
+            s_v[wave][3 * lane] = rx;
+            s_v[wave][3 * lane + 1] = ry;
+            s_v[wave][3 * lane + 2] = rz;
+            if (INDEX)
+            {
+                __builtin_nontemporal_store((uint64_t(j) << 32) | uint64_t(i),
+                                            reinterpret_cast<uint64_t*>(nb_out) + bidx);
+                __builtin_nontemporal_store(d, d_out + bidx);
+                __builtin_nontemporal_store(1.0f, w_out + bidx);
+            }
+            else
+            {
+                s_b[wave][lane] = bidx;
+                reinterpret_cast<uint2*>(nb_out)[bidx] = make_uint2(i, j);
+                d_out[bidx] = d;
+                w_out[bidx] = 1.0f;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the wave's vectors are in LDS
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c)
+        {
+            uint32_t const f = c * 64u + lane;
+            if (f < 3u * have)
+            {
+                float const v = s_v[wave][f];
+                if (INDEX)
+                    __builtin_nontemporal_store(v, v_out + 3 * uint64_t(first + t0) + f);
+                else
+                {
+                    uint32_t const m = f / 3u;
+                    v_out[3 * uint64_t(s_b[wave][m]) + (f - 3u * m)] = v;
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // and may be overwritten
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -225,6 +335,7 @@ __device__ inline void ball_fill_body(const DevBox& b, const DevGrid& g, const f
     // the kernel keeps its occupancy (blocks over the capacity use gkeys_raw)
     K* s_keys = reinterpret_cast<K*>(fa_dyn_lds);
     uint32_t const CAP = key_cap;
+    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
     __shared__ uint32_t s_off[kBlock + 1];
     __shared__ uint32_t s_i[kBlock];
     __shared__ uint32_t s_tmp[kBlock];
@@ -269,7 +380,13 @@ __device__ inline void ball_fill_body(const DevBox& b, const DevGrid& g, const f
                                                 ++k;
                                             }
                                         });
-        insertion_sort(keys + beg, k - beg);
+        if (in_lds)
+        {
+            mark_owner(s_own, beg, cnt);
+            sort_keys(s_keys + beg, k - beg);
+        }
+        else
+            insertion_sort(keys + beg, k - beg);
         if (!in_lds)
             for (uint32_t m = 0; m < k - beg; ++m)
                 write_bond<FORMULA, BYDIST>(b, qpts, pts, i, uint64_t(keys[beg + m]), uint64_t(offsets[i]) + m,
@@ -277,8 +394,8 @@ __device__ inline void ball_fill_body(const DevBox& b, const DevGrid& g, const f
     }
     __syncthreads();
     if (in_lds)
-        store_block_bonds<FORMULA, BYDIST>(b, s_q, pts, keys, total, nloc, s_off, s_i, offsets, nb_out, d_out,
-                                           w_out, v_out);
+        store_block_bonds<FORMULA, BYDIST, K, false>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets, 0u, nb_out,
+                                                     d_out, w_out, v_out);
 }
 
 // ------------------------------------------------------------------ ball query: one walk
@@ -385,6 +502,7 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
 {
     using K = typename std::conditional<BYDIST, uint64_t, uint32_t>::type;
     K* s_keys = reinterpret_cast<K*>(fa_dyn_lds);
+    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
     __shared__ uint32_t s_off[kBlock + 1];
     __shared__ uint32_t s_i[kBlock];
     __shared__ uint32_t s_tmp[kBlock];
@@ -432,6 +550,8 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
         return K(jc);
     };
     bool const coop = in_lds && C > 0;
+    if (in_lds && tid < nloc)
+        mark_owner(s_own, excl, cnt);
     if (coop)
     {
         // The staged key rows into LDS, element t by thread t: one load
@@ -443,7 +563,7 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
         __syncthreads();
         for (uint32_t t = tid; t < total; t += kBlock)
         {
-            uint32_t const lo = segment_of(s_off, nloc, t);
+            uint32_t const lo = s_own[t];
             uint32_t const r0 = s_row[lo];
             if (r0 != ~0u)
                 s_keys[t] = key_of(rows[r0 + (t - s_off[lo])], s_q[3 * lo], s_q[3 * lo + 1], s_q[3 * lo + 2]);
@@ -479,7 +599,10 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
                                          }
                                      });
         }
-        insertion_sort(keys + beg, cnt);
+        if (in_lds)
+            sort_keys(s_keys + beg, cnt);
+        else
+            insertion_sort(keys + beg, cnt);
         if (!in_lds)
             for (uint32_t m = 0; m < cnt; ++m)
                 write_bond_at<FORMULA, BYDIST>(b, qx, qy, qz, pts, i, uint64_t(keys[beg + m]),
@@ -487,8 +610,8 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
     }
     __syncthreads();
     if (in_lds)
-        store_block_bonds<FORMULA, BYDIST, K, INDEX>(b, s_q, pts, keys, total, nloc, s_off, s_i, offsets, nb_out,
-                                                     d_out, w_out, v_out);
+        store_block_bonds<FORMULA, BYDIST, K, INDEX>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets,
+                                                     INDEX ? offsets[p0] : 0u, nb_out, d_out, w_out, v_out);
 }
 
 template<int FORMULA, bool BYDIST, bool SELF, bool INDEX>
@@ -518,6 +641,76 @@ __global__ void counts_segments_kernel(const uint32_t* __restrict__ offsets, uin
     uint32_t const c = offsets[i + 1] - offsets[i];
     counts[i] = c;
     segments[i] = c ? offsets[i] : 0u;
+}
+
+// ------------------------------------------------------------------ dense ball queries
+// Lists too long for the walk's LDS key stage (33 bonds per point and more) are
+// counted, then walked again by the emission.  Up to kDenseSlots expected bonds
+// the keys are sorted in registers: an insertion sort in LDS took half of the
+// emission's time.  (Keeping the first walk's keys in device memory instead
+// made the walk dearer, 112 -> 199 us, than the second walk it saved.)
+// 500,000 random points, 28 bonds each: emission 640 -> 485 us.
+// The emission, in processing order, kDensePoints points per workgroup (their
+// keys fit 20 KB of LDS at 38 bonds each; workgroups over the capacity sort in
+// device memory, waves with a longer list than kDenseSlots by insertion).
+constexpr uint32_t kDensePoints = 128;
+template<int FORMULA, bool SELF>
+__global__ __launch_bounds__(kBlock) void ball_emit_dense_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
+                                                                 uint32_t nq, const float* __restrict__ pts,
+                                                                 float r_max_sq, float r_min_sq, int exclude_ii, int R,
+                                                                 fa::CQGrid cq, const uint32_t* __restrict__ offsets,
+                                                                 uint32_t* __restrict__ nb_out,
+                                                                 float* __restrict__ d_out, float* __restrict__ w_out,
+                                                                 float* __restrict__ v_out,
+                                                                 uint32_t* __restrict__ gkeys, uint32_t key_cap)
+{
+    uint32_t* const s_keys = reinterpret_cast<uint32_t*>(fa_dyn_lds);
+    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
+    __shared__ uint32_t s_off[kBlock + 1];
+    __shared__ uint32_t s_i[kBlock];
+    __shared__ uint32_t s_tmp[kBlock];
+    __shared__ float s_q[3 * kBlock];
+    uint32_t const tid = threadIdx.x;
+    uint32_t const p0 = fa::xcd_tile(blockIdx.x, gridDim.x) * kDensePoints;
+    uint32_t const nloc = min(kDensePoints, nq - p0);
+    float qx = 0.0f, qy = 0.0f, qz = 0.0f;
+    uint32_t i = 0, cnt = 0;
+    if (tid < nloc)
+    {
+        i = query_at<SELF>(g, qpts, p0 + tid, qx, qy, qz);
+        cnt = offsets[i + 1] - offsets[i];
+        s_i[tid] = i;
+        s_q[3 * tid] = qx;
+        s_q[3 * tid + 1] = qy;
+        s_q[3 * tid + 2] = qz;
+    }
+    uint32_t excl;
+    uint32_t const total = block_exclusive_scan(cnt, s_tmp, excl);
+    bool const in_lds = total <= key_cap;
+    if (tid < nloc)
+    {
+        s_off[tid] = excl;
+        uint32_t* const keys = in_lds ? s_keys + excl : gkeys + offsets[i];
+        if (in_lds)
+            mark_owner(s_own, excl, cnt);
+        uint32_t k = 0;
+        fa::visit_bonds<FORMULA>(b, g, cq, qx, qy, qz, R, [&](uint32_t j, float, float, float, float r_sq, int code) {
+            if (r_sq < r_max_sq && r_sq >= r_min_sq && k < cnt && !(exclude_ii && j == i))
+                keys[k++] = (j << 5) | uint32_t(code);
+        });
+        if (in_lds && !__builtin_amdgcn_ballot_w64(cnt > kDenseSlots))
+            register_sort_keys<int(kDenseSlots)>(s_keys + excl, cnt);
+        else
+            insertion_sort(keys, k);
+        if (!in_lds)
+            for (uint32_t m = 0; m < cnt; ++m)
+                write_bond_at<FORMULA, false>(b, qx, qy, qz, pts, i, uint64_t(keys[m]), uint64_t(offsets[i]) + m,
+                                              nb_out, d_out, w_out, v_out);
+    }
+    __syncthreads();
+    if (in_lds)
+        store_block_bonds<FORMULA, false, uint32_t, false>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets, 0u,
+                                                           nb_out, d_out, w_out, v_out);
 }
 
 // ------------------------------------------------------------------ kNN
@@ -1273,8 +1466,9 @@ __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, 
                                                            uint64_t* __restrict__ tmp, uint32_t key_cap)
 {
     using K = typename std::conditional<BYDIST, uint64_t, uint32_t>::type;
-    K* s_keys = reinterpret_cast<K*>(fa_dyn_lds); // key_cap entries (dynamic LDS)
+    K* s_keys = reinterpret_cast<K*>(fa_dyn_lds); // key_cap entries (dynamic LDS), then their owners
     uint32_t const CAP = key_cap;
+    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
     __shared__ uint32_t s_off[kBlock + 1];
     __shared__ uint32_t s_i[kBlock];
     __shared__ uint32_t s_tmp[kBlock];
@@ -1323,16 +1517,19 @@ __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, 
         // steps keeps ~12 MB of rows per XCD half read, far beyond its L2, and
         // fetched them about four times.)
         if (tid < nloc)
+        {
             s_row[tid] = INDEX && SELF ? pos[i] : p0 + tid;
+            mark_owner(s_own, excl, n);
+        }
         __syncthreads();
         for (uint32_t t = tid; t < total; t += kBlock)
         {
-            uint32_t const lo = segment_of(s_off, nloc, t);
+            uint32_t const lo = s_own[t];
             s_keys[t] = key_of(sel[uint64_t(s_row[lo]) * k + (t - s_off[lo])]);
         }
         __syncthreads();
         if (tid < nloc)
-            insertion_sort(s_keys + excl, n);
+            sort_keys(s_keys + excl, n);
     }
     else if (tid < nloc)
     {
@@ -1347,8 +1544,8 @@ __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, 
     }
     __syncthreads();
     if (in_lds)
-        store_block_bonds<FORMULA, BYDIST, K, INDEX>(b, s_q, pts, s_keys, total, nloc, s_off, s_i, offsets, nb_out, d_out,
-                                           w_out, v_out);
+        store_block_bonds<FORMULA, BYDIST, K, INDEX>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets,
+                                                     INDEX ? offsets[p0] : 0u, nb_out, d_out, w_out, v_out);
 }
 
 // ------------------------------------------------------------------ all pairs
@@ -1487,7 +1684,7 @@ int batch_ball_fill(const BatchGrid& G, const uint32_t* d_tile_frame, uint32_t n
     // the key staging is sized from the allocation (bonds per point of the batch)
     size_t const kb = fill_key_bytes(capacity, G.total_points, sizeof(uint32_t));
     if (ntiles)
-        FA_KLAUNCH(bball_fill_kernel, dim3(ntiles), dim3(kBlock), kb, stream(), G, d_tile_frame, ntiles, d_pts,
+        FA_KLAUNCH(bball_fill_kernel, dim3(ntiles), dim3(kBlock), owner_lds(kb, sizeof(uint32_t)), stream(), G, d_tile_frame, ntiles, d_pts,
                    r_max * r_max, R, d_offsets, d_total, capacity, nb, dist, wts, vec, gkeys,
                    uint32_t(kb / sizeof(uint32_t)));
     FA_HIP(hipGetLastError());
@@ -1523,7 +1720,7 @@ int batch_ball_emit(const BatchGrid& G, const uint32_t* d_tile_frame, uint32_t n
 {
     size_t const kb = fill_key_bytes(capacity, G.total_points, sizeof(uint32_t));
     if (ntiles)
-        FA_KLAUNCH(bball_emit_kernel, dim3(ntiles), dim3(kBlock), kb, stream(), G, d_tile_frame, ntiles, d_pts,
+        FA_KLAUNCH(bball_emit_kernel, dim3(ntiles), dim3(kBlock), owner_lds(kb, sizeof(uint32_t)), stream(), G, d_tile_frame, ntiles, d_pts,
                    r_max * r_max, R, C, d_pos, d_rows, d_offsets, d_total, capacity, nb, dist, wts, vec, gkeys,
                    uint32_t(kb / sizeof(uint32_t)));
     FA_HIP(hipGetLastError());
@@ -1903,14 +2100,14 @@ int launch_knn_lc(const fa::DevBox& db, const DevGrid& g, const float* qpts, uin
 // again by the emission pass.  When that exceeds 32 (a 32 KB LDS stage per
 // block) the walk only counts (0: every point is walked again, in processing
 // order, as a count pass and a fill pass would).
-uint32_t ball_row_slots(const fa_nq* nq, float r_max)
+uint32_t ball_row_slots(const fa_nq* nq, float r_max, uint32_t most = kWalkMaxSlots)
 {
     double const vol = std::max(double(fa::box_volume(nq->box)), 1e-30);
     double const dens = double(nq->n) / vol;
     double const r = double(r_max);
     double const expect = nq->box.is2D ? dens * M_PI * r * r : dens * (4.0 / 3.0) * M_PI * r * r * r;
     double const c = std::ceil((expect * 1.15 + 4.0) / 4.0) * 4.0;
-    if (c > double(kWalkMaxSlots))
+    if (c > double(most))
         return 0;
     return uint32_t(std::max(c, 8.0));
 }
@@ -2000,6 +2197,7 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
     }
     fa::CQGrid const cq = nq->kind == FA_NQ_CELLQUERY ? fa::cq_grid_for(nq->box, a.r_max) : fa::CQGrid{};
     uint32_t const C = ball_row_slots(nq, a.r_max);
+    bool const dense = !C && !by_distance && ball_row_slots(nq, a.r_max, kDenseSlots) != 0;
     uint32_t* rows = nullptr;
     uint32_t* pos = nullptr;
     if (n_query)
@@ -2046,11 +2244,36 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
     uint32_t const key_cap = uint32_t(kb / (by_distance ? 8 : 4));
     auto emit = [&](auto kern) {
         FA_PROF_BEGIN("ball_emit_kernel");
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), kb, s, db, g, qpts, n_query, nq->d_points, r_max_sq,
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), owner_lds(kb, by_distance ? 8 : 4), s, db, g, qpts, n_query,
+                           nq->d_points, r_max_sq,
                            r_min_sq, a.exclude_ii, R, cq, C, pos, rows, out->offsets, out->neighbors, out->distances,
                            out->weights, out->vectors, gkeys, key_cap);
         FA_PROF_END();
     };
+    if (dense && n_query)
+    {
+        size_t const dkb = fill_key_bytes(total, uint64_t(n_query) * (kBlock / kDensePoints), sizeof(uint32_t));
+        auto emit_dense = [&](auto kern) {
+            FA_PROF_BEGIN("ball_emit_kernel");
+            hipLaunchKernelGGL(kern, dim3((n_query + kDensePoints - 1) / kDensePoints), dim3(kBlock),
+                               owner_lds(dkb, sizeof(uint32_t)), s, db, g, qpts, n_query, nq->d_points, r_max_sq,
+                               r_min_sq, a.exclude_ii, R, cq, out->offsets, out->neighbors, out->distances,
+                               out->weights, out->vectors, static_cast<uint32_t*>(gkeys),
+                               uint32_t(dkb / sizeof(uint32_t)));
+            FA_PROF_END();
+        };
+        if (nq->kind == FA_NQ_AABB)
+            self ? emit_dense(ball_emit_dense_kernel<AABB_FORMULA, true>)
+                 : emit_dense(ball_emit_dense_kernel<AABB_FORMULA, false>);
+        else if (nq->kind == FA_NQ_CELLQUERY)
+            self ? emit_dense(ball_emit_dense_kernel<CELLQUERY_FORMULA, true>)
+                 : emit_dense(ball_emit_dense_kernel<CELLQUERY_FORMULA, false>);
+        else
+            self ? emit_dense(ball_emit_dense_kernel<LINKCELL_FORMULA, true>)
+                 : emit_dense(ball_emit_dense_kernel<LINKCELL_FORMULA, false>);
+        FA_HIP(hipGetLastError());
+        return FA_OK;
+    }
     // self queries of points stored in random order emit in processing order,
     // and so does a walk that kept no keys (the emission pass walks again)
     bool index_order = C > 0;
@@ -2418,7 +2641,7 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
     DevGrid const g = nq->cur->dev();
     auto launch = [&](auto kern) {
         FA_PROF_BEGIN("knn_write_kernel");
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), kb, s, *dbp, g, qpts, n_query, nq->d_points, k, sel,
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), owner_lds(kb, ksz), s, *dbp, g, qpts, n_query, nq->d_points, k, sel,
                            pos, out->offsets, out->neighbors, out->distances, out->weights, out->vectors, wtmp,
                            key_cap);
         FA_PROF_END();

@@ -195,3 +195,26 @@ def test_wave_ball_query_falls_back_on_clumps(oracle):
     for args in (dict(r_max=1.5, exclude_ii=True), dict(num_neighbors=12, exclude_ii=True)):
         ref = oracle.query(_bt(box), pts, pts, args, nthreads=4)
         _assert_same(freud_amd.AABBQuery(box, pts).query(pts, args).toNeighborList(), ref)
+
+
+@pytest.mark.parametrize("kind", ["aabb", "linkcell", "cellquery"])
+@pytest.mark.parametrize("bonds", [7, 15, 30, 37, 45])
+def test_large_ball_queries_by_bond_count(oracle, kind, bonds):
+    """More points than the wave queries take, on both sides of the register
+    sorts (16, 32, 48 keys) and of the LDS and device-memory key stages, with a
+    clump past every stage; consecutive and scattered storage orders."""
+    n, side = 33000, 32.08
+    box = Box.cube(side)
+    rng = np.random.default_rng(bonds)
+    pts = ((rng.random((n, 3)) - 0.5) * side).astype(np.float32)
+    pts[:200] = (rng.standard_normal((200, 3)) * 0.5).astype(np.float32)
+    r = (bonds / 4.18879) ** (1 / 3)
+    cls = {"aabb": freud_amd.AABBQuery, "linkcell": freud_amd.LinkCell, "cellquery": freud_amd.CellQuery}[kind]
+    for points in (pts, pts[np.lexsort((pts[:, 0] // 1, pts[:, 1] // 1, pts[:, 2] // 1))]):
+        nq = cls(box, points) if kind != "linkcell" else cls(box, points, cell_width=r)
+        args = dict(r_max=r, exclude_ii=True)
+        for by_distance in (False, True):
+            ref = oracle.query(_bt(box), points, points, args, nq_type=kind if kind != "cellquery" else "cellquery",
+                               cell_width=r, sort_by_distance=by_distance, nthreads=16)
+            nl = nq.query(points, args).toNeighborList(sort_by_distance=by_distance)
+            _assert_same(nl, ref)
