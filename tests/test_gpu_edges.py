@@ -218,3 +218,33 @@ def test_large_ball_queries_by_bond_count(oracle, kind, bonds):
                                cell_width=r, sort_by_distance=by_distance, nthreads=16)
             nl = nq.query(points, args).toNeighborList(sort_by_distance=by_distance)
             _assert_same(nl, ref)
+
+
+@pytest.mark.parametrize("parts", [1, 3, 70])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, 5000])
+def test_cluster_chains(n, parts):
+    """Chains interleaved through the indices (one, three or more clusters in
+    every wave), every eleventh point alone: sizes and members are whole
+    numbers, equal to a host union's."""
+    members = np.arange(n, dtype=np.uint32)
+    chained = members[members % 11 != 5]
+    a, b = chained[:-parts], chained[parts:]
+    if parts >= len(chained):
+        a = b = chained[:0]
+    label = members.copy()
+    for x, y in zip(a, b):
+        label[y] = label[x]
+    _, inverse, count = np.unique(label, return_inverse=True, return_counts=True)
+    order = np.argsort(-count, kind="stable")
+    rank = np.empty_like(order)
+    rank[order] = np.arange(len(order))
+    box = Box.cube(100.0)
+    pts = np.zeros((n, 3), np.float32)
+    if len(a):
+        nl = freud_amd.locality.NeighborList.from_arrays(n, n, a, b, np.ones((len(a), 3), np.float32))
+    else:
+        pts[:, 0] = np.arange(n) * np.float32(100.0 / (n + 1)) - 50
+        nl = freud_amd.AABBQuery(box, pts).query(pts, dict(r_max=1e-3, exclude_ii=True)).toNeighborList()
+    cl = freud_amd.cluster.Cluster().compute((box, pts), neighbors=nl)
+    assert cl.num_clusters == len(count)
+    npt.assert_array_equal(cl.cluster_idx, rank[inverse])
