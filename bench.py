@@ -113,7 +113,7 @@ def algorithmic_bytes(name, n, b_ball, b_knn, k=12, l=6, bins=200):
         "knn_stage_kernel": 16 * n + 4 * n + 4 * n + 8 * k * n,
         "knn_write_kernel": 8 * k * n + 4 * n + 4 * (n + 1) + 12 * n + 28 * b_knn,
         "rdf_self_kernel": 16 * n + 4 * bins,
-        "rdf_cluster_kernel": 16 * n + 4 * bins,
+        "rdf_est_kernel": 16 * n + 4 * bins,
         "qlm_kernel": 24 * b_ball + 8 * nm * n + 4 * n,
         "qlm_ave_kernel": 4 * b_ball + 4 * (n + 1) + 8 * nm * n + 8 * nm * n + 4 * n,
         "wl_kernel": 8 * nm * n + 4 * n + 4 * n,
