@@ -160,6 +160,8 @@ _SIGS = {
                                             ctypes.POINTER(fa_nlist)]),
     "fa_nlist_all_pairs": (ctypes.c_int, [ctypes.POINTER(fa_box), ctypes.c_void_p, ctypes.c_uint32, ctypes.c_void_p,
                                           ctypes.c_uint32, ctypes.c_int, ctypes.POINTER(fa_nlist)]),
+    "fa_nlist_offsets": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_uint32, ctypes.c_void_p, ctypes.c_void_p,
+                                        ctypes.POINTER(ctypes.c_uint64)]),
     "fa_nlist_filter": (ctypes.c_int, [ctypes.POINTER(fa_nlist), ctypes.c_void_p]),
     "fa_nlist_filter_r": (ctypes.c_int, [ctypes.POINTER(fa_nlist), ctypes.c_float, ctypes.c_float]),
     "fa_nlist_sort": (ctypes.c_int, [ctypes.POINTER(fa_nlist), ctypes.c_int]),

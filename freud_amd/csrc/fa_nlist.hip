@@ -346,6 +346,16 @@ int fa_nlist_sort(fa_nlist* nl, int by_distance)
     return FA_OK;
 }
 
+int fa_nlist_offsets(const uint32_t* d_counts, uint32_t n, uint32_t* d_offsets, uint32_t* d_segments, uint64_t* total)
+{
+    FA_API_LOCK;
+    if (int rc = fa_init())
+        return rc;
+    if (!d_offsets || !total || (n && !d_counts))
+        return fa::fail(FA_ERR_INVALID, "NeighborList offsets need counts, offsets and a total");
+    return fa::exclusive_scan_u32(d_counts, d_offsets, n, total, nullptr, nullptr, 1, d_segments);
+}
+
 int fa_nlist_copy(const fa_nlist* src, fa_nlist* dst)
 {
     FA_API_LOCK;

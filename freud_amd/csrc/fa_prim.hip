@@ -26,6 +26,8 @@ struct widen
 // Up to kScanSingle counts take the second kernel alone.  The input is read
 // twice, so above kOwnScan (16 MiB) rocPRIM's single pass is the better one.
 // No state outlives a call and nothing is cleared, so both can be captured.
+// Offsets wrap at 32 bits, totals are summed in 64: callers refuse a list by
+// its total before anything is sized from it.
 // 250,000 points (a kNN list and its grid): nine commands fewer, 148 -> 138 us for the query and psi_6.
 constexpr uint32_t kScanThreads = 512;
 constexpr uint32_t kScanTile = kScanThreads * 8;
@@ -89,13 +91,14 @@ __global__ __launch_bounds__(kScanThreads) void scan_parts_kernel(const uint32_t
     __shared__ uint64_t s[kScanThreads / 64];
     __shared__ uint32_t s_wave[kScanThreads / 64];
     uint32_t const tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    uint64_t before = 0;
+    uint64_t first = 0, own = 0; // sum of the parts before this one; this thread's counts
     if (blockIdx.x)
     {
         for (uint32_t t = tid; t < blockIdx.x; t += kScanThreads)
-            before += sums[t];
-        before = block_sum(before, s);
+            first += sums[t];
+        first = block_sum(first, s);
     }
+    uint32_t before = uint32_t(first); // offsets are 32 bits wide, the total is not
     uint32_t const beg = blockIdx.x * part, end = min(n - beg, part) + beg;
     for (uint32_t t0 = beg; t0 < end; t0 += kScanTile)
     {
@@ -106,6 +109,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_parts_kernel(const uint32_t
         {
             v[k] = i0 + k < end ? in[i0 + k] : 0u;
             sum += v[k];
+            own += v[k];
         }
         uint32_t incl = sum;
 #pragma unroll
@@ -119,15 +123,14 @@ __global__ __launch_bounds__(kScanThreads) void scan_parts_kernel(const uint32_t
         if (lane == 63u)
             s_wave[wave] = incl;
         __syncthreads();
-        uint32_t base = 0;
-        uint64_t tile = 0;
+        uint32_t base = 0, tile = 0;
 #pragma unroll
         for (uint32_t w = 0; w < kScanThreads / 64; ++w)
         {
             base += w < wave ? s_wave[w] : 0u;
             tile += s_wave[w];
         }
-        uint32_t x = uint32_t(before) + base + (incl - sum);
+        uint32_t x = before + base + (incl - sum);
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k)
         {
@@ -141,12 +144,15 @@ __global__ __launch_bounds__(kScanThreads) void scan_parts_kernel(const uint32_t
         }
         before += tile;
     }
-    if (end == n && tid == 0)
+    if (end != n) // the last part only from here on
+        return;
+    uint64_t const total = first + block_sum(own, s);
+    if (tid == 0)
     {
-        out[n] = uint32_t(before);
+        out[n] = uint32_t(total);
         if (host)
         {
-            __hip_atomic_store(host, before, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(host, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             for (int k = 0; k < n_extra; ++k)
                 __hip_atomic_store(reinterpret_cast<uint32_t*>(host + 1) + k, extra[k], __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_SYSTEM);

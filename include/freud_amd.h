@@ -210,6 +210,10 @@ int fa_nlist_free(fa_nlist* nl);
 int fa_nlist_from_arrays(uint32_t num_query_points, uint32_t num_points, const uint32_t* d_query_point_indices,
                          const uint32_t* d_point_indices, const float* d_vectors, const float* d_weights,
                          uint64_t num_bonds, fa_nlist* out);
+/* Offsets (n + 1), segments (n; may be NULL) and the 64-bit bond total of a list
+ * with the given bond counts per query point, as every query computes them
+ * (NeighborList.cc:199-232).  Offsets wrap at 2^32; the total does not. */
+int fa_nlist_offsets(const uint32_t* d_counts, uint32_t n, uint32_t* d_offsets, uint32_t* d_segments, uint64_t* total);
 /* NeighborList::NeighborList(points, query_points, box, exclude_ii, ...)
  * all_pairs (freud/locality/NeighborList.cc:84-128). */
 int fa_nlist_all_pairs(const fa_box* box, const float* d_points, uint32_t n_points, const float* d_query_points,

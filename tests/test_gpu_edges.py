@@ -1,11 +1,14 @@
 """Sizes at which the launch shapes of the kernels change: tile edges and
 remainders, the smallest systems, and the borders between two code paths."""
 
+import ctypes
+
 import numpy as np
 import numpy.testing as npt
 import pytest
 
 import freud_amd
+from freud_amd import _lib
 from freud_amd.box import Box
 
 pytestmark = pytest.mark.gpu
@@ -137,6 +140,25 @@ def test_scan_sizes_through_filter(bonds):
     npt.assert_array_equal(nl[:], np.stack([i[keep], j[keep]], 1))
     npt.assert_array_equal(nl.vectors, v[keep])
     npt.assert_array_equal(nl.neighbor_counts, np.bincount(i[keep], minlength=n))
+
+
+@pytest.mark.parametrize("n", [0, 1, 511, 512, 8192, 8193, 70001, (1 << 22), (1 << 22) + 5])
+@pytest.mark.parametrize("largest", [3, 9_000_000, 2**32 - 1])
+def test_scan_totals_beyond_32_bits(n, largest):
+    """The total of a list is a 64-bit sum whatever its counts (a query refuses
+    a list by it); offsets and segments are the sums modulo 2^32."""
+    counts = np.random.default_rng(n).integers(largest // 2, largest + 1, n, dtype=np.uint32)
+    counts[::5] = 0
+    d_counts = _lib.DeviceArray.from_numpy(counts)
+    d_offsets, d_segments = _lib.DeviceArray((n + 1,), np.uint32), _lib.DeviceArray((max(n, 1),), np.uint32)
+    total = ctypes.c_uint64()
+    _lib.check(_lib.lib().fa_nlist_offsets(d_counts.ptr, n, d_offsets.ptr, d_segments.ptr,
+                                           ctypes.byref(total)))
+    sums = np.cumsum(np.concatenate([[0], counts]), dtype=np.uint64)
+    assert total.value == int(sums[-1])
+    offsets = (sums & np.uint64(2**32 - 1)).astype(np.uint32)
+    npt.assert_array_equal(d_offsets.numpy(), offsets)
+    npt.assert_array_equal(d_segments.numpy()[:n], np.where(counts > 0, offsets[:-1], 0))
 
 
 @pytest.mark.parametrize("n", [2, 4096, 8192, 8193, 40001])
