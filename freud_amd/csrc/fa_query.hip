@@ -1070,27 +1070,29 @@ __device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float 
     for (int c0 = 0; c0 < ncell; c0 += 64)
     {
         uint32_t beg = 0u, len = 0u;
-        int shift = 0; // image offset of the cell per axis, 10 bits each (biased by 512)
+        // the cell's shift in box lengths per axis, 4 bits each (biased by 8: R is
+        // at most 3); the query's own image offset, of any size, is added below
+        int shift = 0;
         int const t = c0 + int(lane);
         if (t < ncell)
         {
             int const d[3] = {t % side - R, (t / side) % side - R, t / (side * side) - Rz};
-            int cell[3], nb[3];
+            int cell[3], sh[3];
             bool in = true;
 #pragma unroll
             for (int k = 0; k < 3; ++k)
             {
-                int const u = c[k] + d[k], s = fa::floor_div(u, g.dim[k]);
-                cell[k] = u - s * g.dim[k];
-                nb[k] = -w[k] - s;
-                in = in && (outside ? nb[k] >= -500 && nb[k] <= 500 : nb[k] >= -1 && nb[k] <= 1);
+                int const u = c[k] + d[k];
+                sh[k] = fa::floor_div(u, g.dim[k]);
+                cell[k] = u - sh[k] * g.dim[k];
+                in = in && (outside || (-w[k] - sh[k] >= -1 && -w[k] - sh[k] <= 1));
             }
             if (in)
             {
                 uint32_t const id = uint32_t((cell[2] * g.dim[1] + cell[1]) * g.dim[0] + cell[0]);
                 beg = g.cstart[id];
                 len = g.cstart[id + 1] - beg;
-                shift = (nb[0] + 512) | ((nb[1] + 512) << 10) | ((nb[2] + 512) << 20);
+                shift = (sh[0] + 8) | ((sh[1] + 8) << 4) | ((sh[2] + 8) << 8);
             }
         }
         uint32_t e = len; // inclusive scan over the lanes
@@ -1124,7 +1126,7 @@ __device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float 
             }
             bool valid = v < tot;
             float4 const pj = g.cpos[valid ? pos : 0u];
-            int n0 = (code3 & 1023) - 512, n1 = ((code3 >> 10) & 1023) - 512, n2 = ((code3 >> 20) & 1023) - 512;
+            int n0 = 8 - (code3 & 15) - w[0], n1 = 8 - ((code3 >> 4) & 15) - w[1], n2 = 8 - ((code3 >> 8) & 15) - w[2];
             if (outside)
             {
                 int wj[3];

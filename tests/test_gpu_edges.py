@@ -207,6 +207,27 @@ def test_wave_queries(oracle, name, n, outside):
                 _assert_same(nl, ref)
 
 
+@pytest.mark.parametrize("n", [700, 40000])
+@pytest.mark.parametrize("boxes", [-511, -505, -500, 499, 500, 501, 505, 510])
+def test_points_many_boxes_out(oracle, n, boxes):
+    """Unwrapped coordinates hundreds of box lengths out: the image offsets of a
+    point and of its query cancel, on both sides of the wave queries' largest
+    size.  Box lengths and coordinates are dyadic, so that the shift is exact."""
+    side = 8.0 if n < 32768 else 32.0
+    box = Box.cube(side)
+    rng = np.random.default_rng(n)
+    pts = ((rng.integers(0, 2**10, (n, 3)) + 0.5) * (side / 2**10) - side / 2).astype(np.float32)
+    pts[:, 1] += np.float32(side * boxes)
+    nq = freud_amd.AABBQuery(box, pts)
+    q = pts[::3]
+    for args in (dict(r_max=1.0, exclude_ii=True), dict(num_neighbors=6, exclude_ii=True)):
+        for points in (pts, q):
+            ref = oracle.query(_bt(box), pts, points, args, nthreads=16)
+            nl = nq.query(points, args).toNeighborList()
+            _assert_same(nl, ref)
+            assert len(ref["distances"]) > 0
+
+
 def test_wave_ball_query_falls_back_on_clumps(oracle):
     """A clump with more bonds per point than a wave keeps: the per-thread
     query takes the call."""
