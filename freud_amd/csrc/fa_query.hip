@@ -1261,16 +1261,17 @@ __global__ __launch_bounds__(kBlock) void knn_wave_kernel(DevBox b, DevGrid g, c
     for (int R = 1; R <= 3 && !done; ++R)
     {
         float const complete = float(R) * wmin * (1.0f - 1e-4f);
+        bool const whole = complete >= rlim; // the stencil covers every candidate, d = rlim included
         n = 0; // keys with d < complete
         wave_candidates(b, g, qx, qy, qz, R, [&](bool valid, uint32_t j, int code, float r_sq) {
             bool take = valid && r_sq < rlim_sq && r_sq >= rmin_thr && !(exclude_ii && j == i);
             uint64_t const key = knn_key(r_sq, (j << 5) | uint32_t(code));
-            take = take && knn_key_distance(key) < complete;
+            take = take && (whole || knn_key_distance(key) < complete);
             wave_append(keys, n, take, key);
         });
         if (n > kWaveKeys)
             break;
-        done = n >= k || complete >= rlim; // inside `complete` nothing is missing
+        done = n >= k || whole; // inside `complete` nothing is missing
         if (!done && complete >= half_min_plane && rlim > half_min_plane)
             break; // longer searches, and the exhaustive flag, are the ring search's
     }

@@ -228,6 +228,27 @@ def test_points_many_boxes_out(oracle, n, boxes):
             assert len(ref["distances"]) > 0
 
 
+def test_nearest_query_at_the_stencil_radius(oracle):
+    """A search radius equal to the radius that the cells cover (box length
+    20, cells of 5, less 1e-4): a neighbour below it in r_sq whose rounded
+    distance equals it belongs to the answer."""
+    f = np.float32
+    r = f(5) * (f(1) - f(1e-4))
+    ang = np.random.default_rng(0).random(20000) * np.pi / 2
+    x, y = (r * np.cos(ang)).astype(f), (r * np.sin(ang)).astype(f)
+    r_sq = x * x + y * y
+    on = np.nonzero((r_sq < r * r) & (np.sqrt(r_sq) == r))[0][:7]
+    assert len(on) == 7
+    box = Box.cube(20)
+    pts = ((np.random.default_rng(1).random((1000, 3)) - 0.5) * 20).astype(f)
+    pts[:7] = np.stack([x[on], y[on], 0 * x[on]], 1)
+    q = np.zeros((1, 3), f)
+    args = dict(num_neighbors=20, r_max=float(r), r_guess=float(r), r_min=4.999)
+    ref = oracle.query(_bt(box), pts, q, args, nthreads=1)
+    assert 7 <= len(ref["distances"]) < 20
+    _assert_same(freud_amd.AABBQuery(box, pts).query(q, args).toNeighborList(), ref)
+
+
 def test_wave_ball_query_falls_back_on_clumps(oracle):
     """A clump with more bonds per point than a wave keeps: the per-thread
     query takes the call."""
