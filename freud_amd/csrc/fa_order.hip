@@ -186,6 +186,13 @@ template<int L> __device__ inline void accumulate_ylm(float ct, float st, float 
 // stream through L2 (thousands of such streams per CU thrash the cache).
 // Ranges longer than the staging capacity read global memory.
 constexpr uint32_t kStage = 4096;
+
+// Neighbour of bond e: lists hold up to 2^32 - 1 bonds, so 2 e + 1 would wrap.
+__device__ inline uint32_t bond_neighbor(const uint32_t* __restrict__ nbr, uint32_t e)
+{
+    return reinterpret_cast<const uint2*>(nbr)[e].y;
+}
+
 struct BondSrc
 {
     const uint32_t* nbr;
@@ -194,7 +201,7 @@ struct BondSrc
     const float* sd;
     uint32_t base;
     bool staged;
-    __device__ uint32_t j(uint32_t e) const { return staged ? sj[e - base] : nbr[2 * e + 1]; }
+    __device__ uint32_t j(uint32_t e) const { return staged ? sj[e - base] : bond_neighbor(nbr, e); }
     __device__ float d(uint32_t e) const { return staged ? sd[e - base] : dist[e]; }
 };
 
@@ -645,7 +652,7 @@ __global__ __launch_bounds__(kBlock) void qlm_ave_kernel(uint32_t n, const uint3
         auto row = [&](uint32_t j) { return load_row_part<L>(rows + uint64_t(j) * row_stride, sub); };
         auto fetch = [&](uint32_t e) { return row(src.j(e)); };
         uint32_t e = e0;
-        for (; e + 4 <= e1; e += 4) // four rows in flight
+        for (; e1 - e >= 4u; e += 4) // four rows in flight
         {
             float4 const v0 = fetch(e), v1 = fetch(e + 1), v2 = fetch(e + 2), v3 = fetch(e + 3);
             add(v0);
@@ -1052,7 +1059,7 @@ __device__ inline uint32_t solid_bond_count(uint32_t i, int l, const uint32_t* _
     }
     for (uint32_t e = e0; e < e1; ++e)
     {
-        uint32_t const j = tile.staged ? tile.sj[e - tile.base] : nbr[2 * e + 1];
+        uint32_t const j = tile.staged ? tile.sj[e - tile.base] : bond_neighbor(nbr, e);
         const float2* qj = qlm + uint64_t(j) * nm;
         float re = 0.0f;
         if (NM)
@@ -1136,10 +1143,11 @@ __global__ __launch_bounds__(kBlock) void solid_bonds6_kernel(uint32_t n, const 
         float4 const a = rows[uint64_t(i) * 4 + sub];
         float const qi = quad_lane<3>(a.z);
         uint32_t cnt = 0;
-        for (uint32_t e = e0; e < e1; e += 4)
+        uint32_t const bonds = e1 - e0; // counted from 0: e0 + bonds may be 2^32 - 1
+        for (uint32_t t = 0; t < bonds; t += 4)
         {
-            uint32_t const x = min(e + sub, e1 - 1u);
-            int const j = int(staged ? sj[x - b0] : nbr[2 * x + 1]);
+            uint32_t const x = e0 + min(t + sub, bonds - 1u);
+            int const j = int(staged ? sj[x - b0] : bond_neighbor(nbr, x));
             float4 c[4];
             c[0] = rows[uint64_t(uint32_t(__builtin_amdgcn_mov_dpp(j, 0x00, 0xf, 0xf, true))) * 4 + sub];
             c[1] = rows[uint64_t(uint32_t(__builtin_amdgcn_mov_dpp(j, 0x55, 0xf, 0xf, true))) * 4 + sub];
@@ -1170,12 +1178,12 @@ __global__ __launch_bounds__(kBlock) void solid_bonds6_kernel(uint32_t n, const 
             }
             if (normalize_q)
                 own *= nf / (qi * qj);
-            if (e + sub < e1)
+            if (t + sub < bonds)
             {
                 if (staged)
-                    so[e + sub - b0] = own;
+                    so[x - b0] = own;
                 else
-                    ql_ij[e + sub] = own;
+                    ql_ij[x] = own;
                 cnt += own > q_threshold ? 1u : 0u;
             }
         }
@@ -1371,7 +1379,7 @@ __global__ __launch_bounds__(kBlock) void uf_hook_min_kernel(uint32_t n, const u
         {
             bool const k = !keep || (staged ? sk[e - b0] : keep[e]);
             if (k)
-                m = min(m, staged ? sj[e - b0] : nbr[2 * e + 1]);
+                m = min(m, staged ? sj[e - b0] : bond_neighbor(nbr, e));
         }
         parent[i] = m;
     }
@@ -1565,7 +1573,7 @@ __global__ __launch_bounds__(kBlock) void hexatic_kernel(fa::DevBox b, const flo
     float re = 0.0f, im = 0.0f, total = 0.0f;
     for (uint32_t e = offsets[i]; e < offsets[i + 1]; ++e)
     {
-        uint32_t const j = nbr[2 * e + 1];
+        uint32_t const j = bond_neighbor(nbr, e);
         float dx, dy, dz;
         fa::wrap(b, pts[3 * j] - pts[3 * i], pts[3 * j + 1] - pts[3 * i + 1], pts[3 * j + 2] - pts[3 * i + 2], dx, dy,
                  dz);

@@ -59,6 +59,56 @@ def test_solid_bonds_lane_groups(oracle, l, n, normalize):
         npt.assert_array_equal(sl.cluster_idx, ref["cluster_idx"])
 
 
+@pytest.mark.parametrize("l", [4, 6])
+def test_steinhardt_and_solid_bonds_unstaged(oracle, l):
+    """A clump whose tiles hold more bonds than the LDS stage next to ordinary
+    tiles: both branches of the bond kernels and of the averaged q_l."""
+    box = Box.cube(24.0)
+    rng = np.random.default_rng(l)
+    pts = ((rng.random((3000, 3)) - 0.5) * 24).astype(np.float32)
+    pts[:400] = (rng.standard_normal((400, 3)) * 0.6).astype(np.float32)
+    args = dict(r_max=1.5, exclude_ii=True)
+    nl = freud_amd.AABBQuery(box, pts).query(pts, args).toNeighborList()
+    assert nl.neighbor_counts[:256].sum() > 4096 and nl.neighbor_counts[512:768].sum() < 4096
+    ref_nl = oracle.query(_bt(box), pts, pts, args, nthreads=4)
+    st = freud_amd.order.Steinhardt(l, average=True).compute((box, pts), neighbors=nl)
+    ref = oracle.steinhardt(_bt(box), pts, ref_nl, [l], average=True, nthreads=4)
+    npt.assert_allclose(st.particle_order, ref["ql_ave"][:, 0], atol=1e-5, equal_nan=True)
+    sl = freud_amd.order.SolidLiquid(l, 0.3, 4).compute((box, pts), neighbors=nl)
+    one = freud_amd.order.Steinhardt(l).compute((box, pts), neighbors=nl)
+    ref = oracle.solidliquid(ref_nl, one.particle_harmonics, one.ql, l, 0.3, 4, normalize_q=True)
+    npt.assert_allclose(sl.ql_ij, ref["ql_ij"], rtol=1e-6, atol=1e-7, equal_nan=True)
+
+
+@pytest.mark.parametrize("l", [4, 6])
+def test_solid_bonds_past_two_to_the_31(l):
+    """A list of 2,152,913,600 bonds (60 GB): those past 2^31, the last 117
+    points', have the neighbours that the list says.  q_lm against a run with
+    the points reversed, where those points come first: means of 46,399
+    terms of size 1, each sum within a few hundred ulps of 2^-24 (1e-6 allowed).
+    Dot products against float64 from the run's own q_lm: 13 products and sums
+    of 2^-24 each of |q_i| |q_j| (4e-6 allowed).  Another neighbour differs by
+    1e-3 and 1e-1."""
+    n, tail = 46400, 117
+    box = Box.cube(40.0)
+    pts = ((np.random.default_rng(0).random((n, 3)) - 0.5) * 40).astype(np.float32)
+    qlm = []
+    for points in (pts[::-1].copy(), pts):
+        nl = freud_amd.locality.NeighborList.all_pairs((box, points))
+        sl = freud_amd.order.SolidLiquid(l, 0.5, n).compute((box, points), neighbors=nl)
+        qlm.append(sl.particle_harmonics)
+        first = (n - tail) * (n - 1)
+        assert 2**31 < first < len(nl) == n * (n - 1)
+        dots = _lib.copy_d2h(sl._d_qlij.ptr + 4 * first, (tail, n - 1), np.float32)
+        del sl, nl
+    npt.assert_allclose(qlm[1][-tail:], qlm[0][:tail][::-1], atol=1e-6)
+    q = qlm[1].astype(np.complex128)
+    q /= np.linalg.norm(q, axis=1)[:, None]
+    ref = (q[-tail:] @ q.conj().T).real
+    others = np.arange(n) != np.arange(n - tail, n)[:, None]
+    npt.assert_allclose(dots, ref[others].reshape(tail, n - 1), atol=4e-6)
+
+
 BOXES = {
     "cube": Box.cube(16),
     "triclinic": Box(12.0, 13.0, 14.0, 0.3, -0.2, 0.25),
