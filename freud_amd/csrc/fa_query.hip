@@ -1177,14 +1177,15 @@ template<typename F> __device__ inline void wave_rank(const uint64_t* keys, uint
 }
 
 // Ball query, one wave per query position: the point's keys (j << 5 | image
-// code) in NeighborList order into rows[i * C ..], its bond count, and a mark
-// when some point has more than C bonds (the caller then runs the per-thread
-// query).
+// code) in NeighborList order into rows[pos[i] ..], its bond count, and a mark
+// when some point has more than C bonds (no row: the general emission, which
+// walks such points again, then takes the place of wave_emit_kernel).
 template<bool BYDIST, bool SELF>
 __global__ __launch_bounds__(kBlock) void ball_wave_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
                                                            uint32_t nq, float r_max_sq, float r_min_sq, int exclude_ii,
                                                            int R, uint32_t C, uint32_t* __restrict__ counts,
-                                                           uint32_t* __restrict__ rows, uint32_t* __restrict__ over)
+                                                           uint32_t* __restrict__ pos, uint32_t* __restrict__ rows,
+                                                           uint32_t* __restrict__ over)
 {
     __shared__ uint64_t s_keys[kWaves][kWaveKeys];
     uint32_t const wave = threadIdx.x >> 6;
@@ -1203,6 +1204,7 @@ __global__ __launch_bounds__(kBlock) void ball_wave_kernel(DevBox b, DevGrid g, 
     if ((threadIdx.x & 63u) == 0)
     {
         counts[i] = n;
+        pos[i] = i * C;
         if (n > C)
             *over = 1u; // every writer stores the same value
     }
@@ -1212,7 +1214,6 @@ __global__ __launch_bounds__(kBlock) void ball_wave_kernel(DevBox b, DevGrid g, 
 
 // Emission for ball_wave_kernel: 16 lanes per query point write its bonds from
 // its sorted keys (stride C).
-template<int FORMULA>
 __global__ __launch_bounds__(kBlock) void wave_emit_kernel(DevBox b, const float* __restrict__ qpts, uint32_t nq,
                                                            const float* __restrict__ pts,
                                                            const uint32_t* __restrict__ rows, uint32_t C,
@@ -1226,8 +1227,8 @@ __global__ __launch_bounds__(kBlock) void wave_emit_kernel(DevBox b, const float
     uint32_t const e0 = offsets[i], n = offsets[i + 1] - e0;
     float const qx = qpts[3 * i], qy = qpts[3 * i + 1], qz = qpts[3 * i + 2];
     for (uint32_t m = threadIdx.x & 15u; m < n; m += 16u)
-        write_bond_at<FORMULA, false>(b, qx, qy, qz, pts, i, uint64_t(rows[uint64_t(i) * C + m]), uint64_t(e0) + m,
-                                      nb_out, d_out, w_out, v_out);
+        write_bond_at<AABB_FORMULA, false>(b, qx, qy, qz, pts, i, uint64_t(rows[uint64_t(i) * C + m]),
+                                           uint64_t(e0) + m, nb_out, d_out, w_out, v_out);
 }
 
 // kNN, one wave per query position (see the ring search for what is selected):
@@ -2127,50 +2128,6 @@ uint32_t ball_wave_slots(const fa_nq* nq, float r_max)
     return expect > kWaveKeys / 3 ? 0u : uint32_t(std::min<double>(kWaveKeys, 2.0 * expect + 32.0));
 }
 
-// The ball query of a small system on nq->cur.  handled = false: some point
-// has more bonds than slots (nothing but counts has been written).
-int run_ball_wave(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args& a, int by_distance, bool self,
-                  uint32_t C, fa_nlist* out, bool* handled)
-{
-    *handled = false;
-    hipStream_t s = fa::stream();
-    DevGrid const g = nq->cur->dev();
-    fa::DevBox const& db = nq->cur->dbox;
-    float const r_max_sq = a.r_max * a.r_max, r_min_sq = a.r_min * a.r_min;
-    void* tmp = nullptr;
-    if (int rc = fa::scratch(21, sizeof(uint32_t) * (size_t(n_query) * C + 64), &tmp))
-        return rc;
-    uint32_t* const over = static_cast<uint32_t*>(tmp);
-    uint32_t* const rows = over + 64;
-    if (int rc = fa::zero_u32(over, 1))
-        return rc;
-    auto walk = [&](auto kern) {
-        FA_PROF_BEGIN("ball_wave_kernel");
-        hipLaunchKernelGGL(kern, dim3((n_query + kWaves - 1) / kWaves), dim3(kBlock), 0, s, db, g, qpts, n_query,
-                           r_max_sq, r_min_sq, a.exclude_ii, 1, C, out->counts, rows, over);
-        FA_PROF_END();
-    };
-    if (self)
-        by_distance ? walk(ball_wave_kernel<true, true>) : walk(ball_wave_kernel<false, true>);
-    else
-        by_distance ? walk(ball_wave_kernel<true, false>) : walk(ball_wave_kernel<false, false>);
-    FA_HIP(hipGetLastError());
-    uint64_t total = 0;
-    uint32_t h_over = 0;
-    if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total, over, &h_over, 1, out->segments))
-        return rc;
-    if (h_over)
-        return FA_OK;
-    if (int rc = fa::nlist_reserve(out, total, n_query))
-        return rc;
-    out->num_bonds = total;
-    FA_KLAUNCH(wave_emit_kernel<AABB_FORMULA>, dim3((n_query * 16u + kBlock - 1) / kBlock), dim3(kBlock), 0, s, db, qpts,
-               n_query, nq->d_points, rows, C, out->offsets, out->neighbors, out->distances, out->weights, out->vectors);
-    FA_HIP(hipGetLastError());
-    *handled = true;
-    return FA_OK;
-}
-
 int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args& a, int by_distance, fa_nlist* out)
 {
     hipStream_t s = fa::stream();
@@ -2187,25 +2144,18 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
     unsigned const blocks = (n_query + kBlock - 1) / kBlock;
     // query points == the grid's points: the walk takes them in cell order
     bool const self = (qpts == nq->d_points) && (n_query == nq->n);
-    if (nq->kind == FA_NQ_AABB && n_query && n_query <= kWaveQueries)
-    {
-        // small systems: one wave per query point, unless bonds are many
-        uint32_t const Cw = ball_wave_slots(nq, a.r_max);
-        bool handled = false;
-        if (Cw)
-            if (int rc = run_ball_wave(nq, qpts, n_query, a, by_distance, self, Cw, out, &handled))
-                return rc;
-        if (handled)
-            return FA_OK;
-    }
+    // small systems: one wave per query point, unless bonds are many
+    uint32_t const Cw = nq->kind == FA_NQ_AABB && n_query <= kWaveQueries ? ball_wave_slots(nq, a.r_max) : 0u;
+    bool const wave = Cw != 0;
     fa::CQGrid const cq = nq->kind == FA_NQ_CELLQUERY ? fa::cq_grid_for(nq->box, a.r_max) : fa::CQGrid{};
-    uint32_t const C = ball_row_slots(nq, a.r_max);
+    uint32_t const C = wave ? Cw : ball_row_slots(nq, a.r_max);
     bool const dense = !C && !by_distance && ball_row_slots(nq, a.r_max, kDenseSlots) != 0;
     uint32_t* rows = nullptr;
     uint32_t* pos = nullptr;
+    uint32_t* over = nullptr; // device mark of the wave walk: a point without a row
     if (n_query)
     {
-        // each block owns kBlock * C slots; positions are 32-bit
+        // each block owns kBlock * C slots (each point C in the wave walk); positions are 32-bit
         size_t const slots = size_t(blocks) * kBlock * C;
         if (slots >= (size_t(1) << 32))
             return fa::fail(FA_ERR_RUNTIME, "ball query: too many query points for the key staging");
@@ -2214,6 +2164,7 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
             return rc;
         rows = static_cast<uint32_t*>(tmp);
         pos = rows + slots;
+        over = pos + n_query;
     }
     size_t const walk_lds = sizeof(uint32_t) * size_t(kBlock) * C;
     auto walk = [&](auto kern) {
@@ -2222,8 +2173,23 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
                            a.exclude_ii, R, cq, C, out->counts, pos, rows);
         FA_PROF_END();
     };
+    auto wave_walk = [&](auto kern) {
+        FA_PROF_BEGIN("ball_wave_kernel");
+        hipLaunchKernelGGL(kern, dim3((n_query + kWaves - 1) / kWaves), dim3(kBlock), 0, s, db, g, qpts, n_query,
+                           r_max_sq, r_min_sq, a.exclude_ii, R, C, out->counts, pos, rows, over);
+        FA_PROF_END();
+    };
     if (n_query == 0)
         ;
+    else if (wave)
+    {
+        if (int rc = fa::zero_u32(over, 1))
+            return rc;
+        if (self)
+            by_distance ? wave_walk(ball_wave_kernel<true, true>) : wave_walk(ball_wave_kernel<false, true>);
+        else
+            by_distance ? wave_walk(ball_wave_kernel<true, false>) : wave_walk(ball_wave_kernel<false, false>);
+    }
     else if (nq->kind == FA_NQ_AABB)
         self ? walk(ball_walk_kernel<AABB_FORMULA, true>) : walk(ball_walk_kernel<AABB_FORMULA, false>);
     else if (nq->kind == FA_NQ_CELLQUERY)
@@ -2232,14 +2198,22 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
         self ? walk(ball_walk_kernel<LINKCELL_FORMULA, true>) : walk(ball_walk_kernel<LINKCELL_FORMULA, false>);
     FA_HIP(hipGetLastError());
     uint64_t total = 0;
-    if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total, nullptr, nullptr, 1,
-                                        out->segments))
+    uint32_t h_over = 0;
+    if (int rc = fa::exclusive_scan_u32(out->counts, out->offsets, n_query, &total, wave && n_query ? over : nullptr,
+                                        &h_over, 1, out->segments))
         return rc;
     if (total > 0xffffffffull)
         return fa::fail(FA_ERR_RUNTIME, "NeighborList would exceed 2^32 bonds");
     if (int rc = fa::nlist_reserve(out, total, n_query))
         return rc;
     out->num_bonds = total;
+    if (wave && n_query && !h_over)
+    {
+        FA_KLAUNCH(wave_emit_kernel, dim3((n_query * 16u + kBlock - 1) / kBlock), dim3(kBlock), 0, s, db, qpts, n_query,
+                   nq->d_points, rows, C, out->offsets, out->neighbors, out->distances, out->weights, out->vectors);
+        FA_HIP(hipGetLastError());
+        return FA_OK;
+    }
     void* gkeys = nullptr;
     if (int rc = fa::scratch(3, std::max<uint64_t>(total, 1) * (by_distance ? 8 : 4), &gkeys))
         return rc;

@@ -299,16 +299,25 @@ def test_nearest_query_at_the_stencil_radius(oracle):
     _assert_same(freud_amd.AABBQuery(box, pts).query(q, args).toNeighborList(), ref)
 
 
-def test_wave_ball_query_falls_back_on_clumps(oracle):
-    """A clump with more bonds per point than a wave keeps: the per-thread
-    query takes the call."""
+@pytest.mark.parametrize("by_distance", [False, True])
+def test_wave_ball_query_of_clumps(oracle, by_distance):
+    """A clump with more bonds per point than a wave keeps: the general emission
+    takes over from the wave's walk, which is not done twice."""
     box = Box.cube(20.0)
     rng = np.random.default_rng(8)
     pts = ((rng.random((1500, 3)) - 0.5) * 20).astype(np.float32)
     pts[:600] = (rng.standard_normal((600, 3)) * 0.3).astype(np.float32)
-    for args in (dict(r_max=1.5, exclude_ii=True), dict(num_neighbors=12, exclude_ii=True)):
-        ref = oracle.query(_bt(box), pts, pts, args, nthreads=4)
-        _assert_same(freud_amd.AABBQuery(box, pts).query(pts, args).toNeighborList(), ref)
+    nq = freud_amd.AABBQuery(box, pts)
+    for points in (pts, pts[300:900]):
+        for args in (dict(r_max=1.5, exclude_ii=True), dict(num_neighbors=12, exclude_ii=True)):
+            ref = oracle.query(_bt(box), pts, points, args, sort_by_distance=by_distance, nthreads=4)
+            _lib.profile_reset()
+            _lib.profile_enable()
+            nl = nq.query(points, args).toNeighborList(sort_by_distance=by_distance)
+            ran = _lib.profile_stats()
+            _lib.profile_enable(False)
+            _assert_same(nl, ref)
+            assert "ball_walk_kernel" not in ran
 
 
 @pytest.mark.parametrize("kind", ["aabb", "linkcell", "cellquery"])
