@@ -2433,7 +2433,9 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
         }
         int rc = FA_OK;
         int const key = fa::tune_key(dens, rk) * 128 + int(std::min<uint32_t>(k, 127u));
-        if (k <= kWaveKeys / 4 && n_query <= kWaveKnnQueries)
+        // a caller's preset names a per-thread search, and is kept
+        bool const preset = fa::variant_preset(reuse >= 0 ? fa::TUNE_KNN_REUSE : fa::TUNE_KNN, key);
+        if (k <= kWaveKeys / 4 && n_query <= kWaveKnnQueries && !preset)
         {
             // small systems: one wave per query point, cells as wide as the
             // radius that holds k + 5 sqrt(k) + 8 points, so that one stencil

@@ -256,6 +256,35 @@ def test_knn_staged_paths(oracle, is2D):
                         _assert_nlist_equal(nl, refs[by_d])
 
 
+@pytest.mark.parametrize("variant,mode,kernel", [(0, 0, "knn_aabb_kernel"), (5, 1, "knn_stage_kernel")])
+def test_knn_presets_of_small_systems(variant, mode, kernel):
+    """A preset search runs on systems small enough for the wave-per-query
+    search too, on a fresh grid and on one that a ball query built; without one
+    the wave search runs."""
+    from freud_amd import _lib
+
+    box = Box.cube(12)
+    pts = ((np.random.default_rng(2).random((1500, 3)) - 0.5) * 12).astype(np.float32)
+    qa = dict(num_neighbors=8, exclude_ii=True)
+
+    def ran(first=None):
+        nq = freud_amd.AABBQuery(box, pts)
+        if first:
+            nq.query(pts, first).toNeighborList()
+        _lib.profile_reset()
+        _lib.profile_enable()
+        nq.query(pts, qa).toNeighborList()
+        _lib.profile_enable(False)
+        return set(_lib.profile_stats())
+
+    rk = np.cbrt(3.0 * 2.0 * 8 / (4.0 * np.pi * len(pts) / box.volume))
+    for first in (None, dict(r_max=float(rk), exclude_ii=True)):
+        with _ForcedKnn(box, len(pts), 8, variant, mode):
+            names = ran(first)
+        assert kernel in names and "knn_wave_kernel" not in names
+        assert "knn_wave_kernel" in ran(first)
+
+
 def test_knn_staged_revised_on_hand_backs(oracle):
     """Points irregular enough that the staged kNN search hands many queries
     back to the ring search (sparse points beside dense clumps): whatever the
