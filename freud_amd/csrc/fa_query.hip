@@ -1055,28 +1055,46 @@ constexpr uint32_t kWaveKeys = 256; // keys a wave keeps (2 KB of LDS)
 constexpr uint32_t kWaves = kBlock / 64;
 
 // Calls f(valid, j, code, r_sq) with all lanes for 64 candidates at a time of
-// the stencil of half-width R around q (AABB formula), as for_each_candidate
-// visits them; lanes without a candidate get valid = false.
+// the stencil of half-width R around q (AABB formula; ring_only: its cells at
+// Chebyshev offset R, R > 0), as for_each_candidate visits them; lanes without
+// a candidate get valid = false.
 template<typename F>
-__device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float qx, float qy, float qz, int R, F&& f)
+__device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float qx, float qy, float qz, int R,
+                                       bool ring_only, F&& f)
 {
     int c[3], w[3];
     fa::cell_of(b, g.dim, qx, qy, qz, c, w);
     float const qzz = b.is2D ? 0.0f : qz;
     int const side = 2 * R + 1, Rz = b.is2D ? 0 : R;
-    int const ncell = side * side * (2 * Rz + 1);
+    // a ring: its two faces along z, then the rims of the layers between them
+    int const faces = b.is2D ? 0 : 2 * side * side, rim = 8 * R;
+    int const ncell = ring_only ? faces + rim * (b.is2D ? 1 : 2 * R - 1) : side * side * (2 * Rz + 1);
     bool const outside = *g.outside;
     uint32_t const lane = threadIdx.x & 63u;
     for (int c0 = 0; c0 < ncell; c0 += 64)
     {
         uint32_t beg = 0u, len = 0u;
-        // the cell's shift in box lengths per axis, 4 bits each (biased by 8: R is
-        // at most 3); the query's own image offset, of any size, is added below
+        // the cell's shift in box lengths per axis, 10 bits each (biased by 512:
+        // searches end near half a box length, so that it is a few at most); the
+        // query's own image offset, of any size, is added below
         int shift = 0;
         int const t = c0 + int(lane);
         if (t < ncell)
         {
-            int const d[3] = {t % side - R, (t / side) % side - R, t / (side * side) - Rz};
+            int d[3] = {t % side - R, (t / side) % side - R, t / (side * side) - Rz};
+            if (ring_only)
+            {
+                if (t < faces)
+                    d[2] = t < side * side ? -R : R;
+                else
+                {
+                    int const layer = (t - faces) / rim, e = (t - faces) % rim, o = e % (2 * R);
+                    int const edge = e / (2 * R);
+                    d[0] = edge == 0 ? o - R : edge == 2 ? R - o : edge == 1 ? R : -R;
+                    d[1] = edge == 1 ? o - R : edge == 3 ? R - o : edge == 2 ? R : -R;
+                    d[2] = b.is2D ? 0 : layer - (R - 1);
+                }
+            }
             int cell[3], sh[3];
             bool in = true;
 #pragma unroll
@@ -1092,7 +1110,7 @@ __device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float 
                 uint32_t const id = uint32_t((cell[2] * g.dim[1] + cell[1]) * g.dim[0] + cell[0]);
                 beg = g.cstart[id];
                 len = g.cstart[id + 1] - beg;
-                shift = (sh[0] + 8) | ((sh[1] + 8) << 4) | ((sh[2] + 8) << 8);
+                shift = (sh[0] + 512) | ((sh[1] + 512) << 10) | ((sh[2] + 512) << 20);
             }
         }
         uint32_t e = len; // inclusive scan over the lanes
@@ -1126,7 +1144,8 @@ __device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float 
             }
             bool valid = v < tot;
             float4 const pj = g.cpos[valid ? pos : 0u];
-            int n0 = 8 - (code3 & 15) - w[0], n1 = 8 - ((code3 >> 4) & 15) - w[1], n2 = 8 - ((code3 >> 8) & 15) - w[2];
+            int n0 = 512 - (code3 & 1023) - w[0], n1 = 512 - ((code3 >> 10) & 1023) - w[1];
+            int n2 = 512 - ((code3 >> 20) & 1023) - w[2];
             if (outside)
             {
                 int wj[3];
@@ -1176,6 +1195,55 @@ template<typename F> __device__ inline void wave_rank(const uint64_t* keys, uint
     __builtin_amdgcn_wave_barrier();
 }
 
+// Reduces the wave's n distinct keys (k <= n <= kWaveKeys) to the k smallest, in
+// order, and returns the largest of them.
+__device__ inline uint64_t wave_smallest(uint64_t* keys, uint32_t n, uint32_t k)
+{
+    constexpr uint32_t kOwn = kWaveKeys / 64;
+    uint32_t const lane = threadIdx.x & 63u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint64_t own[kOwn];
+    uint32_t rank[kOwn];
+#pragma unroll
+    for (uint32_t u = 0; u < kOwn; ++u)
+    {
+        own[u] = lane + 64u * u < n ? keys[lane + 64u * u] : ~0ull;
+        rank[u] = 0;
+    }
+    for (uint32_t m = 0; m < n; ++m)
+    {
+        uint64_t const key = keys[m];
+#pragma unroll
+        for (uint32_t u = 0; u < kOwn; ++u)
+            rank[u] += key < own[u] ? 1u : 0u;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // every key has been read
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (uint32_t u = 0; u < kOwn; ++u)
+        if (lane + 64u * u < n && rank[u] < k)
+            keys[rank[u]] = own[u];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return keys[k - 1u];
+}
+
+// How many of the wave's n keys hold a distance below `bound`.
+__device__ inline uint32_t wave_count_below(const uint64_t* keys, uint32_t n, float bound)
+{
+    uint32_t const lane = threadIdx.x & 63u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t c = 0;
+    for (uint32_t t0 = 0; t0 < n; t0 += 64u)
+    {
+        bool const below = t0 + lane < n && knn_key_distance(keys[t0 + lane]) < bound;
+        c += uint32_t(__builtin_popcountll(__builtin_amdgcn_ballot_w64(below)));
+    }
+    return c;
+}
+
 // Ball query, one wave per query position: the point's keys (j << 5 | image
 // code) in NeighborList order into rows[pos[i] ..], its bond count, and a mark
 // when some point has more than C bonds (no row: the general emission, which
@@ -1196,7 +1264,7 @@ __global__ __launch_bounds__(kBlock) void ball_wave_kernel(DevBox b, DevGrid g, 
     uint32_t const i = query_at<SELF>(g, qpts, p, qx, qy, qz);
     uint64_t* const keys = s_keys[wave];
     uint32_t n = 0;
-    wave_candidates(b, g, qx, qy, qz, R, [&](bool valid, uint32_t j, int code, float r_sq) {
+    wave_candidates(b, g, qx, qy, qz, R, false, [&](bool valid, uint32_t j, int code, float r_sq) {
         bool const take = valid && r_sq < r_max_sq && r_sq >= r_min_sq && !(exclude_ii && j == i);
         uint64_t const jc = (uint64_t(j) << 5) | uint32_t(code);
         wave_append(keys, n, take, BYDIST ? (uint64_t(float_order_bits(sqrtf(r_sq))) << 32) | jc : jc);
@@ -1231,20 +1299,24 @@ __global__ __launch_bounds__(kBlock) void wave_emit_kernel(DevBox b, const float
                                            uint64_t(e0) + m, nb_out, d_out, w_out, v_out);
 }
 
-// kNN, one wave per query position (see the ring search for what is selected):
-// the stencil of half-width 1, then 2, .., is searched until k distances lie
-// inside the radius it covers, or it covers rlim.  Positions whose stencils hold more
-// than the wave's keys, or need more than three, are handed back to the ring
-// search, and answers reaching half the smallest plane distance are flagged for
-// the exhaustive one, as there.
+// kNN, one wave per query position (see the ring search for what is selected,
+// where the search ends and what is flagged for the exhaustive kernel).  The
+// stencil of half-width 1 usually holds the answer, and only its candidates
+// inside the radius it covers are kept.  Where it does not, the search starts
+// over with every candidate and goes on ring by ring.  When the wave's keys
+// run out they are reduced to the k smallest, so that clumps and voids of
+// irregular systems stay here: a droplet's wave walks 64 of its many
+// candidates at a time, and a ring's empty cells are 64 loads in flight.
+// (Handing such points to the ring search, one thread each, took 2 to 7 times
+// as long as that search over its own cells.)
 template<bool SELF>
 __global__ __launch_bounds__(kBlock) void knn_wave_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
                                                           uint32_t nq, uint32_t k, float rlim_sq, float rlim,
                                                           float rmin_thr, int exclude_ii, float wmin,
-                                                          float half_min_plane, uint32_t* __restrict__ counts,
-                                                          uint64_t* __restrict__ sel, uint32_t* __restrict__ flagged,
-                                                          uint32_t* __restrict__ nflag, uint32_t* __restrict__ refine,
-                                                          uint32_t* __restrict__ nrefine, uint32_t* __restrict__ pos)
+                                                          float half_min_plane, int rmax_ring,
+                                                          uint32_t* __restrict__ counts, uint64_t* __restrict__ sel,
+                                                          uint32_t* __restrict__ flagged,
+                                                          uint32_t* __restrict__ nflag, uint32_t* __restrict__ pos)
 {
     __shared__ uint64_t s_keys[kWaves][kWaveKeys];
     uint32_t const wave = threadIdx.x >> 6;
@@ -1258,40 +1330,61 @@ __global__ __launch_bounds__(kBlock) void knn_wave_kernel(DevBox b, DevGrid g, c
         pos[i] = p;
     uint64_t* const keys = s_keys[wave];
     uint32_t n = 0;
-    bool done = false;
-    for (int R = 1; R <= 3 && !done; ++R)
-    {
-        float const complete = float(R) * wmin * (1.0f - 1e-4f);
-        bool const whole = complete >= rlim; // the stencil covers every candidate, d = rlim included
-        n = 0; // keys with d < complete
-        wave_candidates(b, g, qx, qy, qz, R, [&](bool valid, uint32_t j, int code, float r_sq) {
-            bool take = valid && r_sq < rlim_sq && r_sq >= rmin_thr && !(exclude_ii && j == i);
+    uint64_t cut = ~0ull; // keys from it on cannot enter the selection
+    // the keys are reduced when they pass this: early, as it tightens `cut`
+    uint32_t const full = k <= 32u ? kWaveKeys / 2 : kWaveKeys;
+    auto walk = [&](int R, bool ring_only, float below) {
+        // as knn_rsq_cut: no candidate with a root below `d` is beyond it
+        auto r_sq_cut = [&](float d) { return d * d * (1.0f + 0x1p-20f) + 1e-37f; };
+        float most = r_sq_cut(below);
+        if (cut != ~0ull)
+            most = fminf(most, r_sq_cut(knn_key_distance(cut)));
+        wave_candidates(b, g, qx, qy, qz, R, ring_only, [&](bool valid, uint32_t j, int code, float r_sq) {
+            bool take = valid && r_sq < rlim_sq && r_sq >= rmin_thr && r_sq <= most && !(exclude_ii && j == i);
+            if (!__builtin_amdgcn_ballot_w64(take))
+                return;
             uint64_t const key = knn_key(r_sq, (j << 5) | uint32_t(code));
-            take = take && (whole || knn_key_distance(key) < complete);
+            take = take && key < cut && knn_key_distance(key) < below;
+            if (n + uint32_t(__builtin_popcountll(__builtin_amdgcn_ballot_w64(take))) > full)
+            {
+                cut = wave_smallest(keys, n, k); // n > full - 64 >= k
+                n = k;
+                most = fminf(most, r_sq_cut(knn_key_distance(cut)));
+                take = take && key < cut;
+            }
             wave_append(keys, n, take, key);
         });
-        if (n > kWaveKeys)
-            break;
-        done = n >= k || whole; // inside `complete` nothing is missing
-        if (!done && complete >= half_min_plane && rlim > half_min_plane)
-            break; // longer searches, and the exhaustive flag, are the ring search's
-    }
+    };
+    auto covered = [&](int R) { return float(R) * wmin * (1.0f - 1e-4f); };
+    int R = 1;
+    float complete = covered(R); // the radius that the stencil covers
+    // at rlim and beyond it holds every candidate, those of d = rlim included
+    walk(R, false, complete >= rlim ? INFINITY : complete);
+    bool done = n >= k || complete >= rlim, extended = false;
     if (!done)
+        n = 0; // (fewer than k: never reduced, `cut` is unset)
+    while (!done)
     {
-        if (lead)
-            refine[atomicAdd(nrefine, 1u)] = p;
-        return;
+        extended = complete >= half_min_plane && rlim > half_min_plane;
+        if (extended || R >= rmax_ring)
+            break;
+        ++R;
+        walk(R, R > 2, INFINITY);
+        complete = covered(R);
+        done = wave_count_below(keys, n, complete) >= k || complete >= rlim;
     }
-    uint32_t const kept = min(n, k);
+    uint32_t const kept = extended ? 0u : min(n, k);
     float last = 0.0f;
-    wave_rank(keys, n, [&](uint32_t rank, uint64_t key) {
-        if (rank < kept)
-            sel[uint64_t(p) * k + rank] = key;
-        if (rank + 1u == kept)
-            last = knn_key_distance(key);
-    });
+    if (kept)
+        wave_rank(keys, n, [&](uint32_t rank, uint64_t key) {
+            if (rank < kept)
+                sel[uint64_t(p) * k + rank] = key;
+            if (rank + 1u == kept)
+                last = knn_key_distance(key);
+        });
     // two images of one point are at least a plane distance apart (see the ring search)
-    bool const flag = __builtin_amdgcn_ballot_w64(rlim > half_min_plane && last >= half_min_plane) != 0;
+    bool const flag =
+        extended || __builtin_amdgcn_ballot_w64(rlim > half_min_plane && last >= half_min_plane) != 0;
     if (lead)
     {
         if (flag)
@@ -2051,39 +2144,18 @@ int launch_knn_aabb(const fa::DevBox& db, const DevGrid& g, const float* qpts, u
     return FA_OK;
 }
 
-// The wave-per-query search, then the ring search over what it hands back.
 int launch_knn_wave(const fa::DevBox& db, const DevGrid& g, const float* qpts, uint32_t nq, uint32_t k, float rlim,
                     float r_min, int exclude_ii, float wmin, float hmp, int rmax_ring, uint32_t* counts, uint64_t* sel,
-                    uint32_t* flagged, uint32_t* nflag, uint32_t* refine, uint32_t* nrefine, const float* self_points,
-                    uint32_t self_n, uint32_t* pos)
+                    uint32_t* flagged, uint32_t* nflag, const float* self_points, uint32_t self_n, uint32_t* pos)
 {
     bool const self = (qpts == self_points) && (nq == self_n);
-    float const rlim_sq = rlim * rlim, rmin_thr = sqrt_threshold(r_min);
     FA_PROF_BEGIN("knn_wave_kernel");
     auto search = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((nq + kWaves - 1) / kWaves), dim3(kBlock), 0, fa::stream(), db, g, qpts, nq, k,
-                           rlim_sq, rlim, rmin_thr, exclude_ii, wmin, hmp, counts, sel, flagged, nflag, refine, nrefine,
-                           pos);
+                           rlim * rlim, rlim, sqrt_threshold(r_min), exclude_ii, wmin, hmp, rmax_ring, counts, sel,
+                           flagged, nflag, pos);
     };
     self ? search(knn_wave_kernel<true>) : search(knn_wave_kernel<false>);
-    FA_PROF_END();
-    FA_HIP(hipGetLastError());
-    FA_PROF_BEGIN("knn_refine_kernel");
-    auto rest = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3((nq + kBlock - 1) / kBlock), dim3(kBlock), 0, fa::stream(), db, g, qpts, nq, k,
-                           rlim_sq, rlim, rmin_thr, exclude_ii, wmin, hmp, rmax_ring, counts, sel, flagged, nflag, pos,
-                           refine, nrefine);
-    };
-#define FA_KNN_REST(KM) (self ? rest(knn_aabb_kernel<KM, true, true>) : rest(knn_aabb_kernel<KM, false, true>))
-    if (k <= 8)
-        FA_KNN_REST(8);
-    else if (k <= 16)
-        FA_KNN_REST(16);
-    else if (k <= 32)
-        FA_KNN_REST(32);
-    else
-        FA_KNN_REST(64);
-#undef FA_KNN_REST
     FA_PROF_END();
     FA_HIP(hipGetLastError());
     return FA_OK;
@@ -2454,8 +2526,7 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
                 wmin = std::min(wmin, npd[d] / float(dims[d]));
             int const rmax_ring = std::max(dims[0], std::max(dims[1], dims[2])) * 2 + 2;
             rc = launch_knn_wave(*dbp, nq->cur->dev(), qpts, n_query, k, rlim, a.r_min, a.exclude_ii, wmin,
-                                 min_pd / 2.0f, rmax_ring, out->counts, sel, flagged, nflag, refine, nrefine,
-                                 nq->d_points, nq->n, pos);
+                                 min_pd / 2.0f, rmax_ring, out->counts, sel, flagged, nflag, nq->d_points, nq->n, pos);
         }
         else if (k <= 64 && reuse >= 0)
         {

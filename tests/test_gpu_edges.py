@@ -299,6 +299,50 @@ def test_nearest_query_at_the_stencil_radius(oracle):
     _assert_same(freud_amd.AABBQuery(box, pts).query(q, args).toNeighborList(), ref)
 
 
+def _irregular(kind, n, is2D, rng):
+    """(box, points): a droplet in a large box, two dense clumps and a vapour, or
+    a slab in an elongated box."""
+    dim = 2 if is2D else 3
+    make = Box.square if is2D else Box.cube
+    if kind == "droplet":
+        box, pts = make(30.0), rng.standard_normal((n, dim)) * 1.7
+    elif kind == "clumps":
+        box, pts = make(24.0), (rng.random((n, dim)) - 0.5) * 24
+        pts[: n // 2] = rng.standard_normal((n // 2, dim)) * 0.4
+        pts[n // 3: n // 2] += 8
+    else:
+        box, pts = (Box(9.0, 60.0) if is2D else Box(9.0, 8.0, 60.0)), (rng.random((n, dim)) - 0.5) * 8
+    if is2D:
+        pts = np.concatenate([pts, np.zeros((n, 1))], 1)
+    return box, np.ascontiguousarray(box.wrap(pts.astype(np.float32)), np.float32)
+
+
+@pytest.mark.parametrize("is2D", [False, True])
+@pytest.mark.parametrize("kind", ["droplet", "clumps", "slab"])
+@pytest.mark.parametrize("n", [40, 900, 6000])
+def test_wave_nearest_of_irregular_systems(oracle, kind, n, is2D):
+    """Stencils with many times the wave's keys, and query points so far from
+    every point that the search takes rings upon rings: all in the one kernel."""
+    rng = np.random.default_rng(n + is2D)
+    box, pts = _irregular(kind, n, is2D, rng)
+    q = ((rng.random((500, 3)) - 0.5) * np.array([box.Lx, box.Ly, box.Lz])).astype(np.float32)
+    if is2D:
+        q[:, 2] = 0
+    moved = pts.copy()
+    moved[::5, 1] += np.float32(3 * box.Ly)
+    nq, out = freud_amd.AABBQuery(box, pts), freud_amd.AABBQuery(box, moved)
+    for args in (dict(num_neighbors=6, exclude_ii=True), dict(num_neighbors=17, r_max=3.9),
+                 dict(num_neighbors=64, exclude_ii=True), dict(num_neighbors=9, r_min=0.3), dict(num_neighbors=1)):
+        for obj, stored, points in ((nq, pts, pts), (nq, pts, q), (out, moved, moved)):
+            ref = oracle.query(_bt(box), stored, points, args, nthreads=16)
+            _lib.profile_reset()
+            _lib.profile_enable()
+            nl = obj.query(points, args).toNeighborList()
+            _lib.profile_enable(False)
+            _assert_same(nl, ref)
+            assert "knn_wave_kernel" in _lib.profile_stats() and "knn_refine_kernel" not in _lib.profile_stats()
+
+
 @pytest.mark.parametrize("by_distance", [False, True])
 def test_wave_ball_query_of_clumps(oracle, by_distance):
     """A clump with more bonds per point than a wave keeps: the general emission
