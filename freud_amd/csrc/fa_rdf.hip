@@ -1462,6 +1462,27 @@ __global__ __launch_bounds__(kBlock) void rdf_query_kernel(DevBox b, DevGrid g, 
     hist_epilogue<LDS_HIST>(hist, nbins, counts);
 }
 
+// Few distinct query points (AABB formula): one wave per query point, 64
+// candidates of its stencil at a time (see cross_route).  Bound by launches and the walk's dependent loads.
+__global__ __launch_bounds__(kBlock) void rdf_wave_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
+                                                          uint32_t nq, int R, float lo, float hi,
+                                                          const float* __restrict__ T, uint32_t nbins, float vmin,
+                                                          float inv_width, uint32_t* __restrict__ counts)
+{
+    extern __shared__ uint32_t hist_only[];
+    for (uint32_t t = threadIdx.x; t < nbins; t += blockDim.x)
+        hist_only[t] = 0u;
+    __syncthreads();
+    constexpr uint32_t kWaves = kBlock / 64;
+    for (uint32_t i = blockIdx.x * kWaves + (threadIdx.x >> 6); i < nq; i += gridDim.x * kWaves)
+        fa::wave_candidates(b, g, qpts[3 * i], qpts[3 * i + 1], qpts[3 * i + 2], R, false,
+                            [&](bool valid, uint32_t, int, float r_sq) {
+                                if (valid && r_sq >= lo && r_sq < hi)
+                                    atomicAdd(&hist_only[bin_in_range(r_sq, T, nbins, vmin, inv_width)], 1u);
+                            });
+    hist_epilogue<true>(hist_only, nbins, counts);
+}
+
 // freud/util/Histogram.h:152-174 RegularAxis::bin on a distance; nbins for overflow
 __device__ inline uint32_t regular_bin(float value, float vmin, float vmax, float inv_width, uint32_t nbins)
 {
@@ -1722,12 +1743,45 @@ int run_rows(const RowsArgs& a, RowVariant rv, uint32_t* d_counts, bool* handled
                        a.T, a.bins, a.r_min, a.inv_width, d_counts);
 }
 
+// The kernel for n_query distinct query points (AABB formula) by the candidates
+// that their 27-cell stencils hold on average.  Times in ms, uniform points of
+// density 1; each route does best where the rule takes it, or within a tenth.
+enum class CrossRoute
+{
+    rows,   // a grid of the query points, then the row clusters (run_cross_rows)
+    waves,  // one wave per query point (rdf_wave_kernel)
+    threads // one thread per query point (rdf_query_kernel)
+};
+CrossRoute cross_route(const fa_nq* nq, uint32_t n_query, float q_r_max)
+{
+    double const dens = double(nq->n) / std::max(double(fa::box_volume(nq->box)), 1e-30), r = double(q_r_max);
+    double const stencil = nq->box.is2D ? 9.0 * dens * r * r : 27.0 * dens * r * r * r;
+    // Short ranges: the second grid costs more than the pairs.  A wave has 1 us
+    // in 1,000 query points and a little per candidate, a thread a serial walk
+    // that many query points share: 65,536 points, r_max = 1.2 (47 candidates),
+    // 8,192 query points: waves 0.050, threads 0.065, rows 0.148; 60,000: 0.100,
+    // 0.067, 0.121; 1,000,000: 1.351, 0.331, 0.415.
+    if (stencil <= 160.0)
+        return n_query * (1.0 + 0.004 * stencil) <= 5000.0 + 600.0 * stencil ? CrossRoute::waves : CrossRoute::threads;
+    // Few query points: their walks against that grid's cells, which have to be
+    // cleared, scanned and clustered whatever it holds.  1,048,576 points, r_max = 2
+    // (216 candidates): 64 query points: waves 0.020, rows 0.110, threads 0.134;
+    // 60,000: 0.150, 0.257, 0.193; 200,000: 0.425, 0.317, 0.340.  A stencil of
+    // thousands makes a long walk for one wave (r_max = 4.9, 64: 0.045 against
+    // rows 0.064; clumped points 0.827 against 0.103).
+    int dims[3], F = 1;
+    rows_grid_dims(nq->box, nq->n, q_r_max, RowVariant{2, 8}, dims, &F);
+    double const cells = double(dims[0]) * dims[1] * dims[2];
+    return stencil <= 400.0 && stencil * n_query <= std::max(2.0 * cells, 1048576.0) ? CrossRoute::waves
+                                                                                      : CrossRoute::rows;
+}
+
 // RDF of distinct query points (AABB formula, no index exclusion): the query
 // points get a grid of the points' shape and are taken as row clusters of it,
-// against the points' rows.  One cell shape, (R, F) = (2, 8), the one the tuner
-// picks for self RDFs at 10 to 500 neighbours.  The thread-per-query kernel
-// below walks its candidates one by one, each a scattered load and an LDS
-// atomic of its own: 65,000 points and 35,000 query points, r_max = 5:
+// against the points' rows (see cross_route for the calls this takes).  One cell
+// shape, (R, F) = (2, 8), the one the tuner picks for self RDFs at 10 to 500
+// neighbours.  The thread-per-query kernel above walks its candidates one by
+// one, each a scattered load and an LDS atomic of its own: 65,000 points and 35,000 query points, r_max = 5:
 // 1.29 -> 0.06 ms.
 int run_cross_rows(fa_nq* nq, const float* d_query, uint32_t n_query, float q_r_max, float qmax_sq, float qmin_sq,
                    const EstRange& est, const float* T, uint32_t bins, float r_min, float inv_width,
@@ -2283,7 +2337,9 @@ int fa_rdf_accumulate_query(fa_nq* nq, const float* d_query_points, uint32_t n_q
             return FA_OK;
         }
     }
-    if (!self && nq->kind == FA_NQ_AABB && !exclude_ii && est.hi > 0.0f)
+    bool const cross = !self && nq->kind == FA_NQ_AABB && !exclude_ii && est.hi > 0.0f;
+    CrossRoute const route = cross ? cross_route(nq, n_query, q_r_max) : CrossRoute::threads;
+    if (route == CrossRoute::rows)
     {
         bool handled = false;
         if (int rc = run_cross_rows(nq, d_query_points, n_query, q_r_max, qmax_sq, qmin_sq, est, T, bins, r_min,
@@ -2321,6 +2377,10 @@ int fa_rdf_accumulate_query(fa_nq* nq, const float* d_query_points, uint32_t n_q
             FA_RDF_LAUNCH(rdf_self_kernel, LINKCELL_FORMULA, db, g, n_query, qmax_sq, qmin_sq, exclude_ii, R, T, bins,
                           r_min, inv_width, d_counts, cq);
     }
+    else if (route == CrossRoute::waves)
+        FA_KLAUNCH(rdf_wave_kernel, dim3(std::min<unsigned>((n_query + kBlock / 64 - 1) / (kBlock / 64), 2048u)),
+                   dim3(kBlock), sizeof(uint32_t) * bins, s, db, g, d_query_points, n_query, R, est.lo, est.hi, T,
+                   bins, r_min, inv_width, d_counts);
     else
     {
         if (nq->kind == FA_NQ_AABB)

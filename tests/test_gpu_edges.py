@@ -140,6 +140,59 @@ def test_rdf_estimate_borders(oracle, name, n, bins, r_max, r_min):
     npt.assert_array_equal(rdf.compute((box, pts), query_points=q).bin_counts, ref)
 
 
+def _rdf_kernels(run):
+    _lib.profile_reset()
+    _lib.profile_enable()
+    counts = run()
+    _lib.profile_enable(False)
+    return counts, set(_lib.profile_stats())
+
+
+@pytest.mark.parametrize("is2D", [False, True])
+@pytest.mark.parametrize("n,n_query,r_max,kernel", [
+    (30000, 1, 1.1, "rdf_wave_kernel"), (30000, 3001, 1.1, "rdf_wave_kernel"), (30000, 60001, 1.1, "rdf_query_kernel"),
+    (30000, 7, 2.0, "rdf_wave_kernel"), (30000, 2003, 2.0, "rdf_wave_kernel"), (900, 20001, 2.0, "rdf_est_kernel"),
+    (30000, 7, 3.5, "rdf_est_kernel"), (200001, 30001, 2.0, "rdf_est_kernel")])
+def test_rdf_routes_of_query_points(oracle, is2D, n, n_query, r_max, kernel):
+    """Each kernel that takes distinct query points, by the size of their
+    stencils and by their number: bin counts bit for bit, with points and query
+    points inside and outside the box, in a triclinic box too.  (2D boxes have
+    fewer cells and candidates per point: the kernel is not asserted.)"""
+    side = (n / 1.0) ** (1 / 3)
+    rng = np.random.default_rng(n_query)
+    for tilts in ((0.0, 0.0, 0.0), (0.2, -0.1, 0.15)):
+        box = Box.square(n ** 0.5) if is2D else Box(side, side, side, *tilts)
+        frac = rng.random((n + n_query, 3)).astype(np.float32)
+        both = np.ascontiguousarray(box.make_absolute(frac), np.float32)
+        if is2D:
+            both[:, 2] = 0
+        moved = both.copy()
+        moved[::3, 0] += np.float32(box.Lx)
+        for p, q in ((both, both), (moved, both), (both, moved), (moved, moved)):
+            pts, query = p[:n], q[n:]
+            ref = oracle.rdf_accumulate(_bt(box), pts, query, 60, r_max, r_min=0.2, exclude_ii=False, nthreads=16)
+            rdf = freud_amd.density.RDF(60, r_max, r_min=0.2)
+            counts, ran = _rdf_kernels(lambda: rdf.compute((box, pts), query_points=query).bin_counts)
+            npt.assert_array_equal(counts, ref)
+            if not is2D:
+                assert any(kernel in name for name in ran), ran
+
+
+@pytest.mark.parametrize("n_query", [8192, 16384, 16385, 32768, 32769, 65537, 196608, 200001])
+def test_rdf_row_clusters_of_query_points(oracle, n_query):
+    """Row clusters of distinct query points on both sides of the sizes at which
+    8, 4, 2 waves share a cluster and at which a wave takes two."""
+    n, r_max = 3000, 2.4
+    box = Box.cube(14.5)
+    both = ((np.random.default_rng(n_query).random((n + n_query, 3)) - 0.5) * 14.49).astype(np.float32)
+    pts, q = both[:n], both[n:]
+    ref = oracle.rdf_accumulate(_bt(box), pts, q, 80, r_max, exclude_ii=False, nthreads=16)
+    rdf = freud_amd.density.RDF(80, r_max)
+    counts, ran = _rdf_kernels(lambda: rdf.compute((box, pts), query_points=q).bin_counts)
+    npt.assert_array_equal(counts, ref)
+    assert any("rdf_est_kernel" in name for name in ran), ran
+
+
 @pytest.mark.parametrize("which", ["points", "query_points", "both"])
 def test_rdf_points_outside_the_box(oracle, which):
     """Systems with points (or query points) outside the box leave the
