@@ -28,32 +28,39 @@ using fa::DevGrid;
 using fa::LINKCELL_FORMULA;
 
 constexpr int kBlock = 256;
-constexpr int kKeyBytes = 32768; // largest LDS key staging per block
-// keys per point that the one-walk ball query stages in LDS (32 KB per block)
+// largest LDS key staging per block; of a ball query's emission, such that four
+// blocks fit on a CU with its other LDS
+constexpr int kKeyBytes = 32768, kBallKeyBytes = 32256;
 // query points up to which a ball query, and a kNN query (whose per-thread
 // search the tuner fits to larger systems), takes one wave per point
 constexpr uint32_t kWaveQueries = 32768;
 constexpr uint32_t kWaveKnnQueries = 8192;
+// keys per point that the one-walk ball query stages in LDS (32 KB per block)
 constexpr uint32_t kWalkMaxSlots = kKeyBytes / (kBlock * sizeof(uint32_t));
-// keys per point that the dense ball query sorts in registers
-constexpr uint32_t kDenseSlots = 48;
 extern __shared__ __align__(16) unsigned char fa_dyn_lds[];
 
-
 // Dynamic LDS bytes for a fill block's keys: 1.3 x the mean bonds of its query
-// points, between 4 KB and kKeyBytes.
+// points, between 4 KB and kBallKeyBytes.
 size_t fill_key_bytes(uint64_t bonds, uint64_t points, size_t key_size, uint32_t block_points = kBlock)
 {
     double const per = points ? double(bonds) / double(points) : 0.0;
     double const want = std::ceil(per * block_points * 1.3) * double(key_size);
-    size_t const b = size_t(std::min(std::max(want, 4096.0), double(kKeyBytes)));
+    size_t const b = size_t(std::min(std::max(want, 4096.0), double(kBallKeyBytes)));
     return (b + 15) & ~size_t(15);
 }
 
-// LDS of kb bytes of keys and one owner byte per key.
-size_t owner_lds(size_t kb, size_t key_size)
+// Key slots that share an owner byte: one each, but four for more than 20 KB of
+// keys, which leave room for three blocks per CU with a byte each and for four
+// without, if there are blocks enough to fill them.
+__host__ __device__ inline uint32_t owner_stride(size_t kb, uint32_t blocks)
 {
-    return kb + ((kb / key_size + 15) & ~size_t(15));
+    return kb > 20480 && blocks > 3u * 256u ? 4u : 1u;
+}
+
+// LDS of kb bytes of keys and their owner bytes.
+size_t owner_lds(size_t kb, size_t key_size, uint32_t blocks)
+{
+    return kb + ((kb / key_size / owner_stride(kb, blocks) + 1 + 15) & ~size_t(15));
 }
 
 __device__ inline uint32_t float_order_bits(float v)
@@ -137,10 +144,33 @@ template<typename K> __device__ inline void insertion_sort(K* a, uint32_t n)
     }
 }
 
-// Batcher's odd-even merge sort of N registers (K. E. Batcher, 1968): every
-// lane sorts its own keys without a branch or a memory access.  191
-// comparators for 32 keys; an insertion sort in LDS runs the longest lane's
-// ~400 dependent steps.
+// The owners (points lo of the block) of its key slots, a byte per stride of
+// them: one pass of short byte writes instead of a binary search over the
+// offsets per key and pass.
+struct KeyOwners
+{
+    uint8_t* own;
+    const uint32_t* s_off; // exclusive key offsets, nloc + 1 of them
+    uint32_t stride;
+    // every thread tid < nloc calls it with its own range
+    __device__ void mark(uint32_t beg, uint32_t cnt) const
+    {
+        for (uint32_t q = (beg + stride - 1u) / stride; stride * q < beg + cnt; ++q)
+            own[q] = uint8_t(threadIdx.x);
+    }
+    __device__ uint32_t of(uint32_t t) const
+    {
+        if (stride == 1u)
+            return own[t];
+        uint32_t lo = own[t / 4u];
+        while (s_off[lo + 1u] <= t)
+            ++lo;
+        return lo;
+    }
+};
+
+// Batcher's odd-even merge sort of N registers (K. E. Batcher, 1968): every lane sorts its own keys
+// without a branch or a memory access, 63 comparators for 16 keys, 191 for 32.
 template<int N> __device__ inline void register_sort(uint32_t (&v)[N])
 {
 #pragma unroll
@@ -167,6 +197,7 @@ template<int N> __device__ inline void register_sort(uint32_t (&v)[N])
     }
 }
 
+// Sorts the n <= N keys at `a` (LDS) of each of the caller's lanes.
 template<int N> __device__ inline void register_sort_keys(uint32_t* a, uint32_t n)
 {
     uint32_t v[N];
@@ -180,28 +211,112 @@ template<int N> __device__ inline void register_sort_keys(uint32_t* a, uint32_t 
             a[m] = v[m];
 }
 
-// Sorts the n keys at `a` (LDS) of each of the caller's lanes: 32-bit keys in
-// registers, as many as the wave's longest list needs (up to 32), others and
-// longer lists by insertion.
-template<typename K> __device__ inline void sort_keys(K* a, uint32_t n)
+// The same sort of n keys in LDS by one
+// wave, for lists longer than a wave.
+template<typename K> __device__ inline void wave_sort_long(K* a, uint32_t n)
 {
-    if constexpr (sizeof(K) == sizeof(uint32_t))
+    uint32_t const lane = threadIdx.x & 63u;
+    for (uint32_t p = 1; p < n; p *= 2)
+        for (uint32_t k = p; k >= 1; k /= 2)
+        {
+            uint32_t const r = k == p ? 0u : k;
+            for (uint32_t c = lane;; c += 64u)
+            {
+                uint32_t const x = r + 2u * k * (c / k) + c % k;
+                if (!__builtin_amdgcn_ballot_w64(x + k < n))
+                    break;
+                if (x + k < n && x / (2u * p) == (x + k) / (2u * p))
+                {
+                    K const u = a[x], v = a[x + k];
+                    a[x] = u < v ? u : v;
+                    a[x + k] = u < v ? v : u;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the next step reads other lanes' keys
+            __builtin_amdgcn_wave_barrier();
+        }
+}
+
+// Sorts each point's distinct keys (LDS) of a block of nloc points, a quarter
+// of the points by each wave.  Lists of up to NET keys are sorted in a lane's
+// registers, by the smallest network that holds the wave's longest one: the
+// networks' registers stay with the walk and the gathers of the same kernel, so
+// that kernels for short lists carry small networks only (NET = 0: none).
+// Other waves take whole lists for up to 64 keys at a time: a lane ranks its
+// key by reading its list (eight reads in flight, mostly of one address per
+// list), and writes it to its place once the wave has read.  Called by the
+// whole block, after a barrier.
+template<int NET, typename K>
+__device__ inline void block_sort_lists(K* keys, const KeyOwners& owners, uint32_t nloc)
+{
+    const uint32_t* const s_off = owners.s_off;
+    constexpr uint32_t kWaves = kBlock / 64;
+    uint32_t const lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t const share = (nloc + kWaves - 1u) / kWaves;
+    uint32_t const first = min(wave * share, nloc), last = min(first + share, nloc);
+    if constexpr (NET > 0)
     {
-        if (!__builtin_amdgcn_ballot_w64(n > 16u))
-            return register_sort_keys<16>(a, n);
-        if (!__builtin_amdgcn_ballot_w64(n > 32u))
-            return register_sort_keys<32>(a, n);
+        uint32_t const p = first + lane;
+        uint32_t const list = p < last ? s_off[p] : 0u, len = p < last ? s_off[p + 1u] - list : 0u;
+        auto fits = [&](uint32_t most) { return !__builtin_amdgcn_ballot_w64(len > most); };
+        if (fits(16u))
+            return register_sort_keys<16>(keys + list, len);
+        if constexpr (NET >= 32)
+            if (fits(32u))
+                return register_sort_keys<32>(keys + list, len);
+        if constexpr (NET >= 48)
+            if (fits(48u))
+                return register_sort_keys<48>(keys + list, len);
     }
-    insertion_sort(a, n);
+    uint32_t beg = __builtin_amdgcn_readfirstlane(s_off[first]);
+    uint32_t const end = __builtin_amdgcn_readfirstlane(s_off[last]);
+    while (beg < end)
+    {
+        uint32_t stop = min(beg + 64u, end);
+        uint32_t const lo = __builtin_amdgcn_readfirstlane(owners.of(stop - 1u));
+        uint32_t const lo_end = __builtin_amdgcn_readfirstlane(s_off[lo + 1u]);
+        if (lo_end > stop) // the last list does not end here
+        {
+            uint32_t const lo_beg = __builtin_amdgcn_readfirstlane(s_off[lo]);
+            if (lo_beg == beg)
+            {
+                wave_sort_long(keys + beg, lo_end - beg);
+                beg = lo_end;
+                continue;
+            }
+            stop = lo_beg;
+        }
+        uint32_t const t = beg + lane;
+        K key = 0;
+        uint32_t list = 0u, len = 0u, rank = 0u;
+        if (t < stop)
+        {
+            uint32_t const o = owners.of(t);
+            key = keys[t];
+            list = s_off[o];
+            len = s_off[o + 1u] - list;
+        }
+        for (uint32_t m = 0; __builtin_amdgcn_ballot_w64(m < len); m += 8u)
+        {
+            K other[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u)
+                other[u] = keys[list + m + u]; // past the list: other keys or their owners, not counted
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u)
+                rank += (m + u < len && other[u] < key) ? 1u : 0u;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // every lane has read
+        __builtin_amdgcn_wave_barrier();
+        if (t < stop)
+            keys[list + rank] = key;
+        beg = stop;
+    }
 }
 
 // Writes the bond of query point i (at qx, qy, qz) given its key, at bond
 // index bidx.
-// NT: non-temporal stores, for a block's contiguous range of the
-// NeighborList (full lines; the output then does not push the gathered
-// positions out of L2).  Scattered segments keep ordinary stores, whose
-// partial lines merge in L2.
-template<int FORMULA, bool BYDIST, bool NT = false>
+template<int FORMULA>
 __device__ inline void write_bond_at(const DevBox& b, float qx, float qy, float qz, const float* __restrict__ pts,
                                      uint32_t i, uint64_t key, uint64_t bidx, uint32_t* __restrict__ nb_out,
                                      float* __restrict__ d_out, float* __restrict__ w_out, float* __restrict__ v_out)
@@ -212,16 +327,6 @@ __device__ inline void write_bond_at(const DevBox& b, float qx, float qy, float 
     float rx, ry, rz;
     fa::bond_vector<FORMULA>(b, qx, qy, qz, pts[3 * j], pts[3 * j + 1], pts[3 * j + 2], code, rx, ry, rz);
     float const r_sq = (rx * rx + ry * ry) + rz * rz;
-    if (NT)
-    {
-        __builtin_nontemporal_store((uint64_t(j) << 32) | uint64_t(i), reinterpret_cast<uint64_t*>(nb_out) + bidx);
-        __builtin_nontemporal_store(sqrtf(r_sq), d_out + bidx);
-        __builtin_nontemporal_store(1.0f, w_out + bidx);
-        __builtin_nontemporal_store(rx, v_out + 3 * bidx);
-        __builtin_nontemporal_store(ry, v_out + 3 * bidx + 1);
-        __builtin_nontemporal_store(rz, v_out + 3 * bidx + 2);
-        return;
-    }
     reinterpret_cast<uint2*>(nb_out)[bidx] = make_uint2(i, j);
     d_out[bidx] = sqrtf(r_sq);
     w_out[bidx] = 1.0f;
@@ -230,56 +335,52 @@ __device__ inline void write_bond_at(const DevBox& b, float qx, float qy, float 
     v_out[3 * bidx + 2] = rz;
 }
 
-template<int FORMULA, bool BYDIST>
+template<int FORMULA>
 __device__ inline void write_bond(const DevBox& b, const float* __restrict__ qpts, const float* __restrict__ pts,
                                   uint32_t i, uint64_t key, uint64_t bidx, uint32_t* __restrict__ nb_out,
                                   float* __restrict__ d_out, float* __restrict__ w_out, float* __restrict__ v_out)
 {
-    write_bond_at<FORMULA, BYDIST>(b, qpts[3 * i], qpts[3 * i + 1], qpts[3 * i + 2], pts, i, key, bidx, nb_out, d_out,
+    write_bond_at<FORMULA>(b, qpts[3 * i], qpts[3 * i + 1], qpts[3 * i + 2], pts, i, key, bidx, nb_out, d_out,
                                    w_out, v_out);
 }
 
-// Marks the owner (point lo of the block) of each of its key slots: one pass of
-// short byte writes instead of a binary search over the offsets per key and
-// pass.  Every thread tid < nloc calls it with its own range.
-__device__ inline void mark_owner(uint8_t* own, uint32_t beg, uint32_t cnt)
-{
-    for (uint32_t m = 0; m < cnt; ++m)
-        own[beg + m] = uint8_t(threadIdx.x);
-}
-
 // Block-cooperative store of a block's bonds: keys[t] for t < total belong to
-// the block's query points in processing order (owners own[t], exclusive
-// offsets s_off, point indices s_i, positions s_q); bond t of point lo goes to
-// offsets[s_i[lo]] + t - s_off[lo], which is first + t when the block's points
-// are consecutive (INDEX).  A wave's 64 bond vectors go through LDS, so that
-// every store instruction writes whole lines (three strided dword stores per
-// bond write each line three times).
-template<int FORMULA, bool BYDIST, typename K, bool INDEX>
+// the block's query points in processing order (point indices s_i, positions
+// s_q); bond t of point lo goes to offsets[s_i[lo]] + t - s_off[lo], which is first + t when the block's points
+// are consecutive (INDEX).  A wave's 64 bond vectors are passed between its
+// lanes, so that every store instruction writes whole lines (three strided
+// dword stores per bond write each line three times).  INDEX stores are
+// non-temporal: the block's range is contiguous, and its full lines then do not
+// push the gathered positions out of L2; scattered lists keep ordinary stores,
+// whose partial lines merge there.
+template<int FORMULA, typename K, bool INDEX>
 __device__ inline void store_block_bonds(const DevBox& b, const float* s_q, const float* __restrict__ pts,
-                                         const K* keys, const uint8_t* own, uint32_t total, const uint32_t* s_off,
-                                         const uint32_t* s_i, const uint32_t* __restrict__ offsets, uint32_t first,
+                                         const K* keys, const KeyOwners& owners, uint32_t total, const uint32_t* s_i,
+                                         const uint32_t* __restrict__ offsets, uint32_t first,
                                          uint32_t* __restrict__ nb_out, float* __restrict__ d_out,
                                          float* __restrict__ w_out, float* __restrict__ v_out)
 {
-    __shared__ float s_v[kBlock / 64][192];
-    __shared__ uint32_t s_b[kBlock / 64][64];
-    uint32_t const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t const lane = threadIdx.x & 63u;
+    uint32_t src[3], turn[3]; // bond m with 3 m + axis = lane (mod 64), and that component's c
+#pragma unroll
+    for (uint32_t axis = 0; axis < 3; ++axis)
+    {
+        src[axis] = ((lane - axis) * 43u) & 63u; // 3 x 43 = 1 (mod 64)
+        turn[axis] = (3u * src[axis] + axis) >> 6;
+    }
     for (uint32_t t0 = threadIdx.x - lane; t0 < total; t0 += kBlock)
     {
         uint32_t const t = t0 + lane, have = min(64u, total - t0);
+        uint32_t bidx = 0u;
+        float rx = 0.0f, ry = 0.0f, rz = 0.0f;
         if (t < total)
         {
-            uint32_t const lo = own[t], i = s_i[lo];
+            uint32_t const lo = owners.of(t), i = s_i[lo];
             uint32_t const jc = uint32_t(keys[t]), j = jc >> 5;
-            uint32_t const bidx = INDEX ? first + t : offsets[i] + (t - s_off[lo]);
-            float rx, ry, rz;
+            bidx = INDEX ? first + t : offsets[i] + (t - owners.s_off[lo]);
             fa::bond_vector<FORMULA>(b, s_q[3 * lo], s_q[3 * lo + 1], s_q[3 * lo + 2], pts[3 * j], pts[3 * j + 1],
                                      pts[3 * j + 2], int(jc & 31u), rx, ry, rz);
             float const d = sqrtf((rx * rx + ry * ry) + rz * rz);
-            s_v[wave][3 * lane] = rx;
-            s_v[wave][3 * lane + 1] = ry;
-            s_v[wave][3 * lane + 2] = rz;
             if (INDEX)
             {
                 __builtin_nontemporal_store((uint64_t(j) << 32) | uint64_t(i),
@@ -289,39 +390,38 @@ __device__ inline void store_block_bonds(const DevBox& b, const float* s_q, cons
             }
             else
             {
-                s_b[wave][lane] = bidx;
                 reinterpret_cast<uint2*>(nb_out)[bidx] = make_uint2(i, j);
                 d_out[bidx] = d;
                 w_out[bidx] = 1.0f;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the wave's vectors are in LDS
-        __builtin_amdgcn_wave_barrier();
+        // lane's component f = 64 c + lane of the wave's 192 is axis f mod 3 of bond
+        // f / 3; over c = 0 .. 2 it takes each axis once, from bond src[axis]
+        float got[3];
+        got[0] = __shfl(rx, int(src[0]));
+        got[1] = __shfl(ry, int(src[1]));
+        got[2] = __shfl(rz, int(src[2]));
 #pragma unroll
         for (uint32_t c = 0; c < 3; ++c)
         {
             uint32_t const f = c * 64u + lane;
+            float const v = turn[0] == c ? got[0] : turn[1] == c ? got[1] : got[2];
+            uint32_t const at = INDEX ? 0u : uint32_t(__shfl(int(bidx), int(f / 3u)));
             if (f < 3u * have)
             {
-                float const v = s_v[wave][f];
                 if (INDEX)
                     __builtin_nontemporal_store(v, v_out + 3 * uint64_t(first + t0) + f);
                 else
-                {
-                    uint32_t const m = f / 3u;
-                    v_out[3 * uint64_t(s_b[wave][m]) + (f - 3u * m)] = v;
-                }
+                    v_out[3 * uint64_t(at) + f % 3u] = v;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // and may be overwritten
-        __builtin_amdgcn_wave_barrier();
     }
 }
 
 // One block's share of the fill pass: query positions [p0, p0 + nloc).  Point
 // indices i are relative to `offsets`, `qpts` and `pts` (a frame of a batch
 // passes pointers advanced to its first point); bond indices are absolute.
-template<int FORMULA, bool BYDIST, bool SELF>
+template<int FORMULA, bool BYDIST, bool SELF, int NET>
 __device__ inline void ball_fill_body(const DevBox& b, const DevGrid& g, const float* __restrict__ qpts, uint32_t p0,
                                       uint32_t nloc, const float* __restrict__ pts, float r_max_sq, float r_min_sq,
                                       int exclude_ii, int R, const uint32_t* __restrict__ offsets,
@@ -335,11 +435,12 @@ __device__ inline void ball_fill_body(const DevBox& b, const DevGrid& g, const f
     // the kernel keeps its occupancy (blocks over the capacity use gkeys_raw)
     K* s_keys = reinterpret_cast<K*>(fa_dyn_lds);
     uint32_t const CAP = key_cap;
-    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
     __shared__ uint32_t s_off[kBlock + 1];
     __shared__ uint32_t s_i[kBlock];
-    __shared__ uint32_t s_tmp[kBlock];
+    KeyOwners const owners{reinterpret_cast<uint8_t*>(s_keys + key_cap), s_off,
+                           owner_stride(size_t(key_cap) * sizeof(K), gridDim.x)};
     __shared__ float s_q[3 * kBlock];
+    uint32_t* const s_tmp = reinterpret_cast<uint32_t*>(fa_dyn_lds); // before the keys
     uint32_t const tid = threadIdx.x;
     float qx = 0.0f, qy = 0.0f, qz = 0.0f;
     uint32_t i = 0, cnt = 0;
@@ -381,21 +482,22 @@ __device__ inline void ball_fill_body(const DevBox& b, const DevGrid& g, const f
                                             }
                                         });
         if (in_lds)
-        {
-            mark_owner(s_own, beg, cnt);
-            sort_keys(s_keys + beg, k - beg);
-        }
+            owners.mark(beg, cnt);
         else
+        {
             insertion_sort(keys + beg, k - beg);
-        if (!in_lds)
             for (uint32_t m = 0; m < k - beg; ++m)
-                write_bond<FORMULA, BYDIST>(b, qpts, pts, i, uint64_t(keys[beg + m]), uint64_t(offsets[i]) + m,
-                                            nb_out, d_out, w_out, v_out);
+                write_bond<FORMULA>(b, qpts, pts, i, uint64_t(keys[beg + m]), uint64_t(offsets[i]) + m, nb_out, d_out,
+                                    w_out, v_out);
+        }
     }
     __syncthreads();
-    if (in_lds)
-        store_block_bonds<FORMULA, BYDIST, K, false>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets, 0u, nb_out,
-                                                     d_out, w_out, v_out);
+    if (!in_lds)
+        return;
+    block_sort_lists<NET>(s_keys, owners, nloc);
+    __syncthreads();
+    store_block_bonds<FORMULA, K, false>(b, s_q, pts, s_keys, owners, total, s_i, offsets, 0u, nb_out, d_out,
+                                         w_out, v_out);
 }
 
 // ------------------------------------------------------------------ ball query: one walk
@@ -491,7 +593,7 @@ __global__ __launch_bounds__(kBlock) void ball_walk_kernel(DevBox b, DevGrid g, 
 // indices with INDEX, else processing positions).  Point indices are relative
 // to qpts, pts, pos and offsets (a frame of a batch passes them advanced to its
 // first point); bond indices and rows slots are absolute.
-template<int FORMULA, bool BYDIST, bool SELF, bool INDEX>
+template<int FORMULA, bool BYDIST, bool SELF, bool INDEX, int NET>
 __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const float* __restrict__ qpts, uint32_t p0,
                                       uint32_t nloc, const float* __restrict__ pts, float r_max_sq, float r_min_sq,
                                       int exclude_ii, int R, const fa::CQGrid& cq, uint32_t C,
@@ -502,10 +604,10 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
 {
     using K = typename std::conditional<BYDIST, uint64_t, uint32_t>::type;
     K* s_keys = reinterpret_cast<K*>(fa_dyn_lds);
-    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
     __shared__ uint32_t s_off[kBlock + 1];
     __shared__ uint32_t s_i[kBlock];
-    __shared__ uint32_t s_tmp[kBlock];
+    KeyOwners const owners{reinterpret_cast<uint8_t*>(s_keys + key_cap), s_off,
+                           owner_stride(size_t(key_cap) * sizeof(K), gridDim.x)};
     __shared__ uint32_t s_row[kBlock];
     __shared__ float s_q[3 * kBlock];
     uint32_t const tid = threadIdx.x;
@@ -529,7 +631,7 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
         s_q[3 * tid + 2] = qz;
     }
     uint32_t excl;
-    uint32_t const total = block_exclusive_scan(cnt, s_tmp, excl);
+    uint32_t const total = block_exclusive_scan(cnt, reinterpret_cast<uint32_t*>(fa_dyn_lds), excl);
     if (tid < nloc)
         s_off[tid] = excl;
     if (tid == 0)
@@ -551,7 +653,7 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
     };
     bool const coop = in_lds && C > 0;
     if (in_lds && tid < nloc)
-        mark_owner(s_own, excl, cnt);
+        owners.mark(excl, cnt);
     if (coop)
     {
         // The staged key rows into LDS, element t by thread t: one load
@@ -563,7 +665,7 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
         __syncthreads();
         for (uint32_t t = tid; t < total; t += kBlock)
         {
-            uint32_t const lo = s_own[t];
+            uint32_t const lo = owners.of(t);
             uint32_t const r0 = s_row[lo];
             if (r0 != ~0u)
                 s_keys[t] = key_of(rows[r0 + (t - s_off[lo])], s_q[3 * lo], s_q[3 * lo + 1], s_q[3 * lo + 2]);
@@ -599,22 +701,24 @@ __device__ inline void ball_emit_body(const DevBox& b, const DevGrid& g, const f
                                          }
                                      });
         }
-        if (in_lds)
-            sort_keys(s_keys + beg, cnt);
-        else
-            insertion_sort(keys + beg, cnt);
         if (!in_lds)
+        {
+            insertion_sort(keys + beg, cnt);
             for (uint32_t m = 0; m < cnt; ++m)
-                write_bond_at<FORMULA, BYDIST>(b, qx, qy, qz, pts, i, uint64_t(keys[beg + m]),
-                                               uint64_t(offsets[i]) + m, nb_out, d_out, w_out, v_out);
+                write_bond_at<FORMULA>(b, qx, qy, qz, pts, i, uint64_t(keys[beg + m]), uint64_t(offsets[i]) + m,
+                                       nb_out, d_out, w_out, v_out);
+        }
     }
     __syncthreads();
-    if (in_lds)
-        store_block_bonds<FORMULA, BYDIST, K, INDEX>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets,
-                                                     INDEX ? offsets[p0] : 0u, nb_out, d_out, w_out, v_out);
+    if (!in_lds)
+        return;
+    block_sort_lists<NET>(s_keys, owners, nloc);
+    __syncthreads();
+    store_block_bonds<FORMULA, K, INDEX>(b, s_q, pts, s_keys, owners, total, s_i, offsets,
+                                         INDEX ? offsets[p0] : 0u, nb_out, d_out, w_out, v_out);
 }
 
-template<int FORMULA, bool BYDIST, bool SELF, bool INDEX>
+template<int FORMULA, bool BYDIST, bool SELF, bool INDEX, int NET>
 __global__ __launch_bounds__(kBlock) void ball_emit_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
                                                            uint32_t nq, const float* __restrict__ pts,
                                                            float r_max_sq, float r_min_sq, int exclude_ii, int R,
@@ -623,12 +727,13 @@ __global__ __launch_bounds__(kBlock) void ball_emit_kernel(DevBox b, DevGrid g, 
                                                            const uint32_t* __restrict__ offsets,
                                                            uint32_t* __restrict__ nb_out, float* __restrict__ d_out,
                                                            float* __restrict__ w_out, float* __restrict__ v_out,
-                                                           void* __restrict__ gkeys_raw, uint32_t key_cap)
+                                                           void* __restrict__ gkeys_raw, uint32_t key_cap,
+                                                           uint32_t points)
 {
-    uint32_t const p0 = fa::xcd_tile(blockIdx.x, gridDim.x) * kBlock;
-    ball_emit_body<FORMULA, BYDIST, SELF, INDEX>(b, g, qpts, p0, min(uint32_t(kBlock), nq - p0), pts, r_max_sq,
-                                                 r_min_sq, exclude_ii, R, cq, C, pos, rows, offsets, nb_out, d_out,
-                                                 w_out, v_out, gkeys_raw, key_cap);
+    uint32_t const p0 = fa::xcd_tile(blockIdx.x, gridDim.x) * points;
+    ball_emit_body<FORMULA, BYDIST, SELF, INDEX, NET>(b, g, qpts, p0, min(points, nq - p0), pts, r_max_sq, r_min_sq,
+                                                 exclude_ii, R, cq, C, pos, rows, offsets, nb_out, d_out, w_out, v_out,
+                                                 gkeys_raw, key_cap);
 }
 
 // Segments with the reference's convention (0 for query points without bonds).
@@ -641,76 +746,6 @@ __global__ void counts_segments_kernel(const uint32_t* __restrict__ offsets, uin
     uint32_t const c = offsets[i + 1] - offsets[i];
     counts[i] = c;
     segments[i] = c ? offsets[i] : 0u;
-}
-
-// ------------------------------------------------------------------ dense ball queries
-// Lists too long for the walk's LDS key stage (33 bonds per point and more) are
-// counted, then walked again by the emission.  Up to kDenseSlots expected bonds
-// the keys are sorted in registers: an insertion sort in LDS took half of the
-// emission's time.  (Keeping the first walk's keys in device memory instead
-// made the walk dearer, 112 -> 199 us, than the second walk it saved.)
-// 500,000 random points, 28 bonds each: emission 640 -> 485 us.
-// The emission, in processing order, kDensePoints points per workgroup (their
-// keys fit 20 KB of LDS at 38 bonds each; workgroups over the capacity sort in
-// device memory, waves with a longer list than kDenseSlots by insertion).
-constexpr uint32_t kDensePoints = 128;
-template<int FORMULA, bool SELF>
-__global__ __launch_bounds__(kBlock) void ball_emit_dense_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts,
-                                                                 uint32_t nq, const float* __restrict__ pts,
-                                                                 float r_max_sq, float r_min_sq, int exclude_ii, int R,
-                                                                 fa::CQGrid cq, const uint32_t* __restrict__ offsets,
-                                                                 uint32_t* __restrict__ nb_out,
-                                                                 float* __restrict__ d_out, float* __restrict__ w_out,
-                                                                 float* __restrict__ v_out,
-                                                                 uint32_t* __restrict__ gkeys, uint32_t key_cap)
-{
-    uint32_t* const s_keys = reinterpret_cast<uint32_t*>(fa_dyn_lds);
-    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
-    __shared__ uint32_t s_off[kBlock + 1];
-    __shared__ uint32_t s_i[kBlock];
-    __shared__ uint32_t s_tmp[kBlock];
-    __shared__ float s_q[3 * kBlock];
-    uint32_t const tid = threadIdx.x;
-    uint32_t const p0 = fa::xcd_tile(blockIdx.x, gridDim.x) * kDensePoints;
-    uint32_t const nloc = min(kDensePoints, nq - p0);
-    float qx = 0.0f, qy = 0.0f, qz = 0.0f;
-    uint32_t i = 0, cnt = 0;
-    if (tid < nloc)
-    {
-        i = query_at<SELF>(g, qpts, p0 + tid, qx, qy, qz);
-        cnt = offsets[i + 1] - offsets[i];
-        s_i[tid] = i;
-        s_q[3 * tid] = qx;
-        s_q[3 * tid + 1] = qy;
-        s_q[3 * tid + 2] = qz;
-    }
-    uint32_t excl;
-    uint32_t const total = block_exclusive_scan(cnt, s_tmp, excl);
-    bool const in_lds = total <= key_cap;
-    if (tid < nloc)
-    {
-        s_off[tid] = excl;
-        uint32_t* const keys = in_lds ? s_keys + excl : gkeys + offsets[i];
-        if (in_lds)
-            mark_owner(s_own, excl, cnt);
-        uint32_t k = 0;
-        fa::visit_bonds<FORMULA>(b, g, cq, qx, qy, qz, R, [&](uint32_t j, float, float, float, float r_sq, int code) {
-            if (r_sq < r_max_sq && r_sq >= r_min_sq && k < cnt && !(exclude_ii && j == i))
-                keys[k++] = (j << 5) | uint32_t(code);
-        });
-        if (in_lds && !__builtin_amdgcn_ballot_w64(cnt > kDenseSlots))
-            register_sort_keys<int(kDenseSlots)>(s_keys + excl, cnt);
-        else
-            insertion_sort(keys, k);
-        if (!in_lds)
-            for (uint32_t m = 0; m < cnt; ++m)
-                write_bond_at<FORMULA, false>(b, qx, qy, qz, pts, i, uint64_t(keys[m]), uint64_t(offsets[i]) + m,
-                                              nb_out, d_out, w_out, v_out);
-    }
-    __syncthreads();
-    if (in_lds)
-        store_block_bonds<FORMULA, false, uint32_t, false>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets, 0u,
-                                                           nb_out, d_out, w_out, v_out);
 }
 
 // ------------------------------------------------------------------ kNN
@@ -1184,7 +1219,7 @@ __global__ __launch_bounds__(kBlock) void wave_emit_kernel(DevBox b, const float
     uint32_t const e0 = offsets[i], n = offsets[i + 1] - e0;
     float const qx = qpts[3 * i], qy = qpts[3 * i + 1], qz = qpts[3 * i + 2];
     for (uint32_t m = threadIdx.x & 15u; m < n; m += 16u)
-        write_bond_at<AABB_FORMULA, false>(b, qx, qy, qz, pts, i, uint64_t(rows[uint64_t(i) * C + m]),
+        write_bond_at<AABB_FORMULA>(b, qx, qy, qz, pts, i, uint64_t(rows[uint64_t(i) * C + m]),
                                            uint64_t(e0) + m, nb_out, d_out, w_out, v_out);
 }
 
@@ -1310,7 +1345,7 @@ __global__ __launch_bounds__(kBlock) void knn_rank_emit_kernel(DevBox b, const f
         uint32_t rank = 0;
         for (uint32_t t = 0; t < n; ++t)
             rank += key_of(row[t]) < own ? 1u : 0u;
-        write_bond_at<AABB_FORMULA, BYDIST>(b, qx, qy, qz, pts, i, own, uint64_t(e0) + rank, nb_out, d_out, w_out, v_out);
+        write_bond_at<AABB_FORMULA>(b, qx, qy, qz, pts, i, own, uint64_t(e0) + rank, nb_out, d_out, w_out, v_out);
     }
 }
 
@@ -1441,7 +1476,7 @@ __global__ __launch_bounds__(kBlock) void knn_exhaustive_kernel(DevBox b, const 
 // selected keys (point-major rows by processing position: pos[i] for
 // cell-ordered self queries) are sorted into the NeighborList order ((i, j) or
 // (i, d, j)), staged in LDS and stored cooperatively.
-template<int FORMULA, bool BYDIST, bool SELF, bool INDEX>
+template<int FORMULA, bool BYDIST, bool SELF, bool INDEX, int NET>
 __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, const float* __restrict__ qpts, uint32_t nq,
                                                            const float* __restrict__ pts, uint32_t k,
                                                            const uint64_t* __restrict__ sel,
@@ -1454,10 +1489,10 @@ __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, 
     using K = typename std::conditional<BYDIST, uint64_t, uint32_t>::type;
     K* s_keys = reinterpret_cast<K*>(fa_dyn_lds); // key_cap entries (dynamic LDS), then their owners
     uint32_t const CAP = key_cap;
-    uint8_t* const s_own = reinterpret_cast<uint8_t*>(s_keys + key_cap);
     __shared__ uint32_t s_off[kBlock + 1];
     __shared__ uint32_t s_i[kBlock];
-    __shared__ uint32_t s_tmp[kBlock];
+    KeyOwners const owners{reinterpret_cast<uint8_t*>(s_keys + key_cap), s_off,
+                           owner_stride(size_t(key_cap) * sizeof(K), gridDim.x)};
     __shared__ uint32_t s_row[kBlock];
     __shared__ float s_q[3 * kBlock];
     uint32_t const tid = threadIdx.x;
@@ -1483,7 +1518,7 @@ __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, 
         s_q[3 * tid + 2] = qz;
     }
     uint32_t excl;
-    uint32_t const total = block_exclusive_scan(n, s_tmp, excl);
+    uint32_t const total = block_exclusive_scan(n, reinterpret_cast<uint32_t*>(fa_dyn_lds), excl);
     if (tid < nloc)
         s_off[tid] = excl;
     if (tid == 0)
@@ -1505,17 +1540,23 @@ __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, 
         if (tid < nloc)
         {
             s_row[tid] = INDEX && SELF ? pos[i] : p0 + tid;
-            mark_owner(s_own, excl, n);
+            owners.mark(excl, n);
         }
         __syncthreads();
         for (uint32_t t = tid; t < total; t += kBlock)
         {
-            uint32_t const lo = s_own[t];
+            uint32_t const lo = owners.of(t);
             s_keys[t] = key_of(sel[uint64_t(s_row[lo]) * k + (t - s_off[lo])]);
         }
         __syncthreads();
-        if (tid < nloc)
-            sort_keys(s_keys + excl, n);
+        if constexpr (BYDIST)
+        {
+            // the selections arrive in this order: one look at each
+            if (tid < nloc)
+                insertion_sort(s_keys + excl, n);
+        }
+        else
+            block_sort_lists<NET>(s_keys, owners, nloc);
     }
     else if (tid < nloc)
     {
@@ -1525,13 +1566,13 @@ __global__ __launch_bounds__(kBlock) void knn_write_kernel(DevBox b, DevGrid g, 
             keys[m] = key_of(row[m]);
         insertion_sort(keys, n);
         for (uint32_t m = 0; m < n; ++m)
-            write_bond<FORMULA, BYDIST>(b, qpts, pts, i, uint64_t(keys[m]), uint64_t(offsets[i]) + m, nb_out, d_out,
+            write_bond<FORMULA>(b, qpts, pts, i, uint64_t(keys[m]), uint64_t(offsets[i]) + m, nb_out, d_out,
                                         w_out, v_out);
     }
     __syncthreads();
     if (in_lds)
-        store_block_bonds<FORMULA, BYDIST, K, INDEX>(b, s_q, pts, s_keys, s_own, total, s_off, s_i, offsets,
-                                                     INDEX ? offsets[p0] : 0u, nb_out, d_out, w_out, v_out);
+        store_block_bonds<FORMULA, K, INDEX>(b, s_q, pts, s_keys, owners, total, s_i, offsets,
+                                             INDEX ? offsets[p0] : 0u, nb_out, d_out, w_out, v_out);
 }
 
 // ------------------------------------------------------------------ all pairs
@@ -1598,7 +1639,7 @@ __global__ __launch_bounds__(kBlock) void bball_fill_kernel(fa::BatchGrid G, con
     uint32_t const local0 = (t - F.tile_base) * fa::kTile;
     DevGrid const g = fa::frame_grid(F, G);
     const float* fp = pts + 3 * size_t(F.pt_base);
-    ball_fill_body<AABB_FORMULA, false, true>(F.box, g, fp, F.pt_base + local0, min(fa::kTile, F.n - local0), fp,
+    ball_fill_body<AABB_FORMULA, false, true, 32>(F.box, g, fp, F.pt_base + local0, min(fa::kTile, F.n - local0), fp,
                                               r_max_sq, 0.0f, 1, R, offsets + F.pt_base, nb_out, d_out, w_out, v_out,
                                               gkeys, key_cap);
 }
@@ -1643,7 +1684,7 @@ __global__ __launch_bounds__(kBlock) void bball_emit_kernel(fa::BatchGrid G, con
     uint32_t const local0 = (t - F.tile_base) * fa::kTile;
     DevGrid const g = fa::frame_grid(F, G);
     const float* fp = pts + 3 * size_t(F.pt_base);
-    ball_emit_body<AABB_FORMULA, false, true, false>(F.box, g, fp, F.pt_base + local0, min(fa::kTile, F.n - local0),
+    ball_emit_body<AABB_FORMULA, false, true, false, 32>(F.box, g, fp, F.pt_base + local0, min(fa::kTile, F.n - local0),
                                                      fp, r_max_sq, 0.0f, 1, R, fa::CQGrid{}, C, pos + F.pt_base, rows,
                                                      offsets + F.pt_base, nb_out, d_out, w_out, v_out, gkeys,
                                                      key_cap);
@@ -1670,7 +1711,7 @@ int batch_ball_fill(const BatchGrid& G, const uint32_t* d_tile_frame, uint32_t n
     // the key staging is sized from the allocation (bonds per point of the batch)
     size_t const kb = fill_key_bytes(capacity, G.total_points, sizeof(uint32_t));
     if (ntiles)
-        FA_KLAUNCH(bball_fill_kernel, dim3(ntiles), dim3(kBlock), owner_lds(kb, sizeof(uint32_t)), stream(), G, d_tile_frame, ntiles, d_pts,
+        FA_KLAUNCH(bball_fill_kernel, dim3(ntiles), dim3(kBlock), owner_lds(kb, sizeof(uint32_t), ntiles), stream(), G, d_tile_frame, ntiles, d_pts,
                    r_max * r_max, R, d_offsets, d_total, capacity, nb, dist, wts, vec, gkeys,
                    uint32_t(kb / sizeof(uint32_t)));
     FA_HIP(hipGetLastError());
@@ -1706,7 +1747,7 @@ int batch_ball_emit(const BatchGrid& G, const uint32_t* d_tile_frame, uint32_t n
 {
     size_t const kb = fill_key_bytes(capacity, G.total_points, sizeof(uint32_t));
     if (ntiles)
-        FA_KLAUNCH(bball_emit_kernel, dim3(ntiles), dim3(kBlock), owner_lds(kb, sizeof(uint32_t)), stream(), G, d_tile_frame, ntiles, d_pts,
+        FA_KLAUNCH(bball_emit_kernel, dim3(ntiles), dim3(kBlock), owner_lds(kb, sizeof(uint32_t), ntiles), stream(), G, d_tile_frame, ntiles, d_pts,
                    r_max * r_max, R, C, d_pos, d_rows, d_offsets, d_total, capacity, nb, dist, wts, vec, gkeys,
                    uint32_t(kb / sizeof(uint32_t)));
     FA_HIP(hipGetLastError());
@@ -2065,14 +2106,14 @@ int launch_knn_lc(const fa::DevBox& db, const DevGrid& g, const float* qpts, uin
 // again by the emission pass.  When that exceeds 32 (a 32 KB LDS stage per
 // block) the walk only counts (0: every point is walked again, in processing
 // order, as a count pass and a fill pass would).
-uint32_t ball_row_slots(const fa_nq* nq, float r_max, uint32_t most = kWalkMaxSlots)
+uint32_t ball_row_slots(const fa_nq* nq, float r_max)
 {
     double const vol = std::max(double(fa::box_volume(nq->box)), 1e-30);
     double const dens = double(nq->n) / vol;
     double const r = double(r_max);
     double const expect = nq->box.is2D ? dens * M_PI * r * r : dens * (4.0 / 3.0) * M_PI * r * r * r;
     double const c = std::ceil((expect * 1.15 + 4.0) / 4.0) * 4.0;
-    if (c > double(most))
+    if (c > double(kWalkMaxSlots))
         return 0;
     return uint32_t(std::max(c, 8.0));
 }
@@ -2110,7 +2151,6 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
     bool const wave = Cw != 0;
     fa::CQGrid const cq = nq->kind == FA_NQ_CELLQUERY ? fa::cq_grid_for(nq->box, a.r_max) : fa::CQGrid{};
     uint32_t const C = wave ? Cw : ball_row_slots(nq, a.r_max);
-    bool const dense = !C && !by_distance && ball_row_slots(nq, a.r_max, kDenseSlots) != 0;
     uint32_t* rows = nullptr;
     uint32_t* pos = nullptr;
     uint32_t* over = nullptr; // device mark of the wave walk: a point without a row
@@ -2178,40 +2218,21 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
     void* gkeys = nullptr;
     if (int rc = fa::scratch(3, std::max<uint64_t>(total, 1) * (by_distance ? 8 : 4), &gkeys))
         return rc;
-    size_t const kb = fill_key_bytes(total, n_query, by_distance ? 8 : 4);
-    uint32_t const key_cap = uint32_t(kb / (by_distance ? 8 : 4));
+    size_t const ksz = by_distance ? 8 : 4;
+    // as many points per workgroup as their keys, with some slack, leave room for
+    // in LDS (lists too long for 32 are sorted in device memory)
+    uint32_t points = kBlock;
+    while (points > 32u && 1.15 * double(total) * points * double(ksz) > double(kBallKeyBytes) * n_query)
+        points /= 2;
+    size_t const kb = fill_key_bytes(total, n_query, ksz, points);
     auto emit = [&](auto kern) {
         FA_PROF_BEGIN("ball_emit_kernel");
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), owner_lds(kb, by_distance ? 8 : 4), s, db, g, qpts, n_query,
-                           nq->d_points, r_max_sq,
-                           r_min_sq, a.exclude_ii, R, cq, C, pos, rows, out->offsets, out->neighbors, out->distances,
-                           out->weights, out->vectors, gkeys, key_cap);
+        unsigned const eblocks = (n_query + points - 1) / points;
+        hipLaunchKernelGGL(kern, dim3(eblocks), dim3(kBlock), owner_lds(kb, ksz, eblocks), s, db, g, qpts, n_query,
+                           nq->d_points, r_max_sq, r_min_sq, a.exclude_ii, R, cq, C, pos, rows, out->offsets,
+                           out->neighbors, out->distances, out->weights, out->vectors, gkeys, uint32_t(kb / ksz), points);
         FA_PROF_END();
     };
-    if (dense && n_query)
-    {
-        size_t const dkb = fill_key_bytes(total, uint64_t(n_query) * (kBlock / kDensePoints), sizeof(uint32_t));
-        auto emit_dense = [&](auto kern) {
-            FA_PROF_BEGIN("ball_emit_kernel");
-            hipLaunchKernelGGL(kern, dim3((n_query + kDensePoints - 1) / kDensePoints), dim3(kBlock),
-                               owner_lds(dkb, sizeof(uint32_t)), s, db, g, qpts, n_query, nq->d_points, r_max_sq,
-                               r_min_sq, a.exclude_ii, R, cq, out->offsets, out->neighbors, out->distances,
-                               out->weights, out->vectors, static_cast<uint32_t*>(gkeys),
-                               uint32_t(dkb / sizeof(uint32_t)));
-            FA_PROF_END();
-        };
-        if (nq->kind == FA_NQ_AABB)
-            self ? emit_dense(ball_emit_dense_kernel<AABB_FORMULA, true>)
-                 : emit_dense(ball_emit_dense_kernel<AABB_FORMULA, false>);
-        else if (nq->kind == FA_NQ_CELLQUERY)
-            self ? emit_dense(ball_emit_dense_kernel<CELLQUERY_FORMULA, true>)
-                 : emit_dense(ball_emit_dense_kernel<CELLQUERY_FORMULA, false>);
-        else
-            self ? emit_dense(ball_emit_dense_kernel<LINKCELL_FORMULA, true>)
-                 : emit_dense(ball_emit_dense_kernel<LINKCELL_FORMULA, false>);
-        FA_HIP(hipGetLastError());
-        return FA_OK;
-    }
     // self queries of points stored in random order emit in processing order,
     // and so does a walk that kept no keys (the emission pass walks again)
     bool index_order = C > 0;
@@ -2222,30 +2243,36 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
             return rc;
         index_order = sorder == nullptr;
     }
-#define FA_BALL_EMIT(FORM)                                                                                       \
-    do                                                                                                           \
-    {                                                                                                            \
-        if (!self)                                                                                               \
-            by_distance ? emit(ball_emit_kernel<FORM, true, false, true>)                                        \
-                        : emit(ball_emit_kernel<FORM, false, false, true>);                                      \
-        else if (index_order)                                                                                    \
-            by_distance ? emit(ball_emit_kernel<FORM, true, true, true>)                                         \
-                        : emit(ball_emit_kernel<FORM, false, true, true>);                                       \
-        else                                                                                                     \
-            by_distance ? emit(ball_emit_kernel<FORM, true, true, false>)                                        \
-                        : emit(ball_emit_kernel<FORM, false, true, false>);                                      \
-    } while (0)
+    // the register networks for the lists' mean length with some spread (block_sort_lists)
+    auto emit_form = [&](auto form, auto by_dist, auto net) {
+        constexpr int F = decltype(form)::value, N = decltype(net)::value;
+        constexpr bool D = decltype(by_dist)::value;
+        self ? index_order ? emit(ball_emit_kernel<F, D, true, true, N>) : emit(ball_emit_kernel<F, D, true, false, N>)
+             : emit(ball_emit_kernel<F, D, false, true, N>);
+    };
+    double const mean = n_query ? double(total) / n_query : 0.0;
+    auto emit_all = [&](auto form) {
+        if (by_distance)
+            emit_form(form, std::true_type{}, std::integral_constant<int, 0>{});
+        else if (mean <= 6.0)
+            emit_form(form, std::false_type{}, std::integral_constant<int, 16>{});
+        else if (mean <= 30.0)
+            emit_form(form, std::false_type{}, std::integral_constant<int, 32>{});
+        else if (mean <= 38.0)
+            emit_form(form, std::false_type{}, std::integral_constant<int, 48>{});
+        else
+            emit_form(form, std::false_type{}, std::integral_constant<int, 0>{});
+    };
     if (n_query)
     {
         if (nq->kind == FA_NQ_AABB)
-            FA_BALL_EMIT(AABB_FORMULA);
+            emit_all(std::integral_constant<int, AABB_FORMULA>{});
         else if (nq->kind == FA_NQ_CELLQUERY)
-            FA_BALL_EMIT(CELLQUERY_FORMULA);
+            emit_all(std::integral_constant<int, CELLQUERY_FORMULA>{});
         else
-            FA_BALL_EMIT(LINKCELL_FORMULA);
+            emit_all(std::integral_constant<int, LINKCELL_FORMULA>{});
         FA_HIP(hipGetLastError());
     }
-#undef FA_BALL_EMIT
     return FA_OK;
 }
 
@@ -2580,10 +2607,23 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
     DevGrid const g = nq->cur->dev();
     auto launch = [&](auto kern) {
         FA_PROF_BEGIN("knn_write_kernel");
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), owner_lds(kb, ksz), s, *dbp, g, qpts, n_query, nq->d_points, k, sel,
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), owner_lds(kb, ksz, blocks), s, *dbp, g, qpts, n_query, nq->d_points, k, sel,
                            pos, out->offsets, out->neighbors, out->distances, out->weights, out->vectors, wtmp,
                            key_cap);
         FA_PROF_END();
+    };
+    // the register network that holds k keys (block_sort_lists)
+    auto write = [&](auto form, auto is_self, auto index) {
+        constexpr int F = decltype(form)::value;
+        constexpr bool S = decltype(is_self)::value, I = decltype(index)::value;
+        if (by_distance)
+            launch(knn_write_kernel<F, true, S, I, 0>);
+        else if (k <= 16)
+            launch(knn_write_kernel<F, false, S, I, 16>);
+        else if (k <= 32)
+            launch(knn_write_kernel<F, false, S, I, 32>);
+        else
+            launch(knn_write_kernel<F, false, S, I, 0>);
     };
     if (nq->kind == FA_NQ_AABB && n_query <= kWaveQueries && k <= 64)
     {
@@ -2610,22 +2650,19 @@ int run_knn(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args&
                 return rc;
             index_order = sorder == nullptr;
         }
+        auto form = std::integral_constant<int, AABB_FORMULA>{};
         if (!self)
-            by_distance ? launch(knn_write_kernel<AABB_FORMULA, true, false, true>)
-                        : launch(knn_write_kernel<AABB_FORMULA, false, false, true>);
+            write(form, std::false_type{}, std::true_type{});
         else if (index_order)
-            by_distance ? launch(knn_write_kernel<AABB_FORMULA, true, true, true>)
-                        : launch(knn_write_kernel<AABB_FORMULA, false, true, true>);
+            write(form, std::true_type{}, std::true_type{});
         else
-            by_distance ? launch(knn_write_kernel<AABB_FORMULA, true, true, false>)
-                        : launch(knn_write_kernel<AABB_FORMULA, false, true, false>);
+            write(form, std::true_type{}, std::false_type{});
     }
     else
     {
         // the LinkCell search runs in index order and stores its selections by
         // point index
-        by_distance ? launch(knn_write_kernel<LINKCELL_FORMULA, true, false, true>)
-                    : launch(knn_write_kernel<LINKCELL_FORMULA, false, false, true>);
+        write(std::integral_constant<int, LINKCELL_FORMULA>{}, std::false_type{}, std::true_type{});
     }
     FA_HIP(hipGetLastError());
     return FA_OK;

@@ -440,6 +440,30 @@ def test_large_ball_queries_by_bond_count(oracle, kind, bonds):
             _assert_same(nl, ref)
 
 
+@pytest.mark.parametrize("kind", ["aabb", "linkcell", "cellquery"])
+@pytest.mark.parametrize("bonds", [90, 130, 230, 300])
+def test_ball_emission_of_long_lists(oracle, kind, bonds):
+    """Lists of more keys than a wave has lanes, from 128 points per workgroup
+    down to 32 and past what fits in LDS, with some points of few bonds; self
+    and with distinct query points, by index and by distance."""
+    n = 2501
+    side = n ** (1 / 3)
+    box = Box.cube(side * 1.2)
+    rng = np.random.default_rng(bonds)
+    pts = ((rng.random((n, 3)) - 0.5) * side).astype(np.float32)
+    r = (bonds / 4.18879) ** (1 / 3)
+    make = {"aabb": freud_amd.AABBQuery, "cellquery": freud_amd.CellQuery,
+            "linkcell": lambda b, p: freud_amd.LinkCell(b, p, cell_width=r)}[kind]
+    nq = make(box, pts)
+    q = np.ascontiguousarray(box.wrap(pts[:1501] + np.float32(0.3)), np.float32)
+    for points in (pts, q):
+        for by_distance in (False, True):
+            args = dict(r_max=r, exclude_ii=True)
+            ref = oracle.query(_bt(box), pts, points, args, nq_type=kind, cell_width=r, sort_by_distance=by_distance,
+                               nthreads=16)
+            _assert_same(nq.query(points, args).toNeighborList(sort_by_distance=by_distance), ref)
+
+
 @pytest.mark.parametrize("parts", [1, 3, 70])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, 5000])
 def test_cluster_chains(n, parts):
