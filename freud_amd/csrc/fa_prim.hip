@@ -146,17 +146,17 @@ __global__ __launch_bounds__(kScanThreads) void scan_parts_kernel(const uint32_t
     }
     if (end != n) // the last part only from here on
         return;
+    if (tid == 0)
+        out[n] = before;
+    if (!host)
+        return;
     uint64_t const total = first + block_sum(own, s);
     if (tid == 0)
     {
-        out[n] = uint32_t(total);
-        if (host)
-        {
-            __hip_atomic_store(host, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            for (int k = 0; k < n_extra; ++k)
-                __hip_atomic_store(reinterpret_cast<uint32_t*>(host + 1) + k, extra[k], __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        __hip_atomic_store(host, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        for (int k = 0; k < n_extra; ++k)
+            __hip_atomic_store(reinterpret_cast<uint32_t*>(host + 1) + k, extra[k], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
