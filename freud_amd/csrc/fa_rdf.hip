@@ -1589,12 +1589,16 @@ struct EstRange
     float lo = 0.0f, hi = 0.0f, slack = 0.0f;
 };
 
-// Waves per cluster: clusters of a small system leave the chip idle (4096
-// points: 600 waves on 256 CUs x 32), so up to 8 waves share one.
+// Waves per cluster: the clusters of a small system leave the chip idle, so up
+// to 8 waves share one, as far as about 2,048 waves.  More of them only add
+// workgroups that copy the bin table and add their histogram.  One call in us,
+// r_max = 3, 100 bins, exact kernel, then about 8,192, 4,096 and 2,048 waves:
+// 3,000 points 48, 42, 41, 36; 7,427 points 50, 61, 47, 41; 12,818 points
+// 49, 60, 46, 43 (r_max = 5: 62, 65, 50, 56).
 uint32_t rows_split(uint32_t n)
 {
     uint32_t split = 1;
-    while (split < 8 && uint64_t(n) / 8 * split * 2 <= 8192)
+    while (split < 8 && uint64_t(n) / 8 * split * 2 <= 2048)
         split *= 2;
     return split;
 }
@@ -1602,11 +1606,12 @@ uint32_t rows_split(uint32_t n)
 // Clusters per wave, one after the other: fewer workgroups copy the table and
 // add their histogram to the counts, and a cluster's first loads overlap its
 // predecessor's pair work.  1,048,576 points: one 0.78 ms, two 0.65, four 0.66,
-// eight 0.76 (the last waves run longer); one while two would leave less than
-// two rounds of resident waves (6 x 1024).
+// eight 0.76 (the last waves run longer); 60,000 points, r_max = 3, one call:
+// one 78 us, two 63.  One while there is less than one round of resident waves
+// (6 x 1024) of them: 30,000 points, r_max = 5: one 64, two 81 us.
 uint32_t rows_per_wave(uint64_t items)
 {
-    return items >= 4 * 6144 ? 2 : 1;
+    return items >= 6144 ? 2 : 1;
 }
 
 int launch_rows(const DevBox& db, const DevGrid& g, const DevGrid* gq, const int dims[3], int R, int F, uint32_t n,

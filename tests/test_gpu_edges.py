@@ -178,11 +178,12 @@ def test_rdf_routes_of_query_points(oracle, is2D, n, n_query, r_max, kernel):
                 assert any(kernel in name for name in ran), ran
 
 
-@pytest.mark.parametrize("n_query", [8192, 16384, 16385, 32768, 32769, 65537, 196608, 200001])
+@pytest.mark.parametrize("n_query", [2055, 2056, 4103, 4104, 8199, 8200, 49151, 49152, 200001])
 def test_rdf_row_clusters_of_query_points(oracle, n_query):
-    """Row clusters of distinct query points on both sides of the sizes at which
-    8, 4, 2 waves share a cluster and at which a wave takes two."""
-    n, r_max = 3000, 2.4
+    """Row clusters of distinct query points, and of the points themselves, on
+    both sides of the sizes at which 8, 4, 2 waves share a cluster and at
+    which a wave takes two."""
+    n, r_max = 3000, 2.5
     box = Box.cube(14.5)
     both = ((np.random.default_rng(n_query).random((n + n_query, 3)) - 0.5) * 14.49).astype(np.float32)
     pts, q = both[:n], both[n:]
@@ -191,6 +192,9 @@ def test_rdf_row_clusters_of_query_points(oracle, n_query):
     counts, ran = _rdf_kernels(lambda: rdf.compute((box, pts), query_points=q).bin_counts)
     npt.assert_array_equal(counts, ref)
     assert any("rdf_est_kernel" in name for name in ran), ran
+    box, pts = _uniform(n_query, seed=n_query)
+    ref = oracle.rdf_accumulate(_bt(box), pts, pts, 80, 1.5, exclude_ii=True, nthreads=16)
+    npt.assert_array_equal(freud_amd.density.RDF(80, 1.5).compute((box, pts)).bin_counts, ref)
 
 
 @pytest.mark.parametrize("which", ["points", "query_points", "both"])
