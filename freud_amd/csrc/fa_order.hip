@@ -1393,7 +1393,7 @@ __global__ void uf_union_kernel(uint64_t nb, const uint32_t* __restrict__ nbr, c
         return;
     uint2 const ij = reinterpret_cast<const uint2*>(nbr)[e];
     uint32_t a = ij.x, c = ij.y;
-    // the trees are flat after the jumps that precede this pass: most bonds
+    // the trees are flat after the rounds that precede this pass: most bonds
     // already have one parent at both ends
     if (parent[a] == parent[c])
         return;
@@ -1417,11 +1417,28 @@ __global__ void uf_union_kernel(uint64_t nb, const uint32_t* __restrict__ nbr, c
     }
 }
 
+// One hooking round (Shiloach and Vishkin, 1982) over every stride-th bond from
+// `first` on: the larger of the ends' parents takes the smaller as its parent.
+// Parents only get smaller and stay in the component, so the forest stays
+// valid.  Where several bonds hook one parent the smallest wins and the others'
+// links are left to later passes; the union pass sees to every bond.
+__global__ void uf_hook_roots_kernel(uint64_t nb, const uint32_t* __restrict__ nbr, const uint8_t* __restrict__ keep,
+                                     uint32_t* parent, uint32_t stride, uint32_t first)
+{
+    uint64_t const e = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) * stride + first;
+    if (e >= nb || (keep && !keep[e]))
+        return;
+    uint2 const ij = reinterpret_cast<const uint2*>(nbr)[e];
+    uint32_t const a = parent[ij.x], c = parent[ij.y];
+    uint32_t const hi = max(a, c), lo = min(a, c);
+    if (lo < parent[hi])
+        atomicMin(&parent[hi], lo);
+}
+
 // One round of pointer jumping, parent <- its third ancestor (three hops), so
 // that the distance to a point's parent grows at least fourfold per round.
 // Parallel hooking can leave long chains (bonds (i, i+1) processed together
-// hook i+1 under i for every i); ceil(log4 n) + 1 rounds bring every point
-// next to its root, so the flatten below walks at most a step or two.
+// hook i+1 under i for every i).
 // Parents only move to ancestors, so the in-place updates are safe.
 __global__ void uf_jump_kernel(uint32_t n, uint32_t* parent)
 {
@@ -2126,17 +2143,33 @@ int fa_cluster(uint32_t n, const fa_nlist* nl, const uint8_t* d_keep, uint32_t* 
         FA_KLAUNCH(uf_hook_min_kernel, dim3(blocks), dim3(kBlock), (size_t(cap) * 5 + 7) & ~size_t(7), s, n,
                    nl->neighbors, nl->offsets, d_keep, parent, cap);
     }
-    // The hooked chains lead to smaller indices bond by bond; three jumps bring
-    // those of up to 64 links under their roots (2,097,152 points: 6 us each, and
-    // the union pass 0.54 -> 0.34 ms).
-    if (nl->num_bonds)
-        for (int r = 0; r < 3; ++r)
-            FA_KLAUNCH(uf_jump_kernel, dim3(blocks), dim3(kBlock), 0, s, n, parent);
-    if (nl->num_bonds)
-        FA_KLAUNCH(uf_union_kernel, dim3(unsigned((nl->num_bonds + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                           nl->num_bonds, nl->neighbors, d_keep, parent);
-    for (uint64_t span = 1; span < n; span *= 4)
-        FA_KLAUNCH(uf_jump_kernel, dim3(blocks), dim3(kBlock), 0, s, n, parent);
+    // The union pass is the slower the more trees it finds and the longer the
+    // chains in which it hangs their roots onto each other (a thread walks them
+    // by itself, and how long they get is a matter of timing).  Hooking rounds
+    // over some two bonds per point, with two jumps after each, leave it few of
+    // either: one round where bonds are few, two where the launches count
+    // (2,000 points with 33 bonds each: one 237, two 91), three elsewhere.  Whole
+    // call in us with three jumps before the union, with none, and now: 100,000
+    // lattice points with 11 bonds each 693, 411, 88; with 4 279, 238, 102;
+    // 100,000 random points with 8 bonds each 1103, 1469, 202; half crystal, half
+    // liquid, 2,097,152 points (SolidLiquid) 2812, 2854, 2700.
+    if (uint64_t const nb = nl->num_bonds)
+    {
+        int const rounds = nb < 3 * uint64_t(n) ? 1 : n <= 8192 ? 2 : 3;
+        uint32_t const stride = uint32_t(std::clamp<uint64_t>(nb / (2 * uint64_t(n)), 1, 8));
+        unsigned const some = unsigned((nb / stride + kBlock) / kBlock); // covers ceil(nb / stride) bonds
+        auto jump = [&] { FA_KLAUNCH(uf_jump_kernel, dim3(blocks), dim3(kBlock), 0, s, n, parent); };
+        jump();
+        for (int r = 0; r < rounds; ++r)
+        {
+            FA_KLAUNCH(uf_hook_roots_kernel, dim3(some), dim3(kBlock), 0, s, nb, nl->neighbors, d_keep, parent, stride,
+                       uint32_t(r) % stride);
+            jump();
+            jump();
+        }
+        FA_KLAUNCH(uf_union_kernel, dim3(unsigned((nb + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, nb, nl->neighbors,
+                   d_keep, parent); // few and short chains: the flatten walks them
+    }
     unsigned const ufblocks = (n + kUfBlock - 1) / kUfBlock;
     FA_KLAUNCH(uf_flatten_kernel, dim3(ufblocks), dim3(kUfBlock), 0, s, n, parent, root, size);
     FA_HIP(hipMemsetAsync(counter, 0, sizeof(uint32_t), s));

@@ -496,3 +496,36 @@ def test_cluster_chains(n, parts):
     cl = freud_amd.cluster.Cluster().compute((box, pts), neighbors=nl)
     assert cl.num_clusters == len(count)
     npt.assert_array_equal(cl.cluster_idx, rank[inverse])
+
+
+@pytest.mark.parametrize("store", ["random", "sorted", "lattice"])
+@pytest.mark.parametrize("n", [500, 8192, 8193, 32000])
+@pytest.mark.parametrize("bonds", [0.8, 2.5, 4, 9, 40])
+def test_cluster_percolation(oracle, store, n, bonds):
+    """Below, at and above percolation, with one to three hooking rounds over
+    every, every other or every eighth bond, points stored in random and in
+    spatial order: labels and sizes equal the oracle's, with and without
+    a mask of kept bonds."""
+    box, pts = _uniform(n, seed=n)
+    if store == "sorted":
+        pts = pts[np.lexsort((pts[:, 0] // 2, pts[:, 1] // 2, pts[:, 2] // 2))]
+    elif store == "lattice":
+        m = int(np.ceil((n / 4) ** (1 / 3)))
+        a = np.arange(m)
+        grid = np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 1, 3)
+        frac = (grid + np.array([[0, 0, 0], [0.5, 0.5, 0], [0.5, 0, 0.5], [0, 0.5, 0.5]])).reshape(-1, 3)[:n]
+        frac = frac + np.random.default_rng(1).standard_normal(frac.shape) * 0.05
+        box = Box.cube(m * 4 ** (1 / 3))
+        pts = np.ascontiguousarray(box.wrap((frac - m / 2) * 4 ** (1 / 3)), np.float32)
+    r = (bonds / 4.18879) ** (1 / 3)
+    nl = freud_amd.AABBQuery(box, pts).query(pts, dict(r_max=r, exclude_ii=True)).toNeighborList()
+    ref_nl = oracle.query(_bt(box), pts, pts, dict(r_max=r, exclude_ii=True), nthreads=16)
+    cl = freud_amd.cluster.Cluster().compute((box, pts), neighbors=nl)
+    idx, num = oracle.cluster(len(pts), ref_nl["ij"])
+    npt.assert_array_equal(cl.cluster_idx, idx)
+    assert cl.num_clusters == num
+    st = freud_amd.order.Steinhardt(6).compute((box, pts), neighbors=nl)
+    sl = freud_amd.order.SolidLiquid(6, 0.4, 2).compute((box, pts), neighbors=nl)
+    ref = oracle.solidliquid(ref_nl, st.particle_harmonics, st.ql, 6, 0.4, 2, normalize_q=True)
+    if not np.any(np.abs(ref["ql_ij"] - 0.4) < 1e-6):
+        npt.assert_array_equal(sl.cluster_idx, ref["cluster_idx"])
