@@ -88,6 +88,9 @@ constexpr int kKnnVariants = 2 * kKnnCellSizes;
 // Keys of the batched analyses are offset by this (the single-frame keys are
 // small integers around 0).
 constexpr int kBatchTuneKey = 1000;
+// Offset of the self RDF's keys for the calls that take the exact pair kernel
+// (keys themselves stay below 60: fewer than 2^27 points in an r^3 volume).
+constexpr int kRdfExactTuneKey = 300;
 bool tuning_enabled();
 int tuned_variant(int analysis, int key); // -1 when not tuned yet
 void record_variant(int analysis, int key, int variant);

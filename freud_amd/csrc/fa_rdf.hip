@@ -2299,8 +2299,13 @@ int fa_rdf_accumulate_query(fa_nq* nq, const float* d_query_points, uint32_t n_q
         // row-cluster kernel; the cell size (r_max / R) is picked by the autotuner
         RowsArgs ra{nq, qmax_sq, qmin_sq, &est, T, bins, r_min, inv_width, q_r_max};
         double const density = double(nq->n) / double(fa::box_volume(nq->box));
-        int const key = fa::tune_key(density, q_r_max);
+        // the two pair kernels cost differently over the cell shapes: a class each.  A
+        // caller's preset holds for both.
+        int const est_key = fa::tune_key(density, q_r_max);
+        int const key = est.hi > 0.0f ? est_key : est_key + fa::kRdfExactTuneKey;
         int variant = fa::tuned_variant(fa::TUNE_RDF_SELF, key);
+        if (variant < 0 && fa::variant_preset(fa::TUNE_RDF_SELF, est_key))
+            variant = fa::tuned_variant(fa::TUNE_RDF_SELF, est_key);
         bool handled = false;
         if (variant < 0 && fa::tuning_enabled())
         {

@@ -407,6 +407,36 @@ def _rdf_variants(box, n, r_max):
         _lib.tune_load({(1, key): before.get((1, key), -1)})
 
 
+def test_rdf_tuned_per_kernel(oracle):
+    """The estimate kernel and the exact one record a cell shape each, whichever
+    runs first; a preset under the class's key holds for both."""
+    from freud_amd import _lib
+
+    box = Box.cube(20)
+    pts = ((np.random.default_rng(9).random((9000, 3)) - 0.5) * 20).astype(np.float32)
+    key = int(np.floor(2.0 * np.log2(len(pts) / box.volume * 2.5 ** 3) + 0.5))
+    counts = {bins: oracle.rdf_accumulate(_bt(box), pts, pts, bins, 2.5, exclude_ii=True, nthreads=8)
+              for bins in (200, 600)}
+    before = _lib.tune_table()
+    try:
+        for order in ((600, 200), (200, 600)):
+            _lib.tune_load({(1, key): -1, (1, key + 300): -1})
+            for bins, other in ((order[0], False), (order[1], True)):
+                rdf = freud_amd.density.RDF(bins, 2.5).compute((box, pts))
+                npt.assert_array_equal(rdf.bin_counts, counts[bins])
+                table = _lib.tune_table()
+                keys = {200: (1, key), 600: (1, key + 300)}
+                assert (keys[bins] in table) and (keys[800 - bins] in table) == other
+        _lib.tune_load({(1, key): 4, (1, key + 300): -1})
+        for bins in (600, 200):
+            rdf = freud_amd.density.RDF(bins, 2.5).compute((box, pts))
+            npt.assert_array_equal(rdf.bin_counts, counts[bins])
+        table = _lib.tune_table()
+        assert table[(1, key)] == 4 and (1, key + 300) not in table
+    finally:
+        _lib.tune_load({(1, k): before.get((1, k), -1) for k in (key, key + 300)})
+
+
 def test_rdf_lj_golden():
     # tests/integration/test_reader_integrations.py:27-40 of the reference
     traj = open_gsd(os.path.join(GOLDEN, "lj.gsd"))
