@@ -450,8 +450,12 @@ int tune(fa_batch* b)
     }
     if (do_rdf(b))
     {
-        int const key = fa::tune_key(density, b->plan.rdf_r_max) + fa::kBatchTuneKey;
+        // a class for each pair kernel, as in the single-frame RDF
+        int const est_key = fa::tune_key(density, b->plan.rdf_r_max) + fa::kBatchTuneKey;
+        int const key = b->rs.est_hi > 0.0f ? est_key : est_key + fa::kRdfExactTuneKey;
         int v = fa::tuned_variant(fa::TUNE_RDF_SELF, key);
+        if (v < 0 && fa::variant_preset(fa::TUNE_RDF_SELF, est_key))
+            v = fa::tuned_variant(fa::TUNE_RDF_SELF, est_key);
         if (v < 0 && fa::tuning_enabled())
         {
             float best = 0;

@@ -179,6 +179,30 @@ def test_batch_rdf_every_launch_shape(oracle):
         _lib.tune_load({(1, key): before.get((1, key), -1)})
 
 
+def test_batch_rdf_tuned_per_kernel():
+    """A batch of more bins than the estimate kernel takes records its cell shape
+    apart from the others; a preset under the class's key holds for both."""
+    from freud_amd import _lib
+
+    frames = _frames(seed=12)
+    pts_total, vol = sum(len(p) for _, p in frames), sum(b.volume for b, _ in frames)
+    key = int(np.floor(2.0 * np.log2(pts_total / vol * R_RDF ** 3) + 0.5)) + 1000
+
+    def run(bins):
+        freud_amd.batch.TrajectoryBatch(frames, rdf_bins=bins, rdf_r_max=R_RDF).compute(use_graph=False)
+        return {k for a, k in _lib.tune_table() if a == 1 and k in (key, key + 300)}
+
+    before = _lib.tune_table()
+    try:
+        _lib.tune_load({(1, key): -1, (1, key + 300): -1})
+        assert run(600) == {key + 300}
+        assert run(100) == {key, key + 300}
+        _lib.tune_load({(1, key): 2, (1, key + 300): -1})
+        assert run(600) == {key} and run(100) == {key}
+    finally:
+        _lib.tune_load({(1, k): before.get((1, k), -1) for k in (key, key + 300)})
+
+
 def test_batched_trajectory_full_size(oracle):
     """The batched trajectory at its benchmark size: 256 frames of 10k-200k
     points (log-uniform; liquid, jittered FCC and BCC; cubic and triclinic),
