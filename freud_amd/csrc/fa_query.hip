@@ -31,8 +31,13 @@ constexpr int kBlock = 256;
 // largest LDS key staging per block; of a ball query's emission, such that four
 // blocks fit on a CU with its other LDS
 constexpr int kKeyBytes = 32768, kBallKeyBytes = 32256;
-// query points up to which a ball query, and a kNN query (whose per-thread
-// search the tuner fits to larger systems), takes one wave per point
+// Query points up to which a ball query, and a kNN query (whose per-thread
+// search the tuner fits to larger systems), takes one wave per point.  Whole
+// query in us, waves against threads: ball, r_max = 1.4, 32,768 points 116 and
+// 123, 70,000 171 and 159; k = 12 nearest, 8,192 uniform points 82 and 279,
+// 70,000 219 and 248.  The kNN line lies where irregular systems, whose cells
+// the tuner fits and the waves' are not, still gain: points of a droplet in a
+// large box, k = 6, 8,192 of them 180 and 191, 16,384 279 and 164.
 constexpr uint32_t kWaveQueries = 32768;
 constexpr uint32_t kWaveKnnQueries = 8192;
 // keys per point that the one-walk ball query stages in LDS (32 KB per block)
@@ -1084,8 +1089,8 @@ __global__ __launch_bounds__(kBlock) void knn_stage_kernel(DevBox b, DevGrid g, 
 // comparing every key with every other.  The candidates, their arithmetic and
 // the selected order are those of the per-thread kernels.
 // 4,096 points, k = 12: search 154 -> 19 us; 20,000 points, r_max = 1.5:
-// walk 47 -> 37 us, emission 93 -> 9 us.  At 100,000 points the per-thread
-// kernels are the faster ones.
+// walk 47 -> 37 us, emission 93 -> 9 us (see kWaveQueries for the line to the
+// per-thread kernels).
 constexpr uint32_t kWaveKeys = 256; // keys a wave keeps (2 KB of LDS)
 constexpr uint32_t kWaves = kBlock / 64;
 

@@ -956,8 +956,7 @@ __device__ inline void rows_est(const DevBox& b, const DevGrid& g, float4 pa, in
         if (bl > a && bl < na)
             est_exact<WAVE_HIST>(B, x, 2u);
     }
-    // the cluster's points, in vector registers (24 more scalar ones would
-    // spill, and be read back with VALU instructions); NaN past na
+    // the cluster's points, in scalar registers; NaN past na
     float qx[8], qy[8], qz[8];
 #pragma unroll
     for (uint32_t k = 0; k < 8; ++k)

@@ -125,8 +125,8 @@ BOXES = {
                                               (1, 3.0, 0.0)])
 def test_rdf_estimate_borders(oracle, name, n, bins, r_max, r_min):
     """Bin counts bit for bit, self and with distinct query points, on both
-    sides of the estimate table's largest bin count, over few and many
-    clusters, dense and nearly empty boxes."""
+    sides of the estimate table's largest bin count, in dense and nearly empty
+    boxes."""
     box = BOXES[name]
     rng = np.random.default_rng(n + bins)
     pts = np.ascontiguousarray(box.make_absolute(rng.random((n, 3)).astype(np.float32)), np.float32)
@@ -268,9 +268,10 @@ def test_scan_totals_beyond_32_bits(n, largest):
     npt.assert_array_equal(d_segments.numpy()[:n], np.where(counts > 0, offsets[:-1], 0))
 
 
-@pytest.mark.parametrize("n", [2, 4096, 8192, 8193, 40001])
+@pytest.mark.parametrize("n", [2, 4096, 8192, 8193, 40001, (1 << 22) + 5])
 def test_query_segments(n):
-    """Offsets, counts and segments (0 for points without bonds) of a query."""
+    """Offsets, counts and segments (0 for points without bonds) of a query, up
+    to more points than the library's own scan takes."""
     box, pts = _uniform(n, density=0.3, seed=n)
     for args in (dict(r_max=1.0, exclude_ii=True), dict(num_neighbors=1, r_max=0.9, exclude_ii=True)):
         nl = freud_amd.AABBQuery(box, pts).query(pts, args).toNeighborList()
@@ -424,8 +425,8 @@ def test_wave_ball_query_of_clumps(oracle, by_distance):
 @pytest.mark.parametrize("kind", ["aabb", "linkcell", "cellquery"])
 @pytest.mark.parametrize("bonds", [7, 15, 30, 37, 45])
 def test_large_ball_queries_by_bond_count(oracle, kind, bonds):
-    """More points than the wave queries take, on both sides of the register
-    sorts (16, 32, 48 keys) and of the LDS and device-memory key stages, with a
+    """More points than the wave queries take, on both sides of the lists that
+    the sort networks hold (16, 32, 48 keys) and of the walk's key stage, with a
     clump past every stage; consecutive and scattered storage orders."""
     n, side = 33000, 32.08
     box = Box.cube(side)
