@@ -16,11 +16,12 @@
 //
 // RDF over AABB queries (up to kEstMaxBins bins over the query's own range): the
 // pair kernel of rows_est below, over row clusters, on estimates of r_sq that
-// fall back to the reference's arithmetic near a bin's threshold.
+// fall back to the reference's arithmetic near a bin's threshold.  Query points
+// of their own take it, or one wave or thread each, as cross_route says.
 //
 // Self RDF with more bins or a narrower query (query points == points, AABB
-// formula, all points inside the box): a cluster-pair kernel over cells at least r_max/2 wide; each wave takes a
-// cluster of up to 8 cell-ordered points and its 64 lanes test 8 x 8 pairs per
+// formula, all points inside the box): a cluster-pair kernel over cells at least
+// r_max/2 wide; each wave takes a cluster of up to 8 cell-ordered points and its 64 lanes test 8 x 8 pairs per
 // step against 8-point chunks of the 5x5x5 stencil cells.  For two cells related
 // without a periodic shift the AABB formula gives bitwise-equal r_sq for (i,j)
 // and (j,i) (x - y == -(y - x) in IEEE arithmetic), so such pairs are evaluated
