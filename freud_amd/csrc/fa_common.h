@@ -490,6 +490,67 @@ __device__ inline void for_each_candidate(const DevBox& b, const DevGrid& g, flo
 }
 
 // Calls f(valid, j, code, r_sq) with all lanes for 64 candidates at a time of
+// the wave's ranges of the cell order, laid end to end: lane t's holds len points
+// from beg, whose cells lie shift box lengths from the box, 10 bits per axis
+// (biased by 512: searches end near half a box length, so that it is a few at
+// most; the query's own image offset w, of any size, is added here).
+template<typename F>
+__device__ inline void wave_ranges(const DevBox& b, const DevGrid& g, float qx, float qy, float qzz, const int w[3],
+                                   bool outside, uint32_t beg, uint32_t len, int shift, F&& f)
+{
+    uint32_t const lane = threadIdx.x & 63u;
+    uint32_t e = len; // inclusive scan over the lanes
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+    {
+        uint32_t const y = __shfl_up(e, d);
+        if (lane >= uint32_t(d))
+            e += y;
+    }
+    uint32_t const p = e - len, sh = beg - p;
+    uint32_t const tot = uint32_t(__builtin_amdgcn_readlane(int(e), 63));
+    uint64_t live = __builtin_amdgcn_ballot_w64(len > 0u);
+    for (uint32_t v0 = 0; v0 < tot; v0 += 64u)
+    {
+        uint32_t const v = v0 + lane;
+        uint32_t pos = 0u;
+        int code3 = 0;
+        for (uint64_t m = live; m; m &= m - 1u)
+        {
+            int const r = __builtin_ctzll(m);
+            uint32_t const sp = uint32_t(__builtin_amdgcn_readlane(int(p), r));
+            if (sp >= v0 + 64u)
+                break;
+            uint32_t const p2 = v + uint32_t(__builtin_amdgcn_readlane(int(sh), r));
+            int const s2 = __builtin_amdgcn_readlane(shift, r);
+            pos = v >= sp ? p2 : pos;
+            code3 = v >= sp ? s2 : code3;
+            if (uint32_t(__builtin_amdgcn_readlane(int(e), r)) <= v0 + 64u)
+                live &= ~(uint64_t(1) << r);
+        }
+        bool valid = v < tot;
+        float4 const pj = g.cpos[valid ? pos : 0u];
+        int n0 = 512 - (code3 & 1023) - w[0], n1 = 512 - ((code3 >> 10) & 1023) - w[1];
+        int n2 = 512 - ((code3 >> 20) & 1023) - w[2];
+        if (outside)
+        {
+            int wj[3];
+            unpack_wrap(g.wrapc[valid ? pos : 0u], wj);
+            n0 += wj[0];
+            n1 += wj[1];
+            n2 = b.is2D ? 0 : n2 + wj[2];
+        }
+        valid = valid && n0 >= -1 && n0 <= 1 && n1 >= -1 && n1 <= 1 && n2 >= -1 && n2 <= 1;
+        int const code = valid ? (n0 + 1) * 9 + (n1 + 1) * 3 + (n2 + 1) : 13;
+        float const pz = b.is2D ? 0.0f : pj.z;
+        float const rx = pj.x - (qx + b.img[code][0]);
+        float const ry = pj.y - (qy + b.img[code][1]);
+        float const rz = pz - (qzz + b.img[code][2]);
+        f(valid, __float_as_uint(pj.w), code, (rx * rx + ry * ry) + rz * rz);
+    }
+}
+
+// Calls f(valid, j, code, r_sq) with all lanes for 64 candidates at a time of
 // the stencil of half-width R around q (AABB formula; ring_only: its cells at
 // Chebyshev offset R, R > 0), as for_each_candidate visits them; lanes without
 // a candidate get valid = false.
@@ -509,9 +570,6 @@ __device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float 
     for (int c0 = 0; c0 < ncell; c0 += 64)
     {
         uint32_t beg = 0u, len = 0u;
-        // the cell's shift in box lengths per axis, 10 bits each (biased by 512:
-        // searches end near half a box length, so that it is a few at most); the
-        // query's own image offset, of any size, is added below
         int shift = 0;
         int const t = c0 + int(lane);
         if (t < ncell)
@@ -548,55 +606,50 @@ __device__ inline void wave_candidates(const DevBox& b, const DevGrid& g, float 
                 shift = (sh[0] + 512) | ((sh[1] + 512) << 10) | ((sh[2] + 512) << 20);
             }
         }
-        uint32_t e = len; // inclusive scan over the lanes
+        wave_ranges(b, g, qx, qy, qzz, w, outside, beg, len, shift, f);
+    }
+}
+
+// wave_candidates over the stencil of half-width RX along x and R across, by the
+// unbroken pieces of its rows of cells: cells narrow along x would take a lane
+// each for a few points.
+template<typename F>
+__device__ inline void wave_row_candidates(const DevBox& b, const DevGrid& g, float qx, float qy, float qz, int R,
+                                           int RX, F&& f)
+{
+    int c[3], w[3];
+    cell_of(b, g.dim, qx, qy, qz, c, w);
+    float const qzz = b.is2D ? 0.0f : qz;
+    int const side = 2 * R + 1, rows = b.is2D ? side : side * side;
+    // a row starts in the box length first of its cells and breaks at each next
+    int const first = floor_div(c[0] - RX, g.dim[0]), parts = floor_div(c[0] + RX, g.dim[0]) - first + 1;
+    bool const outside = *g.outside;
+    uint32_t const lane = threadIdx.x & 63u;
+    for (int t0 = 0; t0 < rows * parts; t0 += 64)
+    {
+        uint32_t beg = 0u, len = 0u;
+        int shift = 0;
+        int const t = t0 + int(lane);
+        if (t < rows * parts)
+        {
+            int const row = t / parts, sx = first + t % parts;
+            int const uy = c[1] + row % side - R, uz = b.is2D ? c[2] : c[2] + row / side - R;
+            int const sy = floor_div(uy, g.dim[1]), sz = floor_div(uz, g.dim[2]);
+            int const sh[3] = {sx, sy, sz};
+            bool in = true;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1)
-        {
-            uint32_t const y = __shfl_up(e, d);
-            if (lane >= uint32_t(d))
-                e += y;
-        }
-        uint32_t const p = e - len, sh = beg - p;
-        uint32_t const tot = uint32_t(__builtin_amdgcn_readlane(int(e), 63));
-        uint64_t live = __builtin_amdgcn_ballot_w64(len > 0u);
-        for (uint32_t v0 = 0; v0 < tot; v0 += 64u)
-        {
-            uint32_t const v = v0 + lane;
-            uint32_t pos = 0u;
-            int code3 = 0;
-            for (uint64_t m = live; m; m &= m - 1u)
+            for (int k = 0; k < 3; ++k)
+                in = in && (outside || (-w[k] - sh[k] >= -1 && -w[k] - sh[k] <= 1));
+            if (in)
             {
-                int const r = __builtin_ctzll(m);
-                uint32_t const sp = uint32_t(__builtin_amdgcn_readlane(int(p), r));
-                if (sp >= v0 + 64u)
-                    break;
-                uint32_t const p2 = v + uint32_t(__builtin_amdgcn_readlane(int(sh), r));
-                int const s2 = __builtin_amdgcn_readlane(shift, r);
-                pos = v >= sp ? p2 : pos;
-                code3 = v >= sp ? s2 : code3;
-                if (uint32_t(__builtin_amdgcn_readlane(int(e), r)) <= v0 + 64u)
-                    live &= ~(uint64_t(1) << r);
+                int const base = ((uz - sz * g.dim[2]) * g.dim[1] + (uy - sy * g.dim[1])) * g.dim[0];
+                int const x0 = max(c[0] - RX - sx * g.dim[0], 0), x1 = min(c[0] + RX - sx * g.dim[0], g.dim[0] - 1);
+                beg = g.cstart[base + x0];
+                len = g.cstart[base + x1 + 1] - beg;
+                shift = (sh[0] + 512) | ((sh[1] + 512) << 10) | ((sh[2] + 512) << 20);
             }
-            bool valid = v < tot;
-            float4 const pj = g.cpos[valid ? pos : 0u];
-            int n0 = 512 - (code3 & 1023) - w[0], n1 = 512 - ((code3 >> 10) & 1023) - w[1];
-            int n2 = 512 - ((code3 >> 20) & 1023) - w[2];
-            if (outside)
-            {
-                int wj[3];
-                unpack_wrap(g.wrapc[valid ? pos : 0u], wj);
-                n0 += wj[0];
-                n1 += wj[1];
-                n2 = b.is2D ? 0 : n2 + wj[2];
-            }
-            valid = valid && n0 >= -1 && n0 <= 1 && n1 >= -1 && n1 <= 1 && n2 >= -1 && n2 <= 1;
-            int const code = valid ? (n0 + 1) * 9 + (n1 + 1) * 3 + (n2 + 1) : 13;
-            float const pz = b.is2D ? 0.0f : pj.z;
-            float const rx = pj.x - (qx + b.img[code][0]);
-            float const ry = pj.y - (qy + b.img[code][1]);
-            float const rz = pz - (qzz + b.img[code][2]);
-            f(valid, __float_as_uint(pj.w), code, (rx * rx + ry * ry) + rz * rz);
         }
+        wave_ranges(b, g, qx, qy, qzz, w, outside, beg, len, shift, f);
     }
 }
 

@@ -1298,9 +1298,10 @@ __global__ __launch_bounds__(kBlock, 6) void rdf_est_kernel(DevBox b, DevGrid g,
     hist_epilogue<true>(words + 2 * kEstCells + 1, nbins, counts);
 }
 
-// The systems rdf_est_kernel leaves out: one thread per query point walks its
-// stencil with every point's own image offset, each ordered pair once.
-template<bool HALF>
+// The systems rdf_est_kernel leaves out: one wave per query point (WAVES), or one
+// thread, walks its stencil with every point's own image offset, each ordered
+// pair once.
+template<bool HALF, bool WAVES>
 __global__ __launch_bounds__(kBlock) void rdf_outside_kernel(DevBox b, DevGrid g, DevGrid gq, uint32_t nq, int R,
                                                              int RX, float lo, float hi, const float* __restrict__ T,
                                                              uint32_t nbins, float vmin, float inv_width,
@@ -1312,17 +1313,25 @@ __global__ __launch_bounds__(kBlock) void rdf_outside_kernel(DevBox b, DevGrid g
     for (uint32_t t = threadIdx.x; t < nbins; t += blockDim.x)
         hist_only[t] = 0u;
     __syncthreads();
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < nq; t += gridDim.x * blockDim.x)
+    constexpr uint32_t kPer = WAVES ? 64u : 1u; // threads per query point
+    uint32_t const stride = gridDim.x * (kBlock / kPer);
+    for (uint32_t t = (blockIdx.x * kBlock + threadIdx.x) / kPer; t < nq; t += stride)
     {
         float4 const q = gq.cpos[t];
         uint32_t const qi = __float_as_uint(q.w);
-        fa::for_each_candidate<AABB_FORMULA>(
-            b, g, q.x, q.y, q.z, R, false,
-            [&](uint32_t j, float, float, float, float r_sq, int) {
-                if (!(HALF && j == qi) && r_sq >= lo && r_sq < hi)
-                    atomicAdd(&hist_only[bin_in_range(r_sq, T, nbins, vmin, inv_width)], 1u);
-            },
-            RX);
+        auto count = [&](uint32_t j, float r_sq) {
+            if (!(HALF && j == qi) && r_sq >= lo && r_sq < hi)
+                atomicAdd(&hist_only[bin_in_range(r_sq, T, nbins, vmin, inv_width)], 1u);
+        };
+        if constexpr (WAVES)
+            fa::wave_row_candidates(b, g, q.x, q.y, q.z, R, RX, [&](bool valid, uint32_t j, int, float r_sq) {
+                if (valid)
+                    count(j, r_sq);
+            });
+        else
+            fa::for_each_candidate<AABB_FORMULA>(
+                b, g, q.x, q.y, q.z, R, false,
+                [&](uint32_t j, float, float, float, float r_sq, int) { count(j, r_sq); }, RX);
     }
     hist_epilogue<true>(hist_only, nbins, counts);
 }
@@ -1614,8 +1623,25 @@ uint32_t rows_per_wave(uint64_t items)
     return items >= 6144 ? 2 : 1;
 }
 
+// Whether rdf_outside_kernel gives each of n query points a wave.  A thread's
+// walk takes as long for few query points as for all the chip's threads, a
+// wave's is shorter by its 64 lanes but has a setup of its own: waves by the
+// candidates per query point.  Density 0.8, one point off the box, ms of one call
+// with threads and with waves: r_max = 1.2 (20 candidates): 4,000 points 0.099,
+// 0.047, 50,000 0.103, 0.099, 100,000 0.109, 0.155; r_max = 2.5 (160): 100,000
+// 0.253, 0.229, 300,000 0.401, 0.622; r_max = 5 (1,300): 4,000 1.189, 0.066,
+// 300,000 1.79, 1.59, 1,000,000 5.28, 5.23.
+bool outside_waves(uint32_t n, uint32_t n_points, const int dims[3], int R, int F, bool is2D)
+{
+    double const rows = is2D ? 2.0 * R + 1.0 : (2.0 * R + 1.0) * (2.0 * R + 1.0);
+    double const cells = double(dims[0]) * dims[1] * dims[2];
+    return n <= 50000.0 + 320.0 * rows * (2.0 * R * F + 1.0) * n_points / cells;
+}
+
+// The row clusters of n query points (of gq, or those of g if null) against the
+// n_points points of g.
 int launch_rows(const DevBox& db, const DevGrid& g, const DevGrid* gq, const int dims[3], int R, int F, uint32_t n,
-                const RowsBuffers& B, float qmax_sq, float qmin_sq, const EstRange& est, const float* T, uint32_t bins,
+                uint32_t n_points, const RowsBuffers& B, float qmax_sq, float qmin_sq, const EstRange& est, const float* T, uint32_t bins,
                 float r_min, float inv_width, uint32_t* d_counts)
 {
     hipStream_t s = fa::stream();
@@ -1665,14 +1691,19 @@ int launch_rows(const DevBox& db, const DevGrid& g, const DevGrid* gq, const int
         }
 #undef FA_EST
         FA_HIP(hipGetLastError());
+        bool const waves = outside_waves(n, n_points, dims, R, F, db.is2D);
         auto outside = [&](auto kern, const DevGrid& query_grid) {
             FA_PROF_BEGIN("rdf_outside_kernel");
-            hipLaunchKernelGGL(kern, dim3(std::min<unsigned>((n + kBlock - 1) / kBlock, 2048u)), dim3(kBlock),
+            unsigned const per_block = waves ? kBlock / 64 : kBlock;
+            hipLaunchKernelGGL(kern, dim3(std::min<unsigned>((n + per_block - 1) / per_block, 2048u)), dim3(kBlock),
                                sizeof(uint32_t) * bins, s, db, g, query_grid, n, R, R * F, est.lo, est.hi, T, bins,
                                r_min, inv_width, d_counts);
             FA_PROF_END();
         };
-        gq ? outside(rdf_outside_kernel<false>, *gq) : outside(rdf_outside_kernel<true>, g);
+        if (gq)
+            waves ? outside(rdf_outside_kernel<false, true>, *gq) : outside(rdf_outside_kernel<false, false>, *gq);
+        else
+            waves ? outside(rdf_outside_kernel<true, true>, g) : outside(rdf_outside_kernel<true, false>, g);
         FA_HIP(hipGetLastError());
         return FA_OK;
     }
@@ -1744,7 +1775,7 @@ int run_rows(const RowsArgs& a, RowVariant rv, uint32_t* d_counts, bool* handled
     B.nclus = static_cast<uint32_t*>(tmp);
     B.cl_off = B.nclus + (nrows + 1);
     B.table = reinterpret_cast<uint4*>(static_cast<char*>(tmp) + ((2 * rb + 15) & ~size_t(15)));
-    return launch_rows(nq->cur->dbox, nq->cur->dev(), nullptr, dims, rv.R, F, nq->n, B, a.qmax_sq, a.qmin_sq, *a.est,
+    return launch_rows(nq->cur->dbox, nq->cur->dev(), nullptr, dims, rv.R, F, nq->n, nq->n, B, a.qmax_sq, a.qmin_sq, *a.est,
                        a.T, a.bins, a.r_min, a.inv_width, d_counts);
 }
 
@@ -1813,7 +1844,7 @@ int run_cross_rows(fa_nq* nq, const float* d_query, uint32_t n_query, float q_r_
     B.cl_off = B.nclus + (nrows + 1);
     B.table = reinterpret_cast<uint4*>(static_cast<char*>(tmp) + ((2 * rb + 15) & ~size_t(15)));
     DevGrid const gq = qgrid.dev();
-    return launch_rows(nq->cur->dbox, nq->cur->dev(), &gq, dims, rv.R, F, n_query, B, qmax_sq, qmin_sq, est, T, bins,
+    return launch_rows(nq->cur->dbox, nq->cur->dev(), &gq, dims, rv.R, F, n_query, nq->n, B, qmax_sq, qmin_sq, est, T, bins,
                        r_min, inv_width, d_counts);
 }
 
@@ -2530,7 +2561,7 @@ int fa_rdf_accumulate_self_noalloc(const fa_box* box, const float* d_points, uin
     float const width = (r_max - r_min) / float(bins);
     float const inv_width = 1.0f / width;
     EstRange const est = est_range(D.est, D.first, D.last, q_r_max * q_r_max, q_r_min * q_r_min);
-    return launch_rows(db, g, nullptr, dims, rv.R, F, n, B, q_r_max * q_r_max, q_r_min * q_r_min, est, T, bins, r_min,
+    return launch_rows(db, g, nullptr, dims, rv.R, F, n, n, B, q_r_max * q_r_max, q_r_min * q_r_min, est, T, bins, r_min,
                        inv_width, d_counts);
 }
 

@@ -216,6 +216,33 @@ def test_rdf_points_outside_the_box(oracle, which):
     npt.assert_array_equal(rdf.compute((box, pts)).bin_counts, ref)
 
 
+@pytest.mark.parametrize("name, n, r", [("small", 300, 2.9), ("thin", 900, 1.9), ("square", 700, 3.0),
+                                        ("cube", 4000, 1.2), ("cube", 56000, 1.0), ("cube", 70000, 1.0)])
+def test_rdf_outside_routes(oracle, name, n, r):
+    """Systems off the box, a wave or a thread per point (from some 54,000 of
+    this density): rows of cells that wrap more than once, boxes of two
+    dimensions and tilted ones, points many boxes away; query points of their
+    own, few and many, with the points in the box or off it."""
+    box = {"small": Box(6.0, 6.0, 6.0, 0.2, -0.1, 0.15), "thin": Box(4.0, 30.0, 8.0),
+           "square": Box.square(26.0), "cube": Box.cube((n / 0.8) ** (1 / 3))}[name]
+    rng = np.random.default_rng(n)
+    inside = box.make_absolute(rng.random((n, 3)).astype(np.float32))
+    if box.is2D:
+        inside[:, 2] = 0
+    images = rng.integers(-3, 4, (n, 3))
+    images[::3] = 0
+    if box.is2D:
+        images[:, 2] = 0
+    off = box.unwrap(inside, images).astype(np.float32)
+    rdf = freud_amd.density.RDF(70, r)
+    ref = oracle.rdf_accumulate(_bt(box), off, off, 70, r, exclude_ii=True, nthreads=16)
+    npt.assert_array_equal(rdf.compute((box, off)).bin_counts, ref)
+    for pts, q in ((inside, off[::2]), (off, inside[: n // 3])):
+        q = np.ascontiguousarray(q)
+        ref = oracle.rdf_accumulate(_bt(box), pts, q, 70, r, exclude_ii=False, nthreads=16)
+        npt.assert_array_equal(rdf.compute((box, pts), query_points=q).bin_counts, ref)
+
+
 def test_rdf_query_ranges_inside_the_histogram(oracle):
     """A query radius inside the histogram's range cuts bins apart (exact
     kernel); index exclusion with distinct query points (general kernel)."""
