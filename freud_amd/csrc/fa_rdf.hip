@@ -1630,12 +1630,16 @@ uint32_t rows_per_wave(uint64_t items)
 // with threads and with waves: r_max = 1.2 (20 candidates): 4,000 points 0.099,
 // 0.047, 50,000 0.103, 0.099, 100,000 0.109, 0.155; r_max = 2.5 (160): 100,000
 // 0.253, 0.229, 300,000 0.401, 0.622; r_max = 5 (1,300): 4,000 1.189, 0.066,
-// 300,000 1.79, 1.59, 1,000,000 5.28, 5.23.
+// 300,000 1.79, 1.59, 1,000,000 5.28, 5.23.  In two dimensions a thread has only
+// five rows to walk: r_max = 1.5 (9): 5,000 0.050, 0.049, 20,000 0.052, 0.071;
+// r_max = 2.5 (26): 20,000 0.070, 0.071; r_max = 4 (66): 40,000 0.109, 0.081,
+// 80,000 0.108, 0.104.
 bool outside_waves(uint32_t n, uint32_t n_points, const int dims[3], int R, int F, bool is2D)
 {
     double const rows = is2D ? 2.0 * R + 1.0 : (2.0 * R + 1.0) * (2.0 * R + 1.0);
     double const cells = double(dims[0]) * dims[1] * dims[2];
-    return n <= 50000.0 + 320.0 * rows * (2.0 * R * F + 1.0) * n_points / cells;
+    double const candidates = rows * (2.0 * R * F + 1.0) * n_points / cells;
+    return n <= (is2D ? 1000.0 * candidates : 50000.0 + 320.0 * candidates);
 }
 
 // The row clusters of n query points (of gq, or those of g if null) against the
