@@ -216,13 +216,15 @@ def test_rdf_points_outside_the_box(oracle, which):
     npt.assert_array_equal(rdf.compute((box, pts)).bin_counts, ref)
 
 
-@pytest.mark.parametrize("name, n, r", [("small", 300, 2.9), ("thin", 900, 1.9), ("square", 700, 3.0), ("square", 3000, 0.2),
-                                        ("cube", 4000, 1.2), ("cube", 50000, 1.0), ("cube", 56000, 1.0)])
+@pytest.mark.parametrize("name, n, r", [("small", 300, 2.9), ("thin", 900, 1.9), ("square", 700, 3.0),
+                                        ("square", 3000, 0.2), ("cube", 4000, 1.2), ("cube", 50000, 1.0),
+                                        ("cube", 56000, 1.0)])
 def test_rdf_outside_routes(oracle, name, n, r):
     """Systems off the box, a wave or a thread per point (above some 53,000
-    points in the cube, 1,000 per candidate in two dimensions): rows of cells that wrap more than once, boxes of two
-    dimensions and tilted ones, points many boxes away; query points of their
-    own, few and many, with the points in the box or off it."""
+    points in the cube, 1,000 per candidate in two dimensions): rows of cells
+    that wrap more than once, boxes of two dimensions and tilted ones, points
+    boxes away; query points of their own, few and many, with the points in the
+    box or off it."""
     box = {"small": Box(6.0, 6.0, 6.0, 0.2, -0.1, 0.15), "thin": Box(4.0, 30.0, 8.0),
            "square": Box.square(26.0), "cube": Box.cube((n / 0.8) ** (1 / 3))}[name]
     rng = np.random.default_rng(n)
