@@ -2229,10 +2229,19 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
     uint32_t points = kBlock;
     while (points > 32u && 1.15 * double(total) * points * double(ksz) > double(kBallKeyBytes) * n_query)
         points /= 2;
-    size_t const kb = fill_key_bytes(total, n_query, ksz, points);
+    // Few points: their sorts and stores over more workgroups, as long as four per
+    // CU hold them all (which also leaves each a full share of LDS for its keys).
+    // Random points, us at 256 and at 64 or 128 points per workgroup: 34,000,
+    // 14 bonds each 47 and 39, 25 bonds 78 and 69, 39 bonds 141 and 112; 130,000,
+    // 14 bonds 69 and 61; with more workgroups than are resident, 260,000 points,
+    // 14 bonds: 82 and 130 (64 points).
+    constexpr uint32_t kResident = 4u * 256u;
+    while (points > 64u && (n_query + points / 2 - 1) / (points / 2) <= kResident)
+        points /= 2;
+    unsigned const eblocks = (n_query + points - 1) / points;
+    size_t const kb = eblocks <= kResident ? size_t(kBallKeyBytes) : fill_key_bytes(total, n_query, ksz, points);
     auto emit = [&](auto kern) {
         FA_PROF_BEGIN("ball_emit_kernel");
-        unsigned const eblocks = (n_query + points - 1) / points;
         hipLaunchKernelGGL(kern, dim3(eblocks), dim3(kBlock), owner_lds(kb, ksz, eblocks), s, db, g, qpts, n_query,
                            nq->d_points, r_max_sq, r_min_sq, a.exclude_ii, R, cq, C, pos, rows, out->offsets,
                            out->neighbors, out->distances, out->weights, out->vectors, gkeys, uint32_t(kb / ksz), points);
@@ -2248,7 +2257,14 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
             return rc;
         index_order = sorder == nullptr;
     }
-    // the register networks for the lists' mean length with some spread (block_sort_lists)
+    // The register networks for the lists' mean length with some spread
+    // (block_sort_lists).  The one of 48 keys costs the kernel a third of its
+    // waves: random points, us with 32 and with 48 keys: 15.6 bonds, 1,500,000
+    // points 642 and 664, 200,000 100 and 88; 20.6 bonds 902 and 841, 126 and 113;
+    // 25 bonds 1174 and 889, 164 and 145; without a network and with it: 39 bonds
+    // 2065 and 1932, 45 bonds 2256 and 2236, a crystal's 40 1852 and 1518.  Its
+    // workgroups take two rounds where one round of the others' (LDS: five per CU)
+    // would do: 160,000 points, 29 bonds: 130 and 187.
     auto emit_form = [&](auto form, auto by_dist, auto net) {
         constexpr int F = decltype(form)::value, N = decltype(net)::value;
         constexpr bool D = decltype(by_dist)::value;
@@ -2261,9 +2277,9 @@ int run_ball(fa_nq* nq, const float* qpts, uint32_t n_query, const fa_query_args
             emit_form(form, std::true_type{}, std::integral_constant<int, 0>{});
         else if (mean <= 6.0)
             emit_form(form, std::false_type{}, std::integral_constant<int, 16>{});
-        else if (mean <= 30.0)
+        else if (mean <= (eblocks <= kResident ? 15.0 : eblocks <= 5u * 256u ? 40.0 : 20.0))
             emit_form(form, std::false_type{}, std::integral_constant<int, 32>{});
-        else if (mean <= 38.0)
+        else if (mean <= 45.0)
             emit_form(form, std::false_type{}, std::integral_constant<int, 48>{});
         else
             emit_form(form, std::false_type{}, std::integral_constant<int, 0>{});

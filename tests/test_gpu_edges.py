@@ -559,3 +559,20 @@ def test_cluster_percolation(oracle, store, n, bonds):
     ref = oracle.solidliquid(ref_nl, st.particle_harmonics, st.ql, 6, 0.4, 2, normalize_q=True)
     if not np.any(np.abs(ref["ql_ij"] - 0.4) < 1e-6):
         npt.assert_array_equal(sl.cluster_idx, ref["cluster_idx"])
+
+
+@pytest.mark.parametrize("n, bonds", [(33001, 5), (33001, 13), (33001, 18), (33001, 28), (33001, 43), (33001, 52),
+                                      (66000, 28), (140000, 18), (140000, 28), (300000, 18)])
+def test_ball_emission_of_systems_of_middle_size(oracle, n, bonds):
+    """Workgroups of 64, 128 and 256 points, up to as many as are resident and
+    beyond, with each network for lists of about its length; in the caller's
+    order and in the walk's."""
+    side = n ** (1 / 3)
+    box = Box.cube(side * 1.0001)
+    rng = np.random.default_rng(bonds)
+    pts = ((rng.random((n, 3)) - 0.5) * side).astype(np.float32)
+    if n == 66000:
+        pts = pts[np.argsort(np.floor(pts[:, 2] / 2), kind="stable")]
+    args = dict(r_max=(bonds / 4.18879) ** (1 / 3), exclude_ii=True)
+    ref = oracle.query(_bt(box), pts, pts, args, nthreads=16)
+    _assert_same(freud_amd.AABBQuery(box, pts).query(pts, args).toNeighborList(), ref)
